@@ -1,0 +1,55 @@
+"""State snapshots (efdc_state_save, efdc_state_load): the one-launch copy of
+an aligned device buffer against the piece-by-piece copies that any other
+buffer takes, on arrays whose bytes are no multiple of 16, and both
+directions against the arrays themselves."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (nx, ny, kc, internal): snapshots below and above 64 MiB, odd and even LCM,
+# with and without the internal mode's pieces (more than one launch's table)
+SIZES = [(3, 3, 1, False), (16, 8, 3, False), (37, 23, 5, True), (331, 293, 11, False)]
+
+
+@pytest.mark.parametrize("store", ["fp64", "fp32"])
+@pytest.mark.parametrize("nx,ny,kc,internal", SIZES)
+def test_snapshot_copies(nx, ny, kc, internal, store):
+    import torch
+    from efdc_amd import grids, lib
+    case = grids.tidal_basin(nx, ny, kc, seed=nx)
+    if internal:
+        grids.add_internal_mode(case, av=1e-3)
+    st = lib.STORE_FP32 if store == "fp32" else lib.STORE_FP64
+    ctx = lib.Context(case.grid, store=st, RSQM=1e-20, ITERM=500)
+    ctx.upload_case(case)
+    for n in (1, 2):
+        ctx.step(case.dt, n, internal=internal)
+    names = ["P", "HP", "H2P", "UHDYE", "CCCI", "SVBO", "HPK", "UHDY2", "W2"]
+    names += ["U1", "AVVI", "W"] if internal else []
+    want = {a: ctx.get(a) for a in names}
+    cons = [ctx.get_constituent(j) for j in range(2)]
+    nb = ctx.state_bytes()
+    # 0xAB in the gaps between the pieces, which no copy may touch
+    a = torch.full((nb,), 0xAB, dtype=torch.uint8, device="cuda")
+    b = torch.full((nb + 8,), 0xAB, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    ctx.state_save(a.data_ptr())
+    ctx.state_save(b.data_ptr() + 8)
+    ctx.synchronize()
+    assert torch.equal(a, b[8:])
+    other = lib.Context(case.grid, store=st, RSQM=1e-20, ITERM=500)
+    other.upload_case(case)
+    if internal:
+        other.step(case.dt, 1, internal=True)
+    for buf in (a.data_ptr(), b.data_ptr() + 8):
+        for name in ("P", "HPK", "W2"):
+            other.set(name, np.ones_like(want[name]))
+        other.state_load(buf)
+        for name in names:
+            assert np.array_equal(other.get(name), want[name]), name
+        for j in range(2):
+            got = other.get_constituent(j)
+            assert np.array_equal(got[0], cons[j][0]) and np.array_equal(got[1], cons[j][1])
+    ctx.close()
+    other.close()
