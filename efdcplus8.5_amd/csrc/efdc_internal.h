@@ -259,7 +259,8 @@ struct efdc_ctx {
   int pcg_pipe_mode = 0;
   bool pcg_pipe_tuned = true;     // the pipelined form (the autotuner's choice)
   double *tune_pbuf = nullptr;    // P saved while solves are timed
-  int tran_ncg = 0, tran_w3 = 0;  // 0: not tuned
+  int tran_ncg = 0, tran_w3 = 0;  // the tuned column kernel (0: k_tran_lay)
+  bool tran_tuned = false;
   int tune_n = 0, tune_best = -1;
   char tune_name[8][32] = {};
   float tune_ms[8] = {};

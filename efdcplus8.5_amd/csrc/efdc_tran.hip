@@ -11,8 +11,10 @@
 // CON1 are two buffers whose roles swap every step (CON1 = CON of
 // EFDC/caltran.f90:59-65 costs nothing).
 //
-// k_tran_colm (the default with mutual neighbour maps) runs one thread per
-// column and 1, 2 or 4 constituents: the transport fields and the
+// k_tran_lay (the default with mutual neighbour maps) puts the layers of a
+// column side by side in a workgroup and solves the columns from LDS.
+// k_tran_colm (the default for long FP32 columns, mutual maps) runs one thread
+// per column and 1, 2 or 4 constituents: the transport fields and the
 // tridiagonal factors are loaded and computed once per layer for all of
 // them.  k_tran_col (any maps) runs one thread per (column, constituent):
 // a workgroup is 64 columns x up to 4 constituent waves.  In both, each
@@ -780,6 +782,317 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   tran_colm_body<T, NCW, FPF>(a, vcus);
 }
 
+// ---------------------------------------------------------------------
+// k_tran_lay: the same column step with the layers of a column side by side.
+//
+// Only the vertical solve couples the layers, so a workgroup owns 64 columns
+// and NCG constituents: nlw waves take the layers (wave w the layers w,
+// w + nlw, ..) and form CON after the upwind step and the open boundaries
+// into LDS, one more wave forms the tridiagonal factors at the same time,
+// and after one barrier a wave per constituent runs the forward sweep and
+// the back substitution from LDS (with the dye decay and, when asked for, the
+// settling sweep, which walks down the column as the back substitution does)
+// and writes the new concentrations once.
+// The column kernels walk the layers one after the other with one layer of
+// loads in flight per wave, which leaves them at a fraction of the copy rate
+// (one exposed round trip per layer); here the loads of all layers are in
+// flight together, over nlw waves and the workgroups that share a CU.
+// Every value and operation order is that of tran_col_body (the flux through
+// a layer's lower face is formed again from the layer below, the same
+// product), so the bits are those of the column kernels.  FP64 in LDS: EEB,
+// CCLB, VCU and NCG x CON per layer and column, plus HPKI in the storage type
+// when a constituent settles.
+// Bound: VALU issue (about 300 FP64 operations a column and layer with four
+// constituents, 43 % busy) and memory (640x512x20, 4 constituents, FP32 with
+// settling: 151 us against 171 + 18 before, 2.5 TB/s of algorithmic bytes)
+// together; on small grids latency (128x64x5, 2 constituents, FP64: 7.7
+// against 12.9 us; 40x40 columns of 11 layers: 6 times faster a step).
+// Prefetching the next layer's values, or fewer registers for six waves a
+// SIMD, measured slower (184 and 350 us at 640x512x20): the waves in flight
+// and spills decide.
+// ---------------------------------------------------------------------
+struct SettleArgs {
+  int on;  // some constituent settles in this launch
+  double dt, ws[EFDC_MAXC], wsetmp[EFDC_MAXC], wese[EFDC_MAXC];
+};
+
+template <typename T, int NCG, bool RARE>
+__device__ __forceinline__ void tran_lay_layers(const TranArgs<T> &a, double *lc, T *lhp, int i,
+                                                int c0, int k0, int kstep, int src0, int rec) {
+  const int KC = a.KC, nc = a.nc;
+  const int w = a.lw[i], s = a.ls[i];
+  const int e = a.rowmajor ? i + 1 : a.le[i];
+  const int n = a.ln[i];
+  const bool eg = a.rowmajor ? (a.le[i] == a.lc0) : (e == a.lc0);
+  const bool ng = (n == a.lc0);
+  // as in tran_colm_run: a missing neighbour or layer reads the column itself
+  const unsigned bi = (unsigned)i * sizeof(T), bw = (unsigned)w * sizeof(T),
+                 bs = (unsigned)s * sizeof(T), be = eg ? bi : (unsigned)e * sizeof(T),
+                 bn = ng ? bi : (unsigned)n * sizeof(T);
+  const size_t pitch = (size_t)a.pitch;
+  const double DDELT = a.dt;
+  const double dxyip = a.dxyip[i];
+  int4 bc = make_int4(-1, -1, -1, -1);
+  if (RARE && rec >= 0) bc = a.bcinfo[rec];
+  bool on[NCG];
+  const T *C1[NCG];
+#pragma unroll
+  for (int j = 0; j < NCG; ++j) {
+    on[j] = j == 0 || c0 + j < nc;
+    C1[j] = a.old[on[j] ? c0 + j : c0];
+  }
+  for (int k = k0; k < KC; k += kstep) {
+    const size_t o = (size_t)k * pitch;
+    const bool below_top = k + 1 < KC, above_bed = k > 0;
+    const size_t ou = below_top ? o + pitch : o, od = above_bed ? o - pitch : o;
+    const T *U = a.uhdy2 + o, *V = a.vhdx2 + o;
+    const T tu_i = ldb(U, bi), tu_e = ldb(U, be), tv_i = ldb(V, bi), tv_n = ldb(V, bn);
+    const T tw = ldb(a.w2 + o + pitch, bi), tw0 = ldb(a.w2 + o, bi);  // KC+1 planes
+    const T th1 = ldb(a.h1pk + o, bi), thi = ldb(a.hpki + o, bi);
+    T c1[NCG], cw[NCG], cs[NCG], ce[NCG], cn[NCG], cup[NCG], cdn[NCG];
+#pragma unroll
+    for (int j = 0; j < NCG; ++j) {
+      const T *P = C1[j] + o;
+      c1[j] = ldb(P, bi);
+      cw[j] = ldb(P, bw);
+      cs[j] = ldb(P, bs);
+      ce[j] = ldb(P, be);
+      cn[j] = ldb(P, bn);
+      cup[j] = ldb(C1[j] + ou, bi);
+      cdn[j] = ldb(C1[j] + od, bi);
+    }
+    const double u_i = (double)tu_i, u_e = eg ? 0.0 : (double)tu_e, v_i = (double)tv_i,
+                 v_n = ng ? 0.0 : (double)tv_n;
+    const double ww = below_top ? (double)tw : 0.0, ww0 = (double)tw0;
+    const double h1pk = (double)th1, hpki = (double)thi;
+    const bool pu = tu_i >= (T)0, pv = tv_i >= (T)0, pue = tu_e >= (T)0, pvn = tv_n >= (T)0,
+               pw = tw >= (T)0, pw0 = tw0 >= (T)0;
+    if (lhp) lhp[k * 64] = thi;
+#pragma unroll
+    for (int j = 0; j < NCG; ++j) {
+      if (!on[j]) continue;
+      const int cc = c0 + j;
+      const double c1d = (double)c1[j];
+      // upwind fluxes (LUPU/LUPV/KUPW of EFDC/calconc.f90:95-118)
+      const double fu_i = u_i * (double)(pu ? cw[j] : c1[j]);
+      const double fv_i = v_i * (double)(pv ? cs[j] : c1[j]);
+      const double fu_e = eg ? 0.0 : u_e * (double)(pue ? c1[j] : ce[j]);
+      const double fv_n = ng ? 0.0 : v_n * (double)(pvn ? c1[j] : cn[j]);
+      const double fw = below_top ? ww * (double)(pw ? c1[j] : cup[j]) : 0.0;
+      const double fw0 = above_bed ? ww0 * (double)(pw0 ? cdn[j] : c1[j]) : 0.0;
+      const double fqc = (RARE && src0 >= 0) ? col_sources(a, src0, k, cc, c1d) : 0.0;
+      // EFDC/caltran.f90:194-196,243
+      const double cd = c1d * h1pk + DDELT * ((fqc + fu_i - fu_e + fv_i - fv_n) * dxyip +
+                                              (fw0 - fw));
+      double con = cd * hpki;
+      if (RARE && rec >= 0)
+        con = col_open_bc(a, bc, rec, k, cc, c1d, con, u_i, u_e, v_i, v_n, fu_i, fu_e, fv_i,
+                          fv_n, dxyip, hpki);
+      if (a.vd) lc[((size_t)j * KC + k) * 64] = con;
+      else stb((T)con, a.nw[cc] + o, bi);
+    }
+  }
+}
+
+// EEB, CCLB and VCU of a column (KC > 1), as in tran_col_body; the AB values
+// are loaded eight layers at a time
+template <typename T>
+__device__ __forceinline__ void tran_lay_factors(const TranArgs<T> &a, int i, double *eebs,
+                                                 double *ccls, double *vcus) {
+  const int KC = a.KC;
+  const size_t pitch = (size_t)a.pitch;
+  const double DELTD2 = a.dt, hpi = a.hpi[i];
+  const bool uni = a.dz_uniform != 0;
+  const T *ab = a.ab + i, *kk = (uni ? a.ab : a.cdzkk) + i, *km = (uni ? a.ab : a.cdzkmk) + i;
+  double vcu_prev = 0.0, ab_prev = 0.0;
+  for (int k0 = 0; k0 < KC; k0 += 8) {
+    T abv[8], ckv[8], cmv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const size_t o = (size_t)(k0 + u < KC ? k0 + u : KC - 1) * pitch;
+      abv[u] = ab[o];
+      if (!uni) {
+        ckv[u] = kk[o];
+        cmv[u] = km[o];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int k = k0 + u, K = k + 1;
+      if (k >= KC) break;
+      const double ckk = uni ? a.cdzkk_k[k] : (double)ckv[u];
+      const double ckm = uni ? a.cdzkmk_k[k] : (double)cmv[u];
+      const double abk = K < KC ? (double)abv[u] : 0.0;
+      double cclb = 0.0, eeb, vcu_k = 0.0;
+      if (K == 1) {
+        const double RCDZKK = -DELTD2 * ckk;
+        const double CCUBTMP = RCDZKK * hpi * abk;
+        const double CCMBTMP = 1.0 - CCUBTMP;
+        eeb = 1.0 / CCMBTMP;
+        vcu_k = CCUBTMP * eeb;
+      } else if (K < KC) {
+        const double RCDZKMK = -DELTD2 * ckm;
+        const double RCDZKK = -DELTD2 * ckk;
+        cclb = RCDZKMK * hpi * ab_prev;
+        const double CCUBTMP = RCDZKK * hpi * abk;
+        const double CCMBTMP = 1.0 - cclb - CCUBTMP;
+        eeb = 1.0 / (CCMBTMP - cclb * vcu_prev);
+        vcu_k = CCUBTMP * eeb;
+      } else {
+        const double RCDZKMK = -DELTD2 * ckm;
+        cclb = RCDZKMK * hpi * ab_prev;
+        const double CCMBTMP = 1.0 - cclb;
+        eeb = 1.0 / (CCMBTMP - cclb * vcu_prev);
+      }
+      eebs[k * 64] = eeb;
+      ccls[k * 64] = cclb;
+      vcus[k * 64] = vcu_k;
+      ab_prev = abk;
+      vcu_prev = vcu_k;
+    }
+  }
+}
+
+// Forward sweep, back substitution, decay and (ws > 0) settling of one
+// column and constituent whose CON lies in lc and whose factors in eebs,
+// ccls, vcus (all at stride 64); writes the new concentrations at bi.
+template <typename T>
+__device__ __forceinline__ void tran_lay_solve(int KC, size_t pitch, double *lc,
+                                               const double *eebs, const double *ccls,
+                                               const double *vcus, const T *lhp, T *out,
+                                               unsigned bi, int dm, double f, double dtsed,
+                                               double ws, double wsetmp, double wese) {
+  double yprev = 0.0;
+  if (KC == 1) {
+    yprev = (double)(T)lc[0];
+  } else {
+#pragma unroll 4
+    for (int k = 0; k < KC; ++k) {
+      const double con = lc[k * 64], eeb = eebs[k * 64];
+      const double y = k == 0 ? con * eeb : (con - ccls[k * 64] * yprev) * eeb;
+      const T yt = (T)y;  // forward values in the storage type
+      yprev = (double)yt;
+      lc[k * 64] = yprev;
+    }
+  }
+  auto fin = [&](double v) { return (T)(dm == 1 ? f * v : (dm == 2 ? v + f : v)); };
+  double up = yprev;
+  if (!(ws > 0.0)) {
+    stb(fin(up), out + (size_t)(KC - 1) * pitch, bi);
+#pragma unroll 4
+    for (int k = KC - 2; k >= 0; --k) {
+      up = lc[k * 64] - vcus[k * 64] * up;
+      stb(fin(up), out + (size_t)k * pitch, bi);
+    }
+    return;
+  }
+  // settling from the top layer down, EFDC/calsed.f90:232-256,308-312, as
+  // k_settle: each layer's flux from its stored value
+  double sedf = 0.0;
+#pragma unroll 4
+  for (int k = KC - 1; k >= 0; --k) {
+    if (k < KC - 1) up = lc[k * 64] - vcus[k * 64] * up;
+    const double x = dmx((double)fin(up), 0.);
+    const double WVEL = dtsed * (double)lhp[k * 64];
+    T v;
+    if (k > 0) {
+      const double CLEFT = 1. + ws * WVEL;
+      const double CRIGHT = k == KC - 1 ? x : x - sedf * WVEL;
+      v = (T)(CRIGHT / CLEFT);
+      sedf = -ws * (double)v;
+    } else {
+      const double CLEFT = 1. + wsetmp * WVEL;
+      const double CRIGHT = x + (wese - sedf) * WVEL;
+      v = (T)(CRIGHT / CLEFT);
+    }
+    stb(v, out + (size_t)k * pitch, bi);
+  }
+}
+
+template <typename T, int NCG>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_tran_lay(
+    TranArgs<T> a, SettleArgs st, int nlw) {
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x, KC = a.KC;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int i = tile * 64 + lane;
+  const int c0 = blockIdx.y * NCG;
+  double *eebs = lds + lane, *ccls = eebs + (size_t)KC * 64, *vcus = ccls + (size_t)KC * 64,
+         *lcs = vcus + (size_t)KC * 64;
+  T *lhp = st.on ? (T *)(lds + (size_t)(3 + NCG) * KC * 64) + lane : nullptr;
+  const bool act = i >= 1 && i <= a.nwet;
+  const bool keep = act && a.lmask && a.lmask[i] == 0;
+  if (act) {
+    if (wv < nlw) {
+      if (keep) {
+        // left out of the transport: CON stays (col_keep)
+        for (int c = c0; c < c0 + NCG && c < a.nc; ++c)
+          for (int k = wv; k < KC; k += nlw)
+            a.nw[c][i + (int64_t)k * a.pitch] = a.old[c][i + (int64_t)k * a.pitch];
+      } else {
+        const int src0 = a.srcrec[i];
+        const int rec = a.bcrec ? a.bcrec[i] : -1;
+        if (__ballot(src0 >= 0 || rec >= 0) != 0)
+          tran_lay_layers<T, NCG, true>(a, lcs, lhp, i, c0, wv, nlw, src0, rec);
+        else
+          tran_lay_layers<T, NCG, false>(a, lcs, lhp, i, c0, wv, nlw, src0, rec);
+      }
+    } else if (a.vd && !keep) {
+      tran_lay_factors(a, i, eebs, ccls, vcus);
+    }
+  }
+  if (!a.vd) return;
+  __syncthreads();
+  if (!act || keep) return;
+  for (int j = wv; j < NCG; j += blockDim.y) {
+    const int c = c0 + j;
+    if (c >= a.nc) break;
+    tran_lay_solve<T>(KC, (size_t)a.pitch, lcs + (size_t)j * KC * 64, eebs, ccls, vcus, lhp,
+                      a.nw[c], (unsigned)i * sizeof(T), a.dye_mode[c], a.dye_f[c], st.dt,
+                      st.on ? st.ws[c] : 0.0, st.wsetmp[c], st.wese[c]);
+  }
+}
+
+// Launch shape of k_tran_lay: NCG constituents per workgroup and nlw layer
+// waves.  ncg = 0: the column kernels are the better ones.  Measured on
+// 64-column tiles by the thousand (us per pass against k_tran_colm):
+// * waves: 3 layer waves and the factor wave are one wave per SIMD, and the
+//   four such workgroups of a CU are in different phases (600x512, 2
+//   constituents, FP32: KC = 6 25.4 against 40.0 with 6 layer waves; KC = 10
+//   36.7 against 55.5); where the LDS holds only two workgroups a CU, or the
+//   grid fills no more, 7 layer waves do better (640x512x20, 4 constituents,
+//   FP32: 135 against 165; 128x128x20: 17.0 against 23.3).
+// * constituents: as many as 80 KiB hold, up to 4; 2 in FP64, whose values
+//   take twice the registers (600x512x10, 4 constituents: 129 against 161).
+// * the column kernels stay for FP32 columns too long for two workgroups a
+//   CU with all their constituents (400x300x40, 2 constituents: 103 against
+//   137) unless the grid is small.
+struct LayShape {
+  int ncg = 0, ngrp = 0, nlw = 0;
+  size_t lds = 0;
+};
+inline LayShape lay_shape(int KC, int nc, int tiles, size_t tsz, bool vd, bool settle) {
+  LayShape s;
+  const size_t half = (size_t)80 << 10, full = (size_t)160 << 10;
+  const int most = std::min(nc, tsz == 8 ? 2 : 4);
+  auto lds_of = [&](int q) {
+    return vd ? (size_t)64 * KC * (8 * (3 + q) + (settle ? tsz : 0)) : (size_t)0;
+  };
+  const bool small = tiles <= 512;
+  if (tsz == 4 && lds_of(most) > half && !small) return s;
+  int q = most;
+  while (q > 1 && lds_of(q) > half) --q;
+  if (lds_of(q) > full) return s;
+  s.ngrp = (nc + q - 1) / q;
+  s.ncg = (nc + s.ngrp - 1) / s.ngrp;
+  s.lds = lds_of(s.ncg);
+  const bool wide = tiles * s.ngrp <= 512 || 3 * s.lds > full;
+  const int per = (KC + (wide ? 6 : 2)) / (wide ? 7 : 3);
+  s.nlw = (KC + per - 1) / per;
+  return s;
+}
+
 // Cohesive settling after the transport (SSEDTOX -> CALSED with DTSED = DT,
 // EFDC/calconc.f90:621-630, WSETA = WSEDO): the implicit upwind sweep from
 // the top layer down, EFDC/calsed.f90:232-256, then the bottom layer with
@@ -1354,10 +1667,10 @@ int adac_pipeline(efdc_ctx *c, TranArgs<T> &ta, const efdc_step_t *step) {
 
 // CON1 of the open-boundary columns, then the CON/CON1 buffer swap.
 template <typename T>
-int finish_tran(efdc_ctx *c, TranArgs<T> &a, const efdc_step_t *step) {
+int finish_tran(efdc_ctx *c, TranArgs<T> &a, const efdc_step_t *step, bool settled = false) {
   for (int j = 0; j < c->nconst; ++j) {
     const efdc_constituent_t &d = c->con[j].desc;
-    if (!(d.wset > 0.0)) continue;
+    if (settled || !(d.wset > 0.0)) continue;
     if (adj_recording(c)) {
       const int s = adj_record_settle(c, j, a.nw[j]);
       if (s) return s;
@@ -1479,9 +1792,37 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
   int qs[3], nq = 0;
   for (int q : {4, 2, 1})
     if (shape_ok(q)) qs[nq++] = q;
-  if (KC <= 64 && off32 && nq > 0) {
+  // k_tran_lay runs for the default shape with mutual maps wherever a
+  // column of one constituent fits the LDS (KC <= 64 does); it settles in the same
+  // pass unless the adjoint records the column before the settling
+  bool settles = false;
+  for (int j = 0; j < nc; ++j) settles |= c->con[j].desc.wset > 0.0;
+  settles = settles && a.vd && !adj_recording(c);
+  const LayShape lay = colm && req == 0 && off32
+                           ? lay_shape(KC, nc, (a.nwet + 64) / 64, sizeof(T), a.vd, settles)
+                           : LayShape();
+  SettleArgs sa;
+  std::memset(&sa, 0, sizeof sa);
+  sa.on = settles ? 1 : 0;
+  sa.dt = step->dt;
+  for (int j = 0; j < nc; ++j) {
+    const efdc_constituent_t &d = c->con[j].desc;
+    sa.ws[j] = settles ? d.wset : 0.0;
+    sa.wsetmp[j] = d.probdep * d.wset;
+    sa.wese[j] = d.wese;
+  }
+  if (KC <= 64 && off32 && (nq > 0 || lay.ncg)) {
     const int nbc = colm ? (a.nwet + 64) / 64 : (a.nwet + 63) / 64;
+    // q = 0: k_tran_lay
     auto launch = [&](int q, int w3) {
+      if (q == 0) {
+        const dim3 grid(nbc, lay.ngrp), lblk(64, lay.nlw + (a.vd && KC > 1 ? 1 : 0));
+        if (lay.ncg == 1) k_tran_lay<T, 1><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
+        else if (lay.ncg == 2) k_tran_lay<T, 2><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
+        else if (lay.ncg == 3) k_tran_lay<T, 3><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
+        else k_tran_lay<T, 4><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
+        return;
+      }
       const dim3 blk(64, waves_of(q));
       const size_t lds = lds_of(q);
       if (!colm) {
@@ -1513,16 +1854,20 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
       int best = -1;
       float best_ms = 1e30f;
       hipEvent_t e0 = timer_event(c), e1 = timer_event(c);
-      for (int qi = 0; qi < nq; ++qi) {
+      int cand[4], ncand = 0;  // k_tran_lay first, then the column kernels
+      if (lay.ncg) cand[ncand++] = 0;
+      for (int qi = 0; qi < nq; ++qi) cand[ncand++] = qs[qi];
+      for (int qi = 0; qi < ncand; ++qi) {
         // variants: 0 the compiler's register budget, 1 at most 168 VGPRs,
         // 2 (k_tran_colm with 1 or 2 constituents per thread) at most 168
         // VGPRs with the transport fields two layers ahead
-        const int nvar = (colm && qs[qi] <= 2) ? 3 : 2;
+        // (one per thread only without them: the report holds 8 entries)
+        const int nvar = cand[qi] == 0 ? 1 : (colm && cand[qi] == 2) ? 3 : 2;
         for (int w3 = 0; w3 < nvar; ++w3) {
           float tot = 0.f;
           for (int r = 0; r < 4; ++r) {
             HIP_TRY(c, hipEventRecord(e0, c->stream));
-            launch(qs[qi], w3);
+            launch(cand[qi], w3);
             HIP_TRY(c, hipEventRecord(e1, c->stream));
             HIP_TRY(c, hipEventSynchronize(e1));
             float ms = 0.f;
@@ -1532,8 +1877,11 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
           const float avg = tot / 3.f;
           int slot = -1;
           if (c->tune_n < 8) {
-            std::snprintf(c->tune_name[c->tune_n], 32, "%s=%d%s",
-                          colm ? "tran_colm ncw" : "tran_col lanes", qs[qi],
+            if (cand[qi] == 0)
+              std::snprintf(c->tune_name[c->tune_n], 32, "tran_layers");
+            else
+              std::snprintf(c->tune_name[c->tune_n], 32, "%s=%d%s",
+                          colm ? "tran_colm ncw" : "tran_col lanes", cand[qi],
                           w3 == 2 ? " vgpr<=168 pf2" : (w3 ? " vgpr<=168" : ""));
             slot = c->tune_n;
             c->tune_ms[c->tune_n++] = avg;
@@ -1541,8 +1889,9 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
           if (avg < best_ms) {
             best_ms = avg;
             best = slot;
-            c->tran_ncg = qs[qi];
+            c->tran_ncg = cand[qi];
             c->tran_w3 = w3;
+            c->tran_tuned = true;
           }
         }
       }
@@ -1550,16 +1899,19 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
       c->ev_pool.push_back(e0);
       c->ev_pool.push_back(e1);
     }
-    // untuned default: 2 constituents per wave (column kernel with mutual
-    // maps), else as many lanes as fit
-    int q = req != 0 ? (req < 0 ? -req : req) : c->tran_ncg;
-    if (q <= 0 || !shape_ok(q)) q = (colm && shape_ok(2)) ? 2 : qs[0];
-    TIMED(c, TK_TRAN, launch(q, req != 0 ? req_var : (c->tran_ncg > 0 ? c->tran_w3 : 0)));
+    // untuned default: k_tran_lay where it fits, else 2 constituents per
+    // wave (column kernel with mutual maps), else as many lanes as fit
+    int q = req != 0 ? (req < 0 ? -req : req) : c->tran_tuned ? c->tran_ncg : 0;
+    int var = req != 0 ? req_var : c->tran_tuned ? c->tran_w3 : 0;
+    if (q == 0 && !lay.ncg) var = 0;
+    if (q == 0 ? !lay.ncg : !shape_ok(q)) q = (colm && shape_ok(2)) ? 2 : qs[0];
+    TIMED(c, TK_TRAN, launch(q, var));
+    const bool settled = q == 0 && settles;
     if (any_adac) {
       int s = adac_pipeline<T>(c, a, step);
       if (s) return s;
     }
-    return finish_tran(c, a, step);
+    return finish_tran(c, a, step, settled);
   }
   if (req != 0) {
     c->err = "tran_shape names a column kernel, which does not fit this grid";
