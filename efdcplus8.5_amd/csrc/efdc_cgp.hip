@@ -61,6 +61,8 @@ constexpr double INNER_MARGIN2 = 1e-2;
 constexpr int WIN = 2048;         // LDS window reach beyond the own range
 constexpr int HMAX = 2 * WIN;     // outside cells of one workgroup, at most
 constexpr int NVMAX = 3;          // partials per exchange, at most
+constexpr int PCGMX_CPT_SMALL = 8;  // cells per thread of every mixed form
+constexpr int PCGMX_CPT_MAX = 16;   // of the pipelined form alone
 constexpr int HX_WORDS = 4;       // 4-byte words per cell and parity in the halo slots
 
 // Halo slots are planes (one per value and parity), so that the stores of
@@ -954,6 +956,29 @@ __device__ bool halo_wait(const Xch &x, unsigned tag, int lo, int hi, const int 
   return true;
 }
 
+// One FP32 word of each outside cell straight into the window: entry h of the
+// list is the window slot of that cell (b0 - WIN + slot is the cell).  The
+// owners' flags must already be up.
+__device__ void fetch_window32(const Xch &x, unsigned tag, const unsigned short *hs, int nhalo,
+                               int b0, float *win) {
+  const int t = threadIdx.x;
+  const unsigned *w32 = x.hx + (size_t)(tag & 1u) * HX_WORDS * (size_t)x.ncell;
+  constexpr int HB = 4;
+  for (int h0 = t; h0 < nhalo; h0 += HB * PB) {
+    unsigned v[HB];
+    int sl[HB];
+#pragma unroll
+    for (int u = 0; u < HB; ++u) {  // every lane loads
+      sl[u] = hs[min(h0 + u * PB, nhalo - 1)];
+      v[u] = get_u32(w32 + (size_t)(sl[u] + b0 - WIN));
+    }
+#pragma unroll
+    for (int u = 0; u < HB; ++u)
+      if (h0 + u * PB < nhalo) win[sl[u]] = __uint_as_float(v[u]);
+  }
+  __syncthreads();
+}
+
 // FP64 value 0 of each outside cell in the slots of exchange `tag` (posted
 // with put_f64 at word 2*i of that parity's first FP64 plane) into raw[h]
 // (low word) and raw[HMAX + h] (high word); the flags must already be up.
@@ -996,28 +1021,58 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
   // the window, then one word that stays zero: a row reads it in place of
   // a neighbour it does not couple to, so that every lane loads
   __shared__ float lds[2 * WIN + CPT * PB + 1];
-  __shared__ int hl[2 * WIN];
-  __shared__ unsigned raw[HMAX];
+  // More than 8 cells per thread (BIG): to stay within 160 KiB of LDS the
+  // outside cells are a list of 16-bit window slots and their values go
+  // straight to the window; towards 256 VGPRs, a row keeps the window slots
+  // of its south and north neighbours in one word, M^-1 v stays in the window,
+  // and the rows' addresses are formed where they are used.  Bound by the
+  // exchanges and, at 16 cells per thread, by about 100 spilled registers.
+  // Against two launches per iteration of the multi-kernel solve (31 inner
+  // iterations, this one 17): 1.10 M cells 988 -> 237 us, 1.37 M 1101 -> 283,
+  // 2.02 M 1335 -> 546.  Up to 8 the plain form is the faster one (6 cells:
+  // 163 against 180 us).
+  constexpr bool BIG = CPT > PCGMX_CPT_SMALL;
+  static_assert(!BIG || 3 * CPT * PB >= 2 * WIN, "the list of outside cells is formed there");
+  __shared__ int hl[BIG ? 1 : 2 * WIN];
+  __shared__ unsigned raw[BIG ? 1 : HMAX];
+  __shared__ unsigned short hs[BIG ? 2 * WIN : 1];
   constexpr int ZS = 2 * WIN + CPT * PB;
   // y, q = M^-1 s and z = A' q of the own rows live in LDS
-  __shared__ float lys[CPT * PB], lqs[CPT * PB], lzs[CPT * PB];
+  __shared__ float lyqz[3 * CPT * PB];
   const int b0 = 1 + (int)blockIdx.x * CPT * PB;
   const int b1 = min(b0 + CPT * PB, a.nwet + 1);
   const int lc0 = a.lc0;
 
   float as_[CPT], an_[CPT], aw_[CPT], ae_[CPT];
   float r[CPT], u[CPT], w[CPT], s[CPT], p[CPT];
-  auto Y = [&](int k) -> float & { return lys[k * PB + threadIdx.x]; };
-  auto Q = [&](int k) -> float & { return lqs[k * PB + threadIdx.x]; };
-  auto Z = [&](int k) -> float & { return lzs[k * PB + threadIdx.x]; };
-  int js[CPT], jn[CPT];
+  auto Y = [&](int k) -> float & { return lyqz[k * PB + threadIdx.x]; };
+  auto Q = [&](int k) -> float & { return lyqz[(CPT + k) * PB + threadIdx.x]; };
+  auto Z = [&](int k) -> float & { return lyqz[(2 * CPT + k) * PB + threadIdx.x]; };
+  int js[BIG ? 1 : CPT], jn[BIG ? 1 : CPT];
+  unsigned jj[BIG ? CPT : 1];
   unsigned expo = 0u;
 
+  // BIG: the compiler works on a few rows at a time (loads of all sixteen in
+  // flight would spill the solve's state)
+  auto fence = [](int k_) {
+    if (BIG && k_ % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  };
   auto inside = [&](int j) { return j >= b0 && j < b1; };
   auto real = [&](int j) { return j > 0 && j != lc0; };
   auto slot = [&](int j) { return j - b0 + WIN; };
+  // the cell of a window slot (ZS: none), and a slot where it is an own cell's
+  auto cellof = [&](int sl) { return sl == ZS ? lc0 : sl - WIN + b0; };
+  auto ownslot = [&](int sl) { return sl >= WIN && sl < b1 - b0 + WIN ? sl : ZS; };
   auto hxw = [&](int i, unsigned tag) {
     return a.xc.hx + (size_t)(tag & 1u) * HX_WORDS * (size_t)a.xc.ncell + (size_t)opaque(i);
+  };
+  // BIG: the outside-read rows' slots, one base per call and no address kept
+  auto post_rows = [&](unsigned tag) {
+    unsigned *h = a.xc.hx + (size_t)(tag & 1u) * HX_WORDS * (size_t)a.xc.ncell +
+                  (size_t)opaque(b0 + (int)threadIdx.x);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k)
+      if (expo & (1u << k)) put_u32(h + k * PB, __float_as_uint(lds[WIN + k * PB + (int)threadIdx.x]));
   };
   // M^-1 v by the local Neumann polynomial, as in k_pcgmx.  No branch per
   // row: the lanes past b1 (the last workgroup's) hold zero coefficients
@@ -1046,6 +1101,45 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
     }
     __syncthreads();
   };
+  // BIG: the same with the result (and every step's values) in the own slots
+  // of the window, one register per row instead of two
+  auto precond_lds = [&](const float (&v)[CPT]) {
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) lds[WIN + k * PB + (int)threadIdx.x] = v[k];
+    for (int d = 1; d < a.pdeg; ++d) {
+      __syncthreads();
+      float tn[CPT];
+      const int tt = opaque((int)threadIdx.x);
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        const unsigned q = (unsigned)opaque((int)jj[k]);
+        const float ts = lds[ownslot((int)(q & 0xffffu))];
+        const float tnn = lds[ownslot((int)(q >> 16))];
+        const float tw = lds[k == 0 && tt == 0 ? ZS : WIN + k * PB + tt - 1];
+        const float te = lds[k * PB + tt + 1 < b1 - b0 ? WIN + k * PB + tt + 1 : ZS];
+        tn[k] = v[k] - (as_[k] * ts + an_[k] * tnn + aw_[k] * tw + ae_[k] * te);
+        fence(k);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) lds[WIN + k * PB + (int)threadIdx.x] = tn[k];
+    }
+  };
+  // y = A' x with x in the window (own slots and outside cells)
+  auto spmv_lds = [&](float (&y)[CPT]) {
+    const int tt = opaque((int)threadIdx.x);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      const int i = b0 + k * PB + tt;
+      const unsigned q = (unsigned)opaque((int)jj[k]);
+      const float vs = lds[q & 0xffffu], vn = lds[q >> 16];
+      const float vw = lds[real(i - 1) ? slot(i - 1) : ZS];
+      const float ve = lds[real(i + 1) ? slot(i + 1) : ZS];
+      const float yk = lds[slot(i)] + as_[k] * vs + an_[k] * vn + aw_[k] * vw + ae_[k] * ve;
+      y[k] = i < b1 ? yk : 0.0f;
+      fence(k);
+    }
+  };
   // y = A' x on the own rows from the LDS window (own slots and outside
   // cells); a lane past b1 may read a slot no one wrote, so its row is
   // replaced by zero
@@ -1062,7 +1156,8 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
     }
   };
 
-  for (int g = threadIdx.x; g < 2 * WIN; g += PB) hl[g] = 0;
+  int *mark = BIG ? (int *)lyqz : hl;  // the list is formed where Y, Q, Z will be
+  for (int g = threadIdx.x; g < 2 * WIN; g += PB) mark[g] = 0;
   if (threadIdx.x == 0) lds[ZS] = 0.0f;
   __syncthreads();
   double fp2 = 0.0;
@@ -1074,12 +1169,16 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
     const bool own = i < b1;
     const int ic = own ? i : b1 - 1;
     r[k] = u[k] = w[k] = s[k] = p[k] = 0.0f;
-    Y(k) = Q(k) = Z(k) = 0.0f;
     const int s_ = a.ls[ic], n_ = a.ln[ic];
     const float as_i = a.as[ic], aw_i = a.aw[ic], as_n = a.as[n_], aw_e = a.aw[ic + 1];
     const double fpt = a.fptmp[ic];
-    js[k] = own ? s_ : lc0;
-    jn[k] = own ? n_ : lc0;
+    if constexpr (BIG) {
+      const unsigned sl = own && real(s_) ? slot(s_) : ZS, nl = own && real(n_) ? slot(n_) : ZS;
+      jj[k] = sl | nl << 16;
+    } else {
+      js[k] = own ? s_ : lc0;
+      jn[k] = own ? n_ : lc0;
+    }
     as_[k] = own ? as_i : 0.0f;
     aw_[k] = own ? aw_i : 0.0f;
     an_[k] = (own && n_ != lc0) ? as_n : 0.0f;
@@ -1092,19 +1191,24 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
         const int j = nbq[q];
         if (real(j) && !inside(j)) {
           out = true;
-          hl[ghost_of(j, b0, b1)] = 1;
+          mark[ghost_of(j, b0, b1)] = 1;
         }
       }
       if (out) expo |= 1u << k;
     }
     fp2 += own ? fpt * fpt : 0.0;
+    fence(k);
   }
   __syncthreads();
-  const int nhalo = compact_halo(hl, b0, b1);
+  const int nhalo = compact_halo(mark, b0, b1);
   // the workgroups that own the outside cells (hl is sorted)
   const int span = CPT * PB;
-  const int nlo = nhalo > 0 ? (hl[0] - 1) / span : 1;
-  const int nhi = nhalo > 0 ? (hl[nhalo - 1] - 1) / span : 0;
+  const int nlo = nhalo > 0 ? (mark[0] - 1) / span : 1;
+  const int nhi = nhalo > 0 ? (mark[nhalo - 1] - 1) / span : 0;
+  if constexpr (BIG) {
+    for (int h = threadIdx.x; h < nhalo; h += PB) hs[h] = (unsigned short)slot(mark[h]);
+    __syncthreads();  // the list is read before Y takes its place
+  }
 
   unsigned tag = a.tag0, gen = 0;
   double rsqm = a.rsqm, bnorm2 = 0.0, rsq64 = 0.0, bn_in = 0.0;
@@ -1120,7 +1224,15 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
     for (int k = 0; k < CPT; ++k) {
       const int i = b0 + k * PB + (int)threadIdx.x;
       const bool own = i < b1;
-      const int s_ = opaque(js[k]), n_ = opaque(jn[k]);
+      int s_, n_;
+      if constexpr (BIG) {
+        const unsigned q = (unsigned)opaque((int)jj[k]);
+        s_ = cellof((int)(q & 0xffffu));
+        n_ = cellof((int)(q >> 16));
+      } else {
+        s_ = opaque(js[k]);
+        n_ = opaque(jn[k]);
+      }
       const int io = opaque(own ? i : b1 - 1);
       const int ie = io + 1;  // <= lc0
       const double *P = a.x;
@@ -1138,20 +1250,28 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
       Y(k) = 0.0f;
       v3[0] += own ? rr * rr : 0.0;
       v3[1] += own ? (double)rs * (double)rs : 0.0;
+      fence(k);
     }
     post_partials<3>(v3, a.xc, tag);
-    precond(r, u);
+    if constexpr (BIG) {
+      precond_lds(r);
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int i = b0 + k * PB + (int)threadIdx.x;
-      lds[slot(i)] = u[k];
-      if (expo & (1u << k)) put_u32(hxw(i, tag), __float_as_uint(u[k]));
+      for (int k = 0; k < CPT; ++k) u[k] = lds[WIN + k * PB + (int)threadIdx.x];
+      post_rows(tag);
+    } else {
+      precond(r, u);
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        const int i = b0 + k * PB + (int)threadIdx.x;
+        lds[slot(i)] = u[k];
+        if (expo & (1u << k)) put_u32(hxw(i, tag), __float_as_uint(u[k]));
+      }
     }
     fp2 = 0.0;
     post_flag(a.xc, tag);
     {
       double s3[3];
-      if (!exchange<3, 1>(a.xc, tag, hl, nhalo, raw, a.bar, s3)) return;
+      if (!exchange<3, BIG ? 0 : 1>(a.xc, tag, hl, nhalo, raw, a.bar, s3)) return;
       if (outer == 0) {
         bnorm2 = s3[2];
         rsqm = a.rel_tol > 0.0 ? a.rel_tol * a.rel_tol * bnorm2 : a.rsqm;
@@ -1164,9 +1284,14 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
     const double rt2 = fmax(a.rtol2, INNER_MARGIN2 * rsqm / rsq64);
 
     // ---- w0 = A' u0; s, p, q, z start at 0
-    for (int h = threadIdx.x; h < nhalo; h += PB) lds[slot(hl[h])] = __uint_as_float(raw[h]);
-    __syncthreads();
-    spmv(u, w);
+    if constexpr (BIG) {
+      fetch_window32(a.xc, tag, hs, nhalo, b0, lds);
+      spmv_lds(w);
+    } else {
+      for (int h = threadIdx.x; h < nhalo; h += PB) lds[slot(hl[h])] = __uint_as_float(raw[h]);
+      __syncthreads();
+      spmv(u, w);
+    }
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       s[k] = p[k] = 0.0f;
@@ -1184,24 +1309,39 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
         v[0] += (double)r[k] * (double)u[k];
         v[1] += (double)w[k] * (double)u[k];
         v[2] += (double)r[k] * (double)r[k];
+        fence(k);
       }
       post_partials<3>(v, a.xc, tag);
       // ... then m = M^-1 w, its outside values, the flag
-      float m[CPT];
-      precond(w, m);
+      float m[BIG ? 1 : CPT];
+      if constexpr (BIG) {
+        precond_lds(w);
+        post_rows(tag);
+      } else {
+        precond(w, m);
 #pragma unroll
-      for (int k = 0; k < CPT; ++k) {
-        const int i = b0 + k * PB + (int)threadIdx.x;
-        lds[slot(i)] = m[k];
-        if (expo & (1u << k)) put_u32(hxw(i, tag), __float_as_uint(m[k]));
+        for (int k = 0; k < CPT; ++k) {
+          const int i = b0 + k * PB + (int)threadIdx.x;
+          lds[slot(i)] = m[k];
+          if (expo & (1u << k)) put_u32(hxw(i, tag), __float_as_uint(m[k]));
+        }
       }
       post_flag(a.xc, tag);
       // n = A' m once the neighbouring workgroups' m has arrived
-      if (nhalo > 0 && !halo_wait(a.xc, tag, nlo, nhi, hl, nhalo, raw, a.bar)) return;
-      for (int h = threadIdx.x; h < nhalo; h += PB) lds[slot(hl[h])] = __uint_as_float(raw[h]);
-      __syncthreads();
+      if constexpr (BIG) {
+        if (nhalo > 0) {
+          if (!halo_poll(a.xc, tag, nlo, nhi, a.bar)) return;
+          fetch_window32(a.xc, tag, hs, nhalo, b0, lds);
+        }
+        __syncthreads();
+      } else {
+        if (nhalo > 0 && !halo_wait(a.xc, tag, nlo, nhi, hl, nhalo, raw, a.bar)) return;
+        for (int h = threadIdx.x; h < nhalo; h += PB) lds[slot(hl[h])] = __uint_as_float(raw[h]);
+        __syncthreads();
+      }
       float n[CPT];
-      spmv(m, n);
+      if constexpr (BIG) spmv_lds(n);
+      else spmv(m, n);
       // the sums of every workgroup
       double s3[3];
       if (!exchange<3, 0>(a.xc, tag, hl, 0, raw, a.bar, s3)) return;
@@ -1222,7 +1362,8 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
         const float zk = fmaf(bf, Z(k), n[k]);
-        const float qk = fmaf(bf, Q(k), m[k]);
+        const float mk = BIG ? lds[WIN + k * PB + (int)threadIdx.x] : m[BIG ? 0 : k];
+        const float qk = fmaf(bf, Q(k), mk);
         s[k] = fmaf(bf, s[k], w[k]);
         p[k] = fmaf(bf, p[k], u[k]);
         Y(k) = fmaf(af, p[k], Y(k));
@@ -1231,6 +1372,7 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
         w[k] = fmaf(-af, zk, w[k]);
         Z(k) = zk;
         Q(k) = qk;
+        fence(k);
       }
       inner += 1;
       gam_prev = gam;
@@ -1248,6 +1390,7 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
       double *P = a.x;
       const double pn = fetch(&P[io]) + a.dis[io] * (double)Y(k);
       if (own) publish(&P[io], pn);
+      fence(k);
     }
     ++outer;
     if (!grid_barrier(a.bar, ++gen)) return;
@@ -1535,7 +1678,6 @@ int occupancy(K kern) {
 
 // Largest cells-per-thread instantiation of each solve.
 constexpr int PCG64_CPT_MAX = 6;
-constexpr int PCGMX_CPT_MAX = 8;
 // Terms of the workgroup-local preconditioner of the mixed persistent solve
 // when the caller leaves the choice to the library.
 constexpr int PCG_PDEG_DEFAULT = 3;
@@ -1555,19 +1697,22 @@ int pcg_prepare(efdc_ctx *c) {
   const int occ64[PCG64_CPT_MAX + 1] = {
       0, occupancy(k_pcg64<1>), occupancy(k_pcg64<2>), occupancy(k_pcg64<3>),
       occupancy(k_pcg64<4>), occupancy(k_pcg64<5>), occupancy(k_pcg64<6>)};
-  const int occmx[PCGMX_CPT_MAX + 1] = {
+  const int occmx[PCGMX_CPT_SMALL + 1] = {
       0, occupancy(k_pcgmx<1>), occupancy(k_pcgmx<2>), occupancy(k_pcgmx<3>),
       occupancy(k_pcgmx<4>), occupancy(k_pcgmx<5>), occupancy(k_pcgmx<6>),
       occupancy(k_pcgmx<7>), occupancy(k_pcgmx<8>)};
+  // 10, 12, 14 and 16 cells per thread in the pipelined form alone
   const int occpl[PCGMX_CPT_MAX + 1] = {
       0, occupancy(k_pcgmx_pl<1>), occupancy(k_pcgmx_pl<2>), occupancy(k_pcgmx_pl<3>),
       occupancy(k_pcgmx_pl<4>), occupancy(k_pcgmx_pl<5>), occupancy(k_pcgmx_pl<6>),
-      occupancy(k_pcgmx_pl<7>), occupancy(k_pcgmx_pl<8>)};
+      occupancy(k_pcgmx_pl<7>), occupancy(k_pcgmx_pl<8>), 0, occupancy(k_pcgmx_pl<10>), 0,
+      occupancy(k_pcgmx_pl<12>), 0, occupancy(k_pcgmx_pl<14>), 0, occupancy(k_pcgmx_pl<16>)};
   const int occ64p[PCG64_CPT_MAX + 1] = {
       0, occupancy(k_pcg64_pl<1>), occupancy(k_pcg64_pl<2>), occupancy(k_pcg64_pl<3>),
       occupancy(k_pcg64_pl<4>), occupancy(k_pcg64_pl<5>), occupancy(k_pcg64_pl<6>)};
   for (int k = 0; k <= PCG64_CPT_MAX; ++k) c->pcg_occ64[k] = std::min(occ64[k], occ64p[k]);
-  for (int k = 0; k <= PCGMX_CPT_MAX; ++k) c->pcg_occmx[k] = std::min(occmx[k], occpl[k]);
+  for (int k = 0; k <= PCGMX_CPT_MAX; ++k)
+    c->pcg_occmx[k] = k <= PCGMX_CPT_SMALL ? std::min(occmx[k], occpl[k]) : occpl[k];
   c->pcg_ncell = c->n_wet() + 2;
   int s;
   if ((s = dev_alloc(c, &c->pcg_hx,
@@ -1597,6 +1742,18 @@ static int pcg_shape(const efdc_ctx *c, const int *occ, int cpt_max, int &nb) {
   return 0;
 }
 
+// The form of the mixed persistent solve, and its shape: more than 8 cells
+// per thread (1.05 to 2.1 million cells on 256 CUs) in the pipelined form
+// alone, which also runs there while the tuner has found the other faster.
+static bool pcg_pipelined(const efdc_ctx *c) {
+  return c->pcg_pipe_mode == 2 || (c->pcg_pipe_mode == 0 && c->pcg_pipe_tuned);
+}
+static int pcg_shape_mx(const efdc_ctx *c, int &nb) {
+  const int cpt = pcg_shape(c, c->pcg_occmx, PCGMX_CPT_SMALL, nb);
+  if (cpt || c->pcg_pipe_mode == 1) return cpt;
+  return pcg_shape(c, c->pcg_occmx, PCGMX_CPT_MAX, nb);
+}
+
 bool pcg_applicable(efdc_ctx *c, bool mixed) {
   if (c->prm.cg_kernel == EFDC_CG_KERNEL_MULTI) return false;
   if (c->band > WIN) return false;  // a neighbour beyond the LDS window
@@ -1607,7 +1764,7 @@ bool pcg_applicable(efdc_ctx *c, bool mixed) {
     return false;
   if (pcg_prepare(c) != EFDC_OK || c->pcg_ncu == 0) return false;
   int nb = 0;
-  return mixed ? pcg_shape(c, c->pcg_occmx, PCGMX_CPT_MAX, nb) > 0
+  return mixed ? pcg_shape_mx(c, nb) > 0
                : pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb) > 0;
 }
 
@@ -1709,7 +1866,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
     TIMED(c, TK_PCG64, s = coop_launch(c, fn, nb, a));
     if (s) return s;
   } else {
-    const int cpt = pcg_shape(c, c->pcg_occmx, PCGMX_CPT_MAX, nb);
+    const int cpt = pcg_shape_mx(c, nb);
     if (!cpt) { c->err = "persistent CG: problem too large"; return EFDC_ERR_ARG; }
     if (!c->mx_coef_ok) {
       const int n = c->n_wet();
@@ -1744,7 +1901,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
     a.pdeg = c->prm.mixed_precond_degree > 0 ? c->prm.mixed_precond_degree
              : c->pcg_pdeg_tuned > 0         ? c->pcg_pdeg_tuned
                                              : PCG_PDEG_DEFAULT;
-    const bool pl = c->pcg_pipe_mode == 2 || (c->pcg_pipe_mode == 0 && c->pcg_pipe_tuned);
+    const bool pl = cpt > PCGMX_CPT_SMALL || pcg_pipelined(c);
     const void *fn = nullptr;
     if (pl) {
       switch (cpt) {
@@ -1755,7 +1912,11 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
         case 5: fn = (const void *)k_pcgmx_pl<5>; break;
         case 6: fn = (const void *)k_pcgmx_pl<6>; break;
         case 7: fn = (const void *)k_pcgmx_pl<7>; break;
-        default: fn = (const void *)k_pcgmx_pl<8>; break;
+        case 8: fn = (const void *)k_pcgmx_pl<8>; break;
+        case 10: fn = (const void *)k_pcgmx_pl<10>; break;
+        case 12: fn = (const void *)k_pcgmx_pl<12>; break;
+        case 14: fn = (const void *)k_pcgmx_pl<14>; break;
+        default: fn = (const void *)k_pcgmx_pl<16>; break;
       }
     } else {
       switch (cpt) {
@@ -1812,7 +1973,10 @@ int pcg_tune_degree(efdc_ctx *c) {
   int best = PCG_PDEG_DEFAULT, best_slot = -1;
   // the degrees are timed in the Chronopoulos-Gear form when the caller
   // leaves the form to the tuner
-  if (c->pcg_pipe_mode == 0) c->pcg_pipe_tuned = false;
+  // (past 8 cells per thread there is only the pipelined one)
+  int tnb = 0;
+  const bool forms = c->pcg_pipe_mode == 0 && pcg_shape_mx(c, tnb) <= PCGMX_CPT_SMALL;
+  if (forms) c->pcg_pipe_tuned = false;
   for (int j = 0; j < 5; ++j) {
     c->pcg_pdeg_tuned = cand[j];
     float tot = 0.f;
@@ -1841,7 +2005,7 @@ int pcg_tune_degree(efdc_ctx *c) {
   }
   c->pcg_pdeg_tuned = best;
   // the pipelined form at that degree, when the caller leaves the choice
-  if (c->pcg_pipe_mode == 0) {
+  if (forms) {
     c->pcg_pipe_tuned = true;
     float tot = 0.f;
     for (int r = 0; r < 3; ++r) {

@@ -349,3 +349,28 @@ def test_fp64_pipelined_form_in_steps(oracle_mod):
             a, b = ctx.get(name)[i], ref.h[name][i]
             assert np.max(np.abs(a - b)) <= 1e-9 * max(1.0, np.max(np.abs(b))), name
     ctx.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(1100, 960), (1500, 1000), (1700, 1050), (2048, 1020)])
+def test_mixed_persistent_many_cells_per_thread(nx, ny):
+    """The pipelined mixed solve with 10, 12, 14 and 16 cells per thread (the
+    last with the widest band the LDS window takes and nearly every CU's
+    rows full) against the multi-kernel mixed solve: both end at a relative
+    residual of 1e-10, P = g eta of order 1 m2/s2 and a condition number of a few
+    hundred at most, so eta agrees to 1e-7 m."""
+    from efdc_amd import grids, lib
+    wet = np.pad(np.ones((ny, nx), bool), 1)
+    wet[ny // 2, 5:nx // 3] = False
+    case = grids.external_case(wet, seed=nx, depth_sigma=1.0, eta_smooth=1.0)
+    kw = dict(cg_mode=lib.CG_MIXED, cg_rel_tol=1e-10, RSQM=0.0, ITERM=1000)
+    a = lib.Context(case.grid, cg_kernel=lib.CG_KERNEL_PERSISTENT, **kw).upload_case(case)
+    b = lib.Context(case.grid, cg_kernel=lib.CG_KERNEL_MULTI, **kw).upload_case(case)
+    for n in (1, 2):
+        sa = a.calpuv2c(case.dt, n)
+        sb = b.calpuv2c(case.dt, n)
+        assert sa["iters"] < sb["iters"] and sa["rsq"] <= sa["rsqm"]
+    i = wet_index(case)
+    assert a.cg_launch() == (0, 0)
+    assert eta_err(a.get("P")[i], b.get("P")[i]) <= 1e-7
+    a.close()
+    b.close()
