@@ -367,10 +367,333 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_uvw_col(UvwArgs<T> a) {
   a.vhe[i] = face_column<T, KM, EXACT>(a, i, true, rcy);
 }
 
+constexpr int UVW_LAY_CT = 9;  // layer constants k_uvw_lay keeps in LDS
+// the workgroup's whole LDS of k_uvw_lay, in bytes (it has no static part)
+template <typename T>
+size_t uvw_lay_lds(int KC) {
+  return 64 * ((3 * (size_t)(KC - 1) + KC) * 8 + (size_t)(KC - 1) * sizeof(T)) +
+         (size_t)KC * UVW_LAY_CT * 8;
+}
+
+// The layer counts with a k_uvw_col of their own (straight-line layer loops).
+constexpr bool uvw_exact(int KC) {
+  return (KC >= 2 && KC <= 6) || KC == 8 || KC == 10 || KC == 12 || KC == 16 || KC == 20;
+}
+
+// Whether the columns take k_uvw_lay.  Up to 560 tiles of 64 cells k_uvw_col
+// has a wave for half of the 1024 SIMDs and every wave waits for its own loads
+// (us a call, layers : columns, FP32 storage; 544 tiles 5 layers 16.2 : 17.8,
+// 10 22.1 : 26.5, 20 44.7 : 50.7, 24 67.6 : 95.5; 128 tiles 20 layers 24.8 :
+// 47.2; but 2 layers 13.9 : 11.3).  From there to one wave a SIMD the columns
+// are faster where they have straight-line code (938 tiles, 10 layers 34.5 :
+// 30.0, 20 72.1 : 64.4), beyond it only below 12 layers (4000 tiles, 10 layers
+// 112 : 105, 12 136 : 177, 16 185 : 215, 20 269 : 277).  Other counts above 8
+// predicate each layer of a larger instance, which is slower at any size (4000
+// tiles, 9 layers 100 : 182; 938 tiles, 13 38 : 66) as long as two workgroups
+// fit a CU's LDS (FP64, 1875 tiles, 32 layers 436 : 306).
+template <typename T>
+bool uvw_lay(int KC, int tiles) {
+  if (tiles <= 560) return KC >= 4 && uvw_lay_lds<T>(KC) <= 160 * 1024;
+  if (uvw_exact(KC)) return KC >= 12 && tiles > 1024;
+  return KC > 8 && uvw_lay_lds<T>(KC) <= 80 * 1024;
+}
+
+// The column step of k_uvw_col with the layers of a face column side by side:
+// a workgroup owns 64 U faces (blockIdx.y = 0) or V faces (1).  Its waves take
+// the layers (wave w the layers w, w + 4, ..) to form the internal shears, split
+// the external flow and stage SUB3D, AVUI and the shear in LDS; one wave runs
+// the sweeps and sums of the columns from LDS in the reference's order; all
+// waves write the layer flows and velocities.  Every value and operation order
+// is that of face_column, so the bits are the same.
+// Bound: the chain of FP64 divides and sums of the solving wave, which the
+// other workgroups of the CU (three at KC = 20) cover with their loads and
+// stores; a thread per column holds the whole column in 512 registers, one
+// wave per SIMD, and waits for its own loads.
+template <typename T>
+__global__ __launch_bounds__(256) void k_uvw_lay(UvwArgs<T> a) {
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int i = xcd_tile(blockIdx.x, gridDim.x) * 64 + lane;
+  const bool vface = blockIdx.y == 1;
+  const int KC = a.KC, KS = KC - 1;
+  const int64_t P = a.P;
+  const LayerConsts &C = *a.lc;
+  // LDS, stride 64: shear (then DU), AVUI, CU, UUU (then the layer flows), SUB3D
+  double *sd = lds + lane, *sa = sd + (size_t)KS * 64, *sc = sa + (size_t)KS * 64,
+         *su = sc + (size_t)KS * 64;
+  // the layer constants the solving wave reads (through LDS: scalar loads in
+  // its loops would make every LDS read wait with them)
+  constexpr int CT = UVW_LAY_CT;
+  double *ct = lds + (size_t)(3 * KS + KC) * 64;
+  T *ss = (T *)(ct + (size_t)KC * CT) + lane;
+  for (int t = threadIdx.x; t < KC * CT; t += 256) {
+    const int k = t / CT, q = t % CT;
+    ct[t] = q == 0 ? C.cdzl[k] : q == 1 ? C.cdzm[k] : q == 2 ? C.cdzu[k] : q == 3 ? C.cdzr[k]
+          : q == 4 ? C.dzg[k] : q == 5 ? C.cdzd[k] : q == 6 ? C.sg[k]
+          : q == 7 ? C.cerr[k] : C.cerr_closed[k];
+  }
+  const bool act = i >= 1 && i <= a.nwet;
+  const bool wet = act && wet_at(a, i);
+  const double *avi = vface ? a.avvi : a.avui;
+  const double *din = vface ? a.dv : a.du;
+  double *vel1 = vface ? a.v1 : a.u1;
+  const T *s3d = vface ? a.svb3d : a.sub3d;
+  double *flowf = vface ? a.vhdxf : a.uhdyf;
+  double *flow = vface ? a.vhdx : a.uhdy;
+  double *vel = vface ? a.v : a.u;
+  double *ek = vface ? a.vhdxek : a.uhdyek;
+  const double *extp = vface ? a.vhdxe : a.uhdye;
+  bool open = false, nb_dry = false;
+  double hh = 0.0, hhi = 0.0, sb = 0.0, ext = 0.0;
+  const bool dscale = a.isdry > 0;
+  if (wet) {
+    open = (vface ? a.svbo[i] : a.subo[i]) > 0.0;
+    hh = vface ? a.hv[i] : a.hu[i];
+    hhi = vface ? a.hvi[i] : a.hui[i];
+    sb = vface ? a.svb[i] : a.sub[i];
+    ext = extp[i];
+    const double h1 = vface ? a.h1v[i] : a.h1u[i];
+    const double ts = vface ? a.tsy[i] : a.tsx[i];
+    const double de = ext - extp[vface ? a.ln[i] : a.le[i]];
+    // the old level of a face shared with a dry cell is zero (:230-262)
+    nb_dry = a.lmask != nullptr && a.lmask[vface ? a.ls[i] : a.lw[i]] == 0;
+    for (int k = wv; k < KC; k += 4) {
+      const int64_t j = i + (int64_t)k * P;
+      if (nb_dry) {
+        (vface ? a.vhdx1 : a.uhdy1)[j] = 0.0;
+        (vface ? a.vhdxf1 : a.uhdyf1)[j] = 0.0;
+        vel1[j] = 0.0;
+      }
+      if (k >= KS) continue;
+      const double av = avi[j];
+      const T s3 = s3d[j];
+      const double dz = (double)a.dzc[j];
+      double d;
+      if (a.shear) {
+        const double r0 = vel1[j], r1 = vel1[j + P];
+        const double v0 = nb_dry ? 0.0 : r0, v1 = nb_dry ? 0.0 : r1;
+        const double cf = open ? C.cdzf[k] : 0.0;
+        d = cf * (h1 * (v1 - v0) * a.dti + 0.0);
+        if (a.wind && k == KS - 1) d = d - (open ? C.cdzu[k] : 0.0) * ts;
+      } else {
+        d = din[j];
+      }
+      ek[j] = dz * de;  // the external flow split by layer (:332-345)
+      sd[k * 64] = (dscale ? sb * (double)s3 : (double)s3) * d;
+      sa[k * 64] = av;
+      ss[k * 64] = s3;
+    }
+  } else if (act) {
+    // a dry cell, as zero_dry_column: the U arrays (and W) by the U
+    // faces' workgroup, the V arrays by the V faces'
+    for (int k = wv; k < KC; k += 4) {
+      const int64_t j = i + (int64_t)k * P;
+      flowf[j] = flow[j] = vel[j] = 0.0;
+      (vface ? a.vhdxf1 : a.uhdyf1)[j] = (vface ? a.vhdx1 : a.uhdy1)[j] = vel1[j] = 0.0;
+      (vface ? a.vhdxf2 : a.uhdyf2)[j] = 0.0;
+      (vface ? a.vhdx2 : a.uhdy2)[j] = (vface ? a.v2 : a.u2)[j] = (T)0;
+      ek[j] = (vface ? a.vhdx1ek : a.uhdy1ek)[j];
+      if (!vface) {
+        a.w[j + P] = a.w1[j + P] = 0.0;
+        a.w2[j + P] = (T)0;
+      }
+    }
+    if (wv == 0) (vface ? a.tvarn : a.tvare)[i] = 0.0;
+  }
+  __syncthreads();
+  if (wet && wv == 0) {
+    // bottom drag coefficient, ISTL = 2 (:296-330); U = U1 here
+    const double b1 = nb_dry ? 0.0 : vel1[i];
+    const double x1 = vface ? a.u1v[i] : a.v1u[i], x0 = vface ? a.uv[i] : a.vu[i];
+    const double q1 = sqrt(b1 * b1 + x1 * x1), q2 = sqrt(b1 * b1 + x0 * x0);
+    const double st = vface ? a.stby[i] : a.stbx[i];
+    const double h1 = vface ? a.h1v[i] : a.h1u[i];
+    const double rc = a.avcon1 < 0.00001 ? st * sqrt(q1 * q2)
+                                         : a.avcon1 / sqrt(h1 * hh) + st * sqrt(q1 * q2);
+    double *uhep = vface ? a.vhe : a.uhe;
+    double uhe = uhep[i];
+    const double dti = a.dti;
+    auto s3of = [&](int k) { return dscale ? sb * (double)ss[k * 64] : (double)ss[k * 64]; };
+    // Every loop takes its values from LDS four layers at a time, before
+    // the chunk's stores (a load after a store would wait for it).
+    constexpr int U = 4;
+    // forward sweep (:419-486)
+    double cu = 0.0, du = 0.0, uu = 0.0;
+    for (int k0 = 0; k0 < KS; k0 += U) {
+      double av[U], d[U], zl[U], zm[U], zu[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = min(k0 + q, KS - 1);
+        av[q] = sa[k * 64];
+        d[q] = sd[k * 64];
+        zl[q] = ct[k * CT + 0];
+        zm[q] = ct[k * CT + 1];
+        zu[q] = ct[k * CT + 2];
+      }
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = k0 + q;
+        if (k >= KS) break;
+        const double cl = open ? zl[q] : 0.0;
+        const double cm = (open ? zm[q] : 0.0) * dti;
+        const double cuu = open ? zu[q] : 0.0;
+        const double cmu = 1. + cm * hh * av[q];
+        if (k > 0) {
+          const double eu = 1. / (cmu - cl * cu);
+          cu = cuu * eu;
+          du = (d[q] - cl * du) * eu;
+          uu = -cl * uu * eu;
+        } else {
+          const double eu = 1. / cmu;
+          cu = cuu * eu;
+          du = (d[q] - cl * rc * uhe * hhi) * eu;
+          uu = eu;
+        }
+        sc[k * 64] = cu;
+        sd[k * 64] = du;
+        su[k * 64] = uu;
+      }
+    }
+    // back substitution (:477-486)
+    for (int k0 = KS - 2; k0 >= 0; k0 -= U) {
+      double c[U], d[U], w[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = max(k0 - q, 0);
+        c[q] = sc[k * 64];
+        d[q] = sd[k * 64];
+        w[q] = su[k * 64];
+      }
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = k0 - q;
+        if (k < 0) break;
+        du = d[q] - c[q] * du;
+        uu = w[q] - c[q] * uu;
+        sd[k * 64] = du;
+        su[k * 64] = uu;
+      }
+    }
+    // Sherman-Morrison step for the bottom drag (:489-524)
+    double aa = 0., bb = 1.;
+    for (int k0 = 0; k0 < KS; k0 += U) {
+      double av[U], d[U], w[U], zr[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = min(k0 + q, KS - 1);
+        av[q] = sa[k * 64];
+        d[q] = sd[k * 64];
+        w[q] = su[k * 64];
+        zr[q] = ct[k * CT + 3];
+      }
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        if (k0 + q >= KS) break;
+        const double cr = (open ? zr[q] : 0.0) * rc * av[q];
+        aa = aa + cr * d[q];
+        bb = bb + cr * w[q];
+      }
+    }
+    aa = aa / bb;
+    // layer flows (:527-567)
+    for (int k0 = 0; k0 < KS; k0 += U) {
+      double av[U], d[U], w[U], zg[U], zd[U], s3[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = min(k0 + q, KS - 1);
+        av[q] = sa[k * 64];
+        d[q] = sd[k * 64];
+        w[q] = su[k * 64];
+        s3[q] = s3of(k);
+        zg[q] = ct[k * CT + 4];
+        zd[q] = ct[k * CT + 5];
+      }
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        if (k0 + q >= KS) break;
+        const double x = s3[q] * (open ? zg[q] : 0.0) * hh * av[q] * (d[q] - aa * w[q]);
+        sd[(k0 + q) * 64] = x;
+        uhe = uhe + (open ? zd[q] : 0.0) * x;
+      }
+    }
+    const double width = vface ? a.dxv[i] : a.dyu[i];
+    double f = uhe * sb;
+    su[KS * 64] = f * width;
+    for (int k0 = KS - 1; k0 >= 0; k0 -= U) {
+      double d[U], s3[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = max(k0 - q, 0);
+        d[q] = sd[k * 64];
+        s3[q] = s3of(k);
+      }
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        if (k0 - q < 0) break;
+        f = s3[q] * (f - d[q]);
+        su[(k0 - q) * 64] = f * width;
+      }
+    }
+    // correction to the external solution (:571-611)
+    double tv = 0.;
+    for (int k0 = 0; k0 < KC; k0 += U) {
+      double w[U], zs[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = min(k0 + q, KC - 1);
+        w[q] = su[k * 64];
+        zs[q] = ct[k * CT + 6];
+      }
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+        if (k0 + q < KC) tv = tv + w[q] * (open ? zs[q] : 0.0);
+    }
+    tv = tv - ext;
+    double un = 0.;
+    for (int k0 = 0; k0 < KC; k0 += U) {
+      double w[U], zs[U], ze[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int k = min(k0 + q, KC - 1);
+        w[q] = su[k * 64];
+        zs[q] = ct[k * CT + 6];
+        ze[q] = ct[k * CT + (open ? 7 : 8)];
+      }
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        if (k0 + q >= KC) break;
+        const double g = w[q] - tv * ze[q];
+        su[(k0 + q) * 64] = g;
+        un = un + g * (open ? zs[q] : 0.0);
+      }
+    }
+    uhep[i] = un * (vface ? a.dxiv[i] : a.dyiu[i]);
+  }
+  __syncthreads();
+  if (wet) {
+    const double widthi = vface ? a.dxiv[i] : a.dyiu[i];
+    for (int k = wv; k < KC; k += 4) {
+      const int64_t j = i + (int64_t)k * P;
+      const double f = su[k * 64];
+      flowf[j] = f;
+      flow[j] = f * (open ? C.sg[k] : 0.0);
+      // velocities (:613-647): two roundings as in the reference
+      const double ve = f * hhi;
+      vel[j] = ve * widthi;
+    }
+  }
+}
+
 // W from the layer continuity, ISTL = 2 (:665-683), zero on LOBCS cells
 // (:687-694); the averages of the two levels (:770-791) and the column sums
-// of the averaged layer flows (:813-836).
-template <typename T>
+// of the averaged layer flows (:813-836), one pass over the layers.
+// Bound by memory.  With more than one layer the new level's UHDY = UHDYF*SGZU,
+// U = UHDYF*HUI*DYIU and UHDYEK = DZC*(difference of UHDYE) are formed again,
+// with the column kernel's operations (the same bits), from the UHDYF plane
+// that the averages read anyway: six planes of FP64 less than reading them
+// back, 2.8 instead of 3.8 KB a column at KC = 20.
+template <typename T, bool LAYERS>
 __global__ __launch_bounds__(EFDC_BLOCK) void k_uvw_w(UvwArgs<T> a) {
   const int i = uvw_cell(a.nwet);
   if (i > a.nwet || !wet_at(a, i)) return;
@@ -379,29 +702,55 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_uvw_w(UvwArgs<T> a) {
   const int e = a.le[i], n = a.ln[i];
   const bool obc = (a.lobflag[i] & 1) != 0;
   const double dxyip = a.dxyip[i], qsume = a.qsume[i], half = 0.5 * dxyip;
+  const LayerConsts &C = *a.lc;
+  const bool ge = e == a.lc0, gn = n == a.lc0;  // land: the ghost's own entries
+  const bool ou = a.subo[i] > 0.0, ov = a.svbo[i] > 0.0, oe = a.subo[e] > 0.0,
+             on = a.svbo[n] > 0.0;
+  const double hui = a.hui[i], hvi = a.hvi[i], dyiu = a.dyiu[i], dxiv = a.dxiv[i];
+  const double de = a.uhdye[i] - a.uhdye[e], dn = a.vhdxe[i] - a.vhdxe[n];
+  const double *pe = LAYERS && !ge ? a.uhdyf : a.uhdy, *pn = LAYERS && !gn ? a.vhdxf : a.vhdx;
   double wprev = a.w[i];
-  for (int k = 0; k < KC - 1; ++k) {
-    const int64_t j = i + k * P, je = e + k * P, jn = n + k * P;
-    const double wk =
-        wprev -
-        half * (a.uhdy[je] - a.uhdy[j] + a.uhdyek[j] + a.uhdy1[je] - a.uhdy1[j] + a.uhdy1ek[j] +
-                a.vhdx[jn] - a.vhdx[j] + a.vhdxek[j] + a.vhdx1[jn] - a.vhdx1[j] + a.vhdx1ek[j]) +
-        ((double)a.qsum[j] - (double)a.dzc[j] * qsume) * dxyip;
-    a.w[j + P] = obc ? 0.0 : wk;
-    wprev = wk;
-  }
   double te = 0.0, tn = 0.0;
   for (int k = 0; k < KC; ++k) {
-    const int64_t j = i + k * P;
-    a.uhdyf2[j] = 0.5 * (a.uhdyf[j] + a.uhdyf1[j]);
-    a.vhdxf2[j] = 0.5 * (a.vhdxf[j] + a.vhdxf1[j]);
-    const double uh2 = 0.5 * (a.uhdy[j] + a.uhdy1[j]);
-    const double vh2 = 0.5 * (a.vhdx[j] + a.vhdx1[j]);
+    const int64_t j = i + k * P, je = e + k * P, jn = n + k * P;
+    const double fu = a.uhdyf[j], fv = a.vhdxf[j], fu1 = a.uhdyf1[j], fv1 = a.vhdxf1[j];
+    const double uy1 = a.uhdy1[j], vx1 = a.vhdx1[j], w1k = a.w1[j + P];
+    double uy, vx, un, vn;
+    if (LAYERS) {
+      const double sg = C.sg[k];
+      uy = fu * (ou ? sg : 0.0);
+      vx = fv * (ov ? sg : 0.0);
+      un = fu * hui * dyiu;
+      vn = fv * hvi * dxiv;
+    } else {
+      uy = a.uhdy[j];
+      vx = a.vhdx[j];
+      un = a.u[j];
+      vn = a.v[j];
+    }
+    double wk = 0.0;
+    if (k < KC - 1) {
+      const double qe = pe[je], qn = pn[jn], dz = (double)a.dzc[j];
+      const double uye = LAYERS && !ge ? qe * (oe ? C.sg[k] : 0.0) : qe;
+      const double vxn = LAYERS && !gn ? qn * (on ? C.sg[k] : 0.0) : qn;
+      const double uek = LAYERS ? dz * de : a.uhdyek[j], vek = LAYERS ? dz * dn : a.vhdxek[j];
+      wk = wprev - half * (uye - uy + uek + a.uhdy1[je] - uy1 + a.uhdy1ek[j] + vxn - vx + vek +
+                           a.vhdx1[jn] - vx1 + a.vhdx1ek[j]) +
+           ((double)a.qsum[j] - dz * qsume) * dxyip;
+      wprev = wk;
+      wk = obc ? 0.0 : wk;
+      a.w[j + P] = wk;
+    } else {
+      wk = a.w[j + P];
+    }
+    a.uhdyf2[j] = 0.5 * (fu + fu1);
+    a.vhdxf2[j] = 0.5 * (fv + fv1);
+    const double uh2 = 0.5 * (uy + uy1), vh2 = 0.5 * (vx + vx1);
     a.uhdy2[j] = (T)uh2;
     a.vhdx2[j] = (T)vh2;
-    a.u2[j] = (T)(0.5 * (a.u[j] + a.u1[j]));
-    a.v2[j] = (T)(0.5 * (a.v[j] + a.v1[j]));
-    a.w2[j + P] = (T)(0.5 * (a.w[j + P] + a.w1[j + P]));
+    a.u2[j] = (T)(0.5 * (un + a.u1[j]));
+    a.v2[j] = (T)(0.5 * (vn + a.v1[j]));
+    a.w2[j + P] = (T)(0.5 * (wk + w1k));
     te = te + uh2;
     tn = tn + vh2;
   }
@@ -482,52 +831,63 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_uvw_obc_side(UvwArgs<T> a, UvwOb
 }
 
 // The averages, W2 and column sums of the cells whose faces or W the sides
-// changed: one thread per listed cell.
+// changed: one thread per (layer, listed cell) for the averages and, past
+// them, one per cell for the sums, in the order of the layers and with all of
+// a batch's loads in flight (a thread per cell that walked its layers,
+// storing as it went, took 100 us for 400 cells of 20 layers: every layer's
+// loads waited for the stores before them).
 template <typename T>
 __global__ __launch_bounds__(EFDC_BLOCK) void k_uvw_obc_avg(UvwArgs<T> a, UvwObcDev b) {
   const int KC = a.KC;
   const int64_t P = a.P;
   int q = blockIdx.x * EFDC_BLOCK + (int)threadIdx.x;
-  if (q < b.navg_u) {
-    const int x = b.avg_u[q];
+  if (q < b.navg_u * KC) {
+    const int x = b.avg_u[q % b.navg_u];
     if (!wet_at(a, x)) return;
-    double te = 0.0;
-    for (int k = 0; k < KC; ++k) {
-      const int64_t j = x + k * P;
-      a.uhdyf2[j] = 0.5 * (a.uhdyf[j] + a.uhdyf1[j]);
-      const double uh2 = 0.5 * (a.uhdy[j] + a.uhdy1[j]);
-      a.uhdy2[j] = (T)uh2;
-      a.u2[j] = (T)(0.5 * (a.u[j] + a.u1[j]));
-      te = te + uh2;
-    }
-    a.tvare[x] = te;
+    const int64_t j = x + (q / b.navg_u) * P;
+    a.uhdyf2[j] = 0.5 * (a.uhdyf[j] + a.uhdyf1[j]);
+    a.uhdy2[j] = (T)(0.5 * (a.uhdy[j] + a.uhdy1[j]));
+    a.u2[j] = (T)(0.5 * (a.u[j] + a.u1[j]));
     return;
   }
-  q -= b.navg_u;
-  if (q < b.navg_v) {
-    const int x = b.avg_v[q];
+  q -= b.navg_u * KC;
+  if (q < b.navg_v * KC) {
+    const int x = b.avg_v[q % b.navg_v];
     if (!wet_at(a, x)) return;
-    double tn = 0.0;
-    for (int k = 0; k < KC; ++k) {
-      const int64_t j = x + k * P;
-      a.vhdxf2[j] = 0.5 * (a.vhdxf[j] + a.vhdxf1[j]);
-      const double vh2 = 0.5 * (a.vhdx[j] + a.vhdx1[j]);
-      a.vhdx2[j] = (T)vh2;
-      a.v2[j] = (T)(0.5 * (a.v[j] + a.v1[j]));
-      tn = tn + vh2;
-    }
-    a.tvarn[x] = tn;
+    const int64_t j = x + (q / b.navg_v) * P;
+    a.vhdxf2[j] = 0.5 * (a.vhdxf[j] + a.vhdxf1[j]);
+    a.vhdx2[j] = (T)(0.5 * (a.vhdx[j] + a.vhdx1[j]));
+    a.v2[j] = (T)(0.5 * (a.v[j] + a.v1[j]));
     return;
   }
-  q -= b.navg_v;
-  if (q < b.nwz) {
-    const int x = b.wz[q];
+  q -= b.navg_v * KC;
+  if (q < b.nwz * KC) {
+    const int x = b.wz[q % b.nwz];
     if (!wet_at(a, x)) return;
-    for (int k = 0; k < KC; ++k) {
-      const int64_t j = x + k * P;
-      a.w2[j + P] = (T)(0.5 * (a.w[j + P] + a.w1[j + P]));
-    }
+    const int64_t j = x + (q / b.nwz) * P;
+    a.w2[j + P] = (T)(0.5 * (a.w[j + P] + a.w1[j + P]));
+    return;
   }
+  q -= b.nwz * KC;
+  if (q >= b.navg_u + b.navg_v) return;
+  const bool vf = q >= b.navg_u;
+  const int x = vf ? b.avg_v[q - b.navg_u] : b.avg_u[q];
+  if (!wet_at(a, x)) return;
+  const double *f0 = (vf ? a.vhdx : a.uhdy) + x, *f1 = (vf ? a.vhdx1 : a.uhdy1) + x;
+  double sum = 0.0;
+  for (int k0 = 0; k0 < KC; k0 += 8) {
+    double x0[8], x1[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t o = (int64_t)(k0 + u < KC ? k0 + u : KC - 1) * P;
+      x0[u] = f0[o];
+      x1[u] = f1[o];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (k0 + u < KC) sum = sum + 0.5 * (x0[u] + x1[u]);
+  }
+  (vf ? a.tvarn : a.tvare)[x] = sum;
 }
 
 // The depth from the layer flows, 2TL (:949-1040), HP of open-boundary
@@ -866,7 +1226,11 @@ int uvw_launch(efdc_ctx *c, const efdc_step_t *st, const efdc_uvw_opts_t *o) {
   const UvwArgs<T> a = uvw_args<T>(c, st, o);
   const int nb = efdc_grid_blocks(c->n_wet() + 1);
   const int KC = c->KC;
-  switch (KC) {  // the common layer counts get a kernel of their own
+  const int tiles = (c->n_wet() + 64) / 64;
+  if (uvw_lay<T>(KC, tiles)) {
+    TIMED(c, TK_UVW_COL,
+          (k_uvw_lay<T><<<dim3(tiles, 2), 256, uvw_lay_lds<T>(KC), c->stream>>>(a)));
+  } else switch (KC) {  // the common layer counts get a kernel of their own
 #define UVW_EXACT(n)                                                                     \
   case n:                                                                                \
     TIMED(c, TK_UVW_COL, k_uvw_col<T, n, true><<<nb, EFDC_BLOCK, 0, c->stream>>>(a)); \
@@ -877,16 +1241,15 @@ int uvw_launch(efdc_ctx *c, const efdc_step_t *st, const efdc_uvw_opts_t *o) {
     default:
       if (KC <= 8)
         TIMED(c, TK_UVW_COL, k_uvw_col<T, 8, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
-      else if (KC <= 16)
-        TIMED(c, TK_UVW_COL, k_uvw_col<T, 16, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
-      else if (KC <= 24)
-        TIMED(c, TK_UVW_COL, k_uvw_col<T, 24, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
-      else if (KC <= 32)
+      else if (KC <= 32)  // (9 to 31 take k_uvw_lay)
         TIMED(c, TK_UVW_COL, k_uvw_col<T, 32, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
       else
         TIMED(c, TK_UVW_COL, k_uvw_col<T, 64, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
   }
-  TIMED(c, TK_UVW_W, k_uvw_w<T><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
+  if (KC > 1)
+    TIMED(c, TK_UVW_W, (k_uvw_w<T, true><<<nb, EFDC_BLOCK, 0, c->stream>>>(a)));
+  else
+    TIMED(c, TK_UVW_W, (k_uvw_w<T, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a)));
   const UvwObcDev &b = u->obc;
   if (b.n[0] + b.n[1] + b.n[2] + b.n[3] > 0) {
     for (int side = 0; side < 4; ++side) {
@@ -895,7 +1258,7 @@ int uvw_launch(efdc_ctx *c, const efdc_step_t *st, const efdc_uvw_opts_t *o) {
       TIMED(c, TK_UVW_OBC,
             k_uvw_obc_side<T><<<nt, EFDC_BLOCK, 0, c->stream>>>(a, b, side));
     }
-    const int na = b.navg_u + b.navg_v + b.nwz;
+    const int na = (b.navg_u + b.navg_v + b.nwz) * KC + b.navg_u + b.navg_v;
     if (na > 0)
       TIMED(c, TK_UVW_OBC, k_uvw_obc_avg<T><<<(na + EFDC_BLOCK - 1) / EFDC_BLOCK, EFDC_BLOCK,
                                                0, c->stream>>>(a, b));
