@@ -13,20 +13,24 @@
 //     neighbour outside the range) and the dot-product partials, as
 //     tagged words in memory.
 //
-// Exchange protocol.  A workgroup writes the values its neighbours need
-// (halo values, into a slot of the exchange's parity) and its dot-product
-// partials with agent-scope stores, which are written through to the
-// coherent memory side; every wave waits for its stores to complete
-// (s_waitcnt), and then thread 0 stores the exchange number into the
-// workgroup's flag word (one 128-byte line per workgroup).  A reader polls
-// the flag words of all workgroups (thread q reads workgroup q's flag)
-// until every one carries the exchange number, and then fetches the
-// partials and the halo values it needs in a single round of loads.  Two
-// slot parities suffice: a workgroup can only write exchange T+2 after it
-// has seen every flag of T+1, and every workgroup raises T+1 only after it
-// has consumed T.  Exchange numbers grow across launches (the host numbers
-// launches), so flags never go backwards; when the numbering wraps the host
-// clears them.
+// Exchange protocol.  Every word that crosses workgroups is 64 bits: 32
+// bits of data and, above them, the number of the exchange (a double is two
+// such words).  The writer stores them with agent-scope atomic stores, which
+// are written through to the coherent memory side, and waits for nothing; a
+// reader polls the words that it needs themselves until every one carries
+// the number.  So an exchange is one trip through memory: with flag words,
+// the writer waited for its stores before raising its flag and the reader
+// fetched the data after seeing it, three trips (us a solve, flags : tagged
+// words; FP64, 29 iterations, 5 k cells 178 : 105, 79 k 216 : 131; mixed, 17
+// to 20 inner iterations, 79 k 126 : 103, 696 k 161 : 151).  A slot of
+// partials is 48 bytes a workgroup: packed closer, the workgroups' stores to
+// one 128-byte line delay each other (79 k FP64 160 : 194), spread over a line
+// each, every poll reads more lines (169).
+// Two slot parities suffice: a workgroup can only write exchange T+2 after
+// it has read every workgroup's sums of T+1, and every workgroup posts those
+// only after it has consumed T.  Exchange numbers grow across launches (the
+// host numbers launches), so a slot never holds a number yet to come; when
+// the numbering wraps the host clears the slots.
 //
 // FP64 (the reference's Jacobi-PCG, EFDC/congrad.f90:52-187): the same
 // recurrences and stop test as the reference, two exchanges per iteration
@@ -61,14 +65,9 @@ constexpr double INNER_MARGIN2 = 1e-2;
 constexpr int WIN = 2048;         // LDS window reach beyond the own range
 constexpr int HMAX = 2 * WIN;     // outside cells of one workgroup, at most
 constexpr int NVMAX = 3;          // partials per exchange, at most
+constexpr int PCG64_CPT_MAX = 6;     // cells per thread, FP64
 constexpr int PCGMX_CPT_SMALL = 8;  // cells per thread of every mixed form
 constexpr int PCGMX_CPT_MAX = 16;   // of the pipelined form alone
-constexpr int HX_WORDS = 4;       // 4-byte words per cell and parity in the halo slots
-
-// Halo slots are planes (one per value and parity), so that the stores of
-// a wave and the loads of a run of outside cells are contiguous: FP32
-// value q of cell i in parity p at word (p*HX_WORDS + q)*ncell + i, FP64
-// value q (two words) at double (p*2 + q)*ncell + i.
 
 typedef unsigned long long u64;
 
@@ -87,18 +86,21 @@ __device__ __forceinline__ int opaque(int v) {
   return v;
 }
 
-__device__ __forceinline__ void put_u32(unsigned *p, unsigned v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Tagged words: data below, the exchange's number above.
+__device__ __forceinline__ void put_word(u64 *p, unsigned tag, unsigned v) {
+  __hip_atomic_store(p, (u64)tag << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ unsigned get_u32(const unsigned *p) {
+__device__ __forceinline__ u64 get_word(const u64 *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void put_f64(unsigned *p, double v) {
+__device__ __forceinline__ bool has_tag(u64 w, unsigned tag) { return (unsigned)(w >> 32) == tag; }
+__device__ __forceinline__ void put_f64(u64 *p, unsigned tag, double v) {
   const u64 b = (u64)__double_as_longlong(v);
-  __hip_atomic_store((u64 *)p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  put_word(p, tag, (unsigned)b);
+  put_word(p + 1, tag, (unsigned)(b >> 32));
 }
-__device__ __forceinline__ u64 get_u64(const unsigned *p) {
-  return __hip_atomic_load((const u64 *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ double f64_of(u64 lo, u64 hi) {
+  return __longlong_as_double((long long)(hi << 32 | (lo & 0xffffffffull)));
 }
 
 // Grid barrier number `gen` (1, 2, ...) with counters, for the few places
@@ -134,22 +136,48 @@ __device__ bool grid_barrier(const Bar &b, unsigned gen) {
   return s_ok != 0;
 }
 
-// Partials: [parity][NVMAX][PB workgroups] doubles.
-__device__ __forceinline__ double *pslot(double *ps, unsigned tag, int j) {
-  return ps + ((size_t)(tag & 1u) * NVMAX + j) * PB;
-}
-
 struct Xch {
-  double *ps;          // partials
-  unsigned *hx;        // halo slots, [2][HX_WORDS][ncell] words
-  unsigned *flag;      // one word per workgroup, TICKET_PAD apart
+  u64 *ps;             // partials: [parity][workgroup][NVMAX][2 words]
+  u64 *hx;             // halo slots: [parity][cell], one word (FP32) or two (FP64) each
   int ncell;
 };
 
+__device__ __forceinline__ u64 *pslot(const Xch &x, unsigned tag, int wg) {
+  return x.ps + ((size_t)(tag & 1u) * PB + wg) * (2 * NVMAX);
+}
+__device__ __forceinline__ u64 *hslot32(const Xch &x, unsigned tag) {
+  return x.hx + (size_t)(tag & 1u) * x.ncell;
+}
+__device__ __forceinline__ u64 *hslot64(const Xch &x, unsigned tag) {
+  return x.hx + (size_t)(tag & 1u) * x.ncell * 2;
+}
+
+// Set by a wave whose wait was abandoned; the workgroup leaves after its
+// next barrier.  Cleared before the kernel's first barrier.
+__device__ __forceinline__ int &bad() {
+  __shared__ int s_bad;
+  return s_bad;
+}
+// One more polling round of a wave: true when it has to give up.
+__device__ __forceinline__ bool give_up(const Bar &b, unsigned &spins) {
+  ++spins;
+  const int ab = (spins & 255u) == 0u
+                     ? __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                           b.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                     : 0;
+  if (spins > b.spin_max || ab) {
+    __hip_atomic_store(b.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bad() = 1;
+    return true;
+  }
+  __builtin_amdgcn_s_sleep(1);
+  return false;
+}
+
 // Block sum of NV partials into this workgroup's slots of exchange `tag`
-// (stored by thread 0, not yet announced).
+// (lane j of wave 0 adds value j in the order of the waves).
 template <int NV>
-__device__ void post_partials(double (&v)[NV], const Xch &x, unsigned tag) {
+__device__ void post(double (&v)[NV], const Xch &x, unsigned tag) {
   __shared__ double sh[NV][PW];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
@@ -159,109 +187,124 @@ __device__ void post_partials(double (&v)[NV], const Xch &x, unsigned tag) {
     for (int j = 0; j < NV; ++j) sh[j][w] = v[j];
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    // all the loads first, so that they are in flight together; the sums
-    // keep the wave order
-    double pv[NV][PW];
+  if (threadIdx.x < NV) {
+    double pv[PW];
 #pragma unroll
-    for (int j = 0; j < NV; ++j)
+    for (int q = 0; q < PW; ++q) pv[q] = sh[threadIdx.x][q];
+    double s = 0.0;
 #pragma unroll
-      for (int q = 0; q < PW; ++q) pv[j][q] = sh[j][q];
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      double s = 0.0;
-#pragma unroll
-      for (int q = 0; q < PW; ++q) s += pv[j][q];
-      __hip_atomic_store(&pslot(x.ps, tag, j)[blockIdx.x], s, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    }
+    for (int q = 0; q < PW; ++q) s += pv[q];
+    put_f64(pslot(x, tag, (int)blockIdx.x) + 2 * threadIdx.x, tag, s);
   }
 }
 
-// The flag of exchange `tag`: every wave's earlier stores (partials, halo
-// values) have completed before thread 0 raises it.
-__device__ void post_flag(const Xch &x, unsigned tag) {
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (threadIdx.x == 0) put_u32(&x.flag[blockIdx.x * TICKET_PAD], tag);
-}
-
-template <int NV>
-__device__ void post(double (&v)[NV], const Xch &x, unsigned tag) {
-  post_partials<NV>(v, x, tag);
-  post_flag(x, tag);
-}
-
-// Wait for exchange `tag`, then fetch the NV partials of every workgroup
-// and NR words of each outside cell (hl[0..nhalo)) into raw[q*HMAX + h].
-// Wave 0 alone polls the flags (lane l reads the flags of workgroups l,
-// l+64, ...; a wave vote ends the loop), so the waiting costs no workgroup
-// barrier per round; after one barrier every wave fetches the halo words
-// while wave 0 adds the partials (lane l adds those of workgroups l, l+64,
-// ... in that order, then a DPP wave sum).  Returns the sums (same bits in
-// every workgroup), or false if the wait was abandoned.
-template <int NV, int NR>
-__device__ bool exchange(const Xch &x, unsigned tag, const int *hl, int nhalo,
-                         unsigned *raw, const Bar &b, double (&sum)[NV]) {
-  __shared__ double shs[NV];
-  __shared__ int s_ok;
-  const int t = threadIdx.x, lane = t & 63;
-  const int nb = (int)gridDim.x;
-  if (t < 64) {
-    unsigned spins = 0;
-    int ok = 1;
-    for (;;) {
-      // every lane loads (past the last workgroup, that one's flag again),
-      // so that the loads of a round are in flight together: loads under a
-      // condition would each wait for its own result
-      // (the lane number made opaque: the flag addresses are formed here,
-      // not held in registers across the caller's loops)
-      const int ln = opaque(lane);
-      unsigned f[PB / 64];
+// Outside cells' words of exchange `tag`, by the calling threads t = 0 ..
+// nt-1 (whole waves): cell(h) is entry h's cell, put(h, value) takes its
+// value.  Every lane loads (past the list's end, its last cell again) and the
+// loads of a batch are in flight together; a vote ends the wave's loop.
+// False if the wait was abandoned.
+template <int HB, typename CellF, typename PutF>
+__device__ __forceinline__ bool halo32(const Xch &x, unsigned tag, int nhalo, int t, int nt,
+                                       const Bar &b, CellF cell, PutF put) {
+  const u64 *base = hslot32(x, tag);
+  const int lane = t & 63;
+  for (int h0 = __builtin_amdgcn_readfirstlane(t - lane); h0 < nhalo; h0 += HB * nt) {
+    int c[HB];
+    u64 v[HB];
 #pragma unroll
-      for (int u = 0; u < PB / 64; ++u)
-        f[u] = get_u32(&x.flag[min(ln + 64 * u, nb - 1) * TICKET_PAD]);
+    for (int u = 0; u < HB; ++u) c[u] = cell(min(h0 + lane + u * nt, nhalo - 1));
+    unsigned spins = 0;
+    for (;;) {
       bool ready = true;
 #pragma unroll
-      for (int u = 0; u < PB / 64; ++u) ready = ready && (ln + 64 * u >= nb || f[u] >= tag);
+      for (int u = 0; u < HB; ++u) v[u] = get_word(base + (size_t)c[u]);
+#pragma unroll
+      for (int u = 0; u < HB; ++u) ready = ready && has_tag(v[u], tag);
       if (__all(ready)) break;
-      ++spins;
-      const int ab = (spins & 255u) == 0u
-                         ? __builtin_amdgcn_readfirstlane(
-                               __hip_atomic_load(b.abort, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT))
-                         : 0;
-      if (spins > b.spin_max || ab) {
-        if (lane == 0)
-          __hip_atomic_store(b.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ok = 0;
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
+      if (give_up(b, spins)) return false;
     }
-    if (lane == 0) s_ok = ok;
+#pragma unroll
+    for (int u = 0; u < HB; ++u)
+      if (h0 + lane + u * nt < nhalo) put(h0 + lane + u * nt, __uint_as_float((unsigned)v[u]));
   }
-  __syncthreads();
-  if (!s_ok) return false;
+  return true;
+}
+template <int HB, typename CellF, typename PutF>
+__device__ __forceinline__ bool halo64(const Xch &x, unsigned tag, int nhalo, int t, int nt,
+                                       const Bar &b, CellF cell, PutF put) {
+  const u64 *base = hslot64(x, tag);
+  const int lane = t & 63;
+  for (int h0 = __builtin_amdgcn_readfirstlane(t - lane); h0 < nhalo; h0 += HB * nt) {
+    int c[HB];
+    u64 lo[HB], hi[HB];
+#pragma unroll
+    for (int u = 0; u < HB; ++u) c[u] = cell(min(h0 + lane + u * nt, nhalo - 1));
+    unsigned spins = 0;
+    for (;;) {
+      bool ready = true;
+#pragma unroll
+      for (int u = 0; u < HB; ++u) {
+        lo[u] = get_word(base + 2 * (size_t)c[u]);
+        hi[u] = get_word(base + 2 * (size_t)c[u] + 1);
+      }
+#pragma unroll
+      for (int u = 0; u < HB; ++u) ready = ready && has_tag(lo[u], tag) && has_tag(hi[u], tag);
+      if (__all(ready)) break;
+      if (give_up(b, spins)) return false;
+    }
+#pragma unroll
+    for (int u = 0; u < HB; ++u)
+      if (h0 + lane + u * nt < nhalo) put(h0 + lane + u * nt, f64_of(lo[u], hi[u]));
+  }
+  return true;
+}
+
+// The sums of exchange `tag`: wave 0 polls the partials of every workgroup
+// (lane l those of workgroups l, l+64, ..., UG at a time) and adds them in
+// that order, then a DPP wave sum; the other waves meanwhile run halo(t, nt)
+// as threads t = 0 .. nt-1.  Returns the sums (same bits in every workgroup)
+// after one workgroup barrier, or false if a wait was abandoned.
+template <int NV, int UG, typename HaloF>
+__device__ __forceinline__ bool exchange(const Xch &x, unsigned tag, const Bar &b,
+                                         double (&sum)[NV], HaloF halo) {
+  __shared__ double shs[NV];
+  const int t = threadIdx.x, lane = t & 63;
+  const int nb = (int)gridDim.x;
   if (t < 64) {
     double v[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) v[j] = 0.0;
-    // four workgroups' partials per lane in flight at a time
-    for (int u0 = 0; 64 * u0 < nb; u0 += 4) {
-      double a[4][NV];
+    bool ok = true;
+    for (int u0 = 0; 64 * u0 < nb && ok; u0 += UG) {
+      u64 lo[UG][NV], hi[UG][NV];
+      unsigned spins = 0;
+      for (;;) {
+        // the lane number made opaque: the addresses are formed here, not
+        // held in registers across the caller's loops
+        const int ln = opaque(lane);
+        bool ready = true;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int q = min(opaque(lane) + 64 * (u0 + u), nb - 1);  // every lane loads
+        for (int u = 0; u < UG; ++u) {
+          const u64 *q = pslot(x, tag, min(ln + 64 * (u0 + u), nb - 1));  // every lane loads
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
-          a[u][j] = __hip_atomic_load(&pslot(x.ps, tag, j)[q], __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
+          for (int j = 0; j < NV; ++j) {
+            lo[u][j] = get_word(q + 2 * j);
+            hi[u][j] = get_word(q + 2 * j + 1);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < UG; ++u)
+#pragma unroll
+          for (int j = 0; j < NV; ++j)
+            ready = ready && has_tag(lo[u][j], tag) && has_tag(hi[u][j], tag);
+        if (__all(ready)) break;
+        if (give_up(b, spins)) { ok = false; break; }
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < UG; ++u)
 #pragma unroll
-        for (int j = 0; j < NV; ++j) v[j] += lane + 64 * (u0 + u) < nb ? a[u][j] : 0.0;
+        for (int j = 0; j < NV; ++j)
+          v[j] += lane + 64 * (u0 + u) < nb ? f64_of(lo[u][j], hi[u][j]) : 0.0;
     }
 #pragma unroll
     for (int j = 0; j < NV; ++j) v[j] = wave_sum_dpp(v[j]);
@@ -269,57 +312,19 @@ __device__ bool exchange(const Xch &x, unsigned tag, const int *hl, int nhalo,
 #pragma unroll
       for (int j = 0; j < NV; ++j) shs[j] = v[j];
     }
+  } else {
+    halo(t - 64, PB - 64);
   }
-  if (NR > 0) {
-    // all loads of a batch of HB outside cells are in flight before the
-    // first result is stored (a store per load would serialise the round
-    // trips)
-    constexpr int HB = 4;
-    const size_t par = tag & 1u, nce = (size_t)x.ncell;
-    const unsigned *w32 = x.hx + par * HX_WORDS * nce;        // FP32 planes
-    const unsigned *w64 = x.hx + par * 2 * 2 * nce;           // FP64 planes
-    for (int h0 = t; h0 < nhalo; h0 += HB * PB) {
-      u64 wv[HB][2];
-      unsigned wz[HB];
-#pragma unroll
-      for (int u = 0; u < HB; ++u) {
-        // every lane loads (past the list's end, its last cell again)
-        const size_t j = (size_t)hl[min(h0 + u * PB, nhalo - 1)];
-        wv[u][0] = wv[u][1] = 0;
-        wz[u] = 0;
-        if (NR == 4) {
-          wv[u][0] = get_u64(w64 + 2 * j);
-          wv[u][1] = get_u64(w64 + 2 * (nce + j));
-        } else {
-          wv[u][0] = get_u32(w32 + j);
-          if (NR >= 2) wv[u][1] = get_u32(w32 + nce + j);
-          if (NR >= 3) wz[u] = get_u32(w32 + 2 * nce + j);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < HB; ++u) {
-        const int h = h0 + u * PB;
-        if (h < nhalo) {
-          if (NR == 4) {
-            raw[h] = (unsigned)wv[u][0];
-            raw[HMAX + h] = (unsigned)(wv[u][0] >> 32);
-            raw[2 * HMAX + h] = (unsigned)wv[u][1];
-            raw[3 * HMAX + h] = (unsigned)(wv[u][1] >> 32);
-          } else {
-            raw[h] = (unsigned)wv[u][0];
-            if (NR >= 2) raw[HMAX + h] = (unsigned)wv[u][1];
-            if (NR >= 3) raw[2 * HMAX + h] = wz[u];
-          }
-        }
-      }
-    }
-  }
+  // shs is written again only after every wave has passed the next post()
   __syncthreads();
+  if (bad()) return false;
 #pragma unroll
   for (int j = 0; j < NV; ++j) sum[j] = shs[j];
-  __syncthreads();
   return true;
 }
+struct NoHalo {
+  __device__ void operator()(int, int) const {}
+};
 
 // neighbour slots of a row
 enum { NS = 0, NN = 1, NW = 2, NE = 3 };
@@ -376,7 +381,7 @@ struct P64Args {
   double *x;                 // P, in/out
   const int *lw, *le, *ls, *ln;
   int nwet, lc0, rowmajor, mutual;
-  Xch xc;                    // exchange slots; halo words: r (2), p (2)
+  Xch xc;
   unsigned tag0;
   Bar bar;
   CgState *st;
@@ -390,8 +395,10 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   // neighbour that is not a cell, so that every lane loads)
   __shared__ double lds[2 * WIN + CPT * PB + 1];
   __shared__ int hl[2 * WIN];
-  __shared__ unsigned raw[4 * HMAX];
+  __shared__ double zh[HMAX];  // z of the outside cells
   constexpr int ZS = 2 * WIN + CPT * PB;
+  // below the most cells per thread there are at most PCG64_NB workgroups
+  constexpr int UG = CPT < PCG64_CPT_MAX ? 2 : 4;
   const int b0 = 1 + (int)blockIdx.x * CPT * PB;
   const int b1 = min(b0 + CPT * PB, a.nwet + 1);
   const bool fast = a.rowmajor && (a.st->symok == 0);
@@ -403,17 +410,14 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   unsigned expo = 0u;        // bit k: another workgroup reads cell k
 
   auto inside = [&](int j) { return j >= b0 && j < b1; };
-  auto real = [&](int j) { return j > 0 && j != lc0; };
+  auto real = [&](int j) { return j > 0 && j < lc0; };
   auto slot = [&](int j) { return j - b0 + WIN; };
-  auto publish_rp = [&](int i, unsigned tag, double rv, double pv) {
-    const size_t nce = (size_t)a.xc.ncell, j = (size_t)opaque(i);
-    unsigned *q = a.xc.hx + (size_t)(tag & 1u) * 2 * 2 * nce;
-    put_f64(q + 2 * j, rv);
-    put_f64(q + 2 * (nce + j), pv);
+  auto publish_z = [&](int i, unsigned tag, double z) {
+    put_f64(hslot64(a.xc, tag) + 2 * (size_t)opaque(i), tag, z);
   };
 
   for (int g = threadIdx.x; g < 2 * WIN; g += PB) hl[g] = 0;
-  if (threadIdx.x == 0) lds[ZS] = 0.0;
+  if (threadIdx.x == 0) { lds[ZS] = 0.0; bad() = 0; }
   __syncthreads();
   double v2[2] = {0.0, 0.0};
 #pragma unroll
@@ -466,17 +470,23 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   __syncthreads();
   const int nhalo = compact_halo(hl, b0, b1);
 
+  // the window keeps p of the outside cells, formed here by their owner's
+  // operations from their published z = CCCI*r
+  for (int h = threadIdx.x; h < nhalo; h += PB) lds[slot(hl[h])] = 0.0;
+
   unsigned tag = a.tag0;
-  // exchange: z = CCCI*r and p (= 0) of the outside cells, RPCG and
-  // |FPTMP|^2 (the owner forms z, the product its neighbours would form, so
-  // they load no CCCI of an outside cell)
+  auto halo = [&](int t, int nt) {
+    halo64<2>(a.xc, tag, nhalo, t, nt, a.bar, [&](int h) { return hl[h]; },
+              [&](int h, double z) { zh[h] = z; });
+  };
+  // exchange: z of the outside cells (the owner forms it, so they load no
+  // CCCI of an outside cell), RPCG and |FPTMP|^2
 #pragma unroll
   for (int k = 0; k < CPT; ++k)
-    if (expo & (1u << k))
-      publish_rp(b0 + k * PB + (int)threadIdx.x, tag, cci[k] * r[k], 0.0);
+    if (expo & (1u << k)) publish_z(b0 + k * PB + (int)threadIdx.x, tag, cci[k] * r[k]);
   post<2>(v2, a.xc, tag);
   double s2[2];
-  if (!exchange<2, 4>(a.xc, tag, hl, nhalo, raw, a.bar, s2)) return;
+  if (!exchange<2, UG>(a.xc, tag, a.bar, s2, halo)) return;
   double rpcg = s2[0];
   const double bnorm2 = s2[1];
   const double rsqm = a.rel_tol > 0.0 ? a.rel_tol * a.rel_tol * bnorm2 : a.rsqm;
@@ -494,14 +504,10 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
       p[k] = cci[k] * r[k] + beta * p[k];
       lds[slot(b0 + k * PB + (int)threadIdx.x)] = p[k];
     }
-    // ... and on the outside cells, from their published z = CCCI*r and p
+    // ... and on the outside cells
     for (int h = threadIdx.x; h < nhalo; h += PB) {
-      const int j = hl[h];
-      const double zj = __longlong_as_double(
-          (long long)(((u64)raw[HMAX + h] << 32) | raw[h]));
-      const double pj = __longlong_as_double(
-          (long long)(((u64)raw[3 * HMAX + h] << 32) | raw[2 * HMAX + h]));
-      lds[slot(j)] = zj + beta * pj;
+      double &pj = lds[slot(hl[h])];
+      pj = zh[h] + beta * pj;
     }
     __syncthreads();
     double v1[1] = {0.0};
@@ -521,7 +527,7 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
     ++tag;
     post<1>(v1, a.xc, tag);
     double s1[1];
-    if (!exchange<1, 0>(a.xc, tag, hl, nhalo, raw, a.bar, s1)) return;
+    if (!exchange<1, UG>(a.xc, tag, a.bar, s1, NoHalo())) return;
     papcg = s1[0];
     alpha = rpcg / papcg;  // :124
     double v[2] = {0.0, 0.0};
@@ -535,10 +541,10 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
       const double z = cci[k] * rr;      // :134
       v[0] += rr * z;
       v[1] += rr * rr;
-      if (expo & (1u << k)) publish_rp(i, tag, z, p[k]);
+      if (expo & (1u << k)) publish_z(i, tag, z);
     }
     post<2>(v, a.xc, tag);
-    if (!exchange<2, 4>(a.xc, tag, hl, nhalo, raw, a.bar, s2)) return;
+    if (!exchange<2, UG>(a.xc, tag, a.bar, s2, halo)) return;
     beta = s2[0] / rpcg;  // :147-148
     rpcg = s2[0];
     rsq = s2[1];
@@ -577,7 +583,7 @@ struct PMxArgs {
   double *x;                 // P, in/out
   const int *ls, *ln;
   int nwet, lc0;
-  Xch xc;                    // exchange slots; halo words: r, w = A r, s = A p
+  Xch xc;
   unsigned tag0;
   Bar bar;
   CgState *st;
@@ -592,7 +598,7 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
   // a neighbour it does not couple to, so that every lane loads
   __shared__ float lds[2 * WIN + CPT * PB + 1];
   __shared__ int hl[2 * WIN];
-  __shared__ unsigned raw[3 * HMAX];
+  __shared__ float zh[HMAX], qh[HMAX];  // u or z, and q, of the outside cells
   constexpr int ZS = 2 * WIN + CPT * PB;
   // y (the inner solution) and z = M^-1 w of the own rows live in LDS:
   // with them in registers the 6..8-cells-per-thread shapes would spill
@@ -610,13 +616,11 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
   unsigned expo = 0u;
 
   auto inside = [&](int j) { return j >= b0 && j < b1; };
-  auto real = [&](int j) { return j > 0 && j != lc0; };
+  auto real = [&](int j) { return j > 0 && j < lc0; };
   auto slot = [&](int j) { return j - b0 + WIN; };
   auto rval = [&](int j) { return lds[real(j) ? slot(j) : ZS]; };
-  // FP32 halo value q of cell i in the slots of exchange `tag`
-  auto hxw = [&](int i, unsigned tag, int q) {
-    return a.xc.hx + ((size_t)(tag & 1u) * HX_WORDS + q) * (size_t)a.xc.ncell +
-           (size_t)opaque(i);
+  auto publish_w = [&](int i, unsigned tag, float v) {
+    put_word(hslot32(a.xc, tag) + (size_t)opaque(i), tag, __float_as_uint(v));
   };
 
   // M^-1 v: the first pdeg terms of the Neumann series of A' restricted to
@@ -656,7 +660,7 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
   };
 
   for (int g = threadIdx.x; g < 2 * WIN; g += PB) hl[g] = 0;
-  if (threadIdx.x == 0) lds[ZS] = 0.0f;
+  if (threadIdx.x == 0) { lds[ZS] = 0.0f; bad() = 0; }
   __syncthreads();
   double fp2 = 0.0;
 #pragma unroll
@@ -697,6 +701,10 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
   const int nhalo = compact_halo(hl, b0, b1);
 
   unsigned tag = a.tag0, gen = 0;
+  auto halo = [&](int t, int nt) {
+    halo32<4>(a.xc, tag, nhalo, t, nt, a.bar, [&](int h) { return hl[h]; },
+              [&](int h, float v) { zh[h] = v; });
+  };
   double rsqm = a.rsqm, bnorm2 = 0.0, rsq64 = 0.0, bn_in = 0.0;
   int total = 0, outer = 0, status = 0, inner = 0;
 
@@ -729,20 +737,19 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
       v3[1] += own ? (double)rs * (double)rs : 0.0;
     }
     // the partials go out while the preconditioner runs
-    post_partials<3>(v3, a.xc, tag);
+    post<3>(v3, a.xc, tag);
     // u0 = M^-1 r0, exported for the neighbours' A u0
     precond(r, u);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       const int i = b0 + k * PB + (int)threadIdx.x;
       lds[slot(i)] = u[k];
-      if (expo & (1u << k)) put_u32(hxw(i, tag, 0), __float_as_uint(u[k]));
+      if (expo & (1u << k)) publish_w(i, tag, u[k]);
     }
     fp2 = 0.0;
-    post_flag(a.xc, tag);
     {
       double s3[3];
-      if (!exchange<3, 1>(a.xc, tag, hl, nhalo, raw, a.bar, s3)) return;
+      if (!exchange<3, 4>(a.xc, tag, a.bar, s3, halo)) return;
       if (outer == 0) {
         bnorm2 = s3[2];
         rsqm = a.rel_tol > 0.0 ? a.rel_tol * a.rel_tol * bnorm2 : a.rsqm;
@@ -755,8 +762,13 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
     const double rt2 = fmax(a.rtol2, INNER_MARGIN2 * rsqm / rsq64);
 
     // ---- w0 = A' u0, z0 = M^-1 w0; gamma0 = (r,u), delta0 = (w,u),
-    // rho0 = (r,r); s_-1 = p_-1 = q_-1 = 0
-    for (int h = threadIdx.x; h < nhalo; h += PB) lds[slot(hl[h])] = __uint_as_float(raw[h]);
+    // rho0 = (r,r); s_-1 = p_-1 = q_-1 = 0.  From here on the window holds u
+    // of the outside cells and qh their q, formed by their owner's operations
+    // from their published z.
+    for (int h = threadIdx.x; h < nhalo; h += PB) {
+      lds[slot(hl[h])] = zh[h];
+      qh[h] = 0.0f;
+    }
     __syncthreads();
     ++tag;
     double v2[3] = {0.0, 0.0, 0.0};
@@ -774,7 +786,7 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
       v2[1] += (double)w[k] * (double)u[k];
       v2[2] += (double)r[k] * (double)r[k];
     }
-    post_partials<3>(v2, a.xc, tag);
+    post<3>(v2, a.xc, tag);
     {
       float zt[CPT];
       precond(w, zt);
@@ -782,18 +794,13 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
       for (int k = 0; k < CPT; ++k) {
         const int i = b0 + k * PB + (int)threadIdx.x;
         Z(k) = zt[k];
-        if (i < b1 && (expo & (1u << k))) {
-          put_u32(hxw(i, tag, 0), __float_as_uint(u[k]));
-          put_u32(hxw(i, tag, 1), __float_as_uint(zt[k]));
-          put_u32(hxw(i, tag, 2), __float_as_uint(0.0f));
-        }
+        if (expo & (1u << k)) publish_w(i, tag, zt[k]);
       }
     }
-    post_flag(a.xc, tag);
     double gam, del;
     {
       double s3[3];
-      if (!exchange<3, 3>(a.xc, tag, hl, nhalo, raw, a.bar, s3)) return;
+      if (!exchange<3, 4>(a.xc, tag, a.bar, s3, halo)) return;
       gam = s3[0];
       del = s3[1];
     }
@@ -824,13 +831,12 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
         u[k] = fmaf(-af, q[k], u[k]);
         lds[slot(i)] = u[k];
       }
-      // the outside cells' u, from their published u, z, q
+      // the outside cells' u
       for (int h = threadIdx.x; h < nhalo; h += PB) {
-        const float uj = __uint_as_float(raw[h]);
-        const float zj = __uint_as_float(raw[HMAX + h]);
-        const float qj0 = __uint_as_float(raw[2 * HMAX + h]);
-        const float qj = fmaf(bf, qj0, zj);
-        lds[slot(hl[h])] = fmaf(-af, qj, uj);
+        const float qj = fmaf(bf, qh[h], zh[h]);
+        qh[h] = qj;
+        float &uj = lds[slot(hl[h])];
+        uj = fmaf(-af, qj, uj);
       }
       __syncthreads();
       ++tag;
@@ -845,7 +851,7 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
         v[1] += (double)w[k] * (double)u[k];
         v[2] += (double)r[k] * (double)r[k];
       }
-      post_partials<3>(v, a.xc, tag);
+      post<3>(v, a.xc, tag);
       {
         float zt[CPT];
         precond(w, zt);
@@ -853,16 +859,11 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
         for (int k = 0; k < CPT; ++k) {
           const int i = b0 + k * PB + (int)threadIdx.x;
           Z(k) = zt[k];
-          if (i < b1 && (expo & (1u << k))) {
-            put_u32(hxw(i, tag, 0), __float_as_uint(u[k]));
-            put_u32(hxw(i, tag, 1), __float_as_uint(zt[k]));
-            put_u32(hxw(i, tag, 2), __float_as_uint(q[k]));
-          }
+          if (expo & (1u << k)) publish_w(i, tag, zt[k]);
         }
       }
-      post_flag(a.xc, tag);
       double s3[3];
-      if (!exchange<3, 3>(a.xc, tag, hl, nhalo, raw, a.bar, s3)) return;
+      if (!exchange<3, 4>(a.xc, tag, a.bar, s3, halo)) return;
       inner += 1;
       gam_prev = gam;
       alpha_prev = alpha;
@@ -901,109 +902,6 @@ __global__ __launch_bounds__(PB) void k_pcgmx(PMxArgs a) {
   }
 }
 
-// Wait until the workgroups lo..hi (the owners of this workgroup's outside
-// cells) have raised the flag of exchange `tag`.  Wave 0 polls (lane l:
-// workgroup lo+l); false if the wait was abandoned.
-__device__ bool halo_poll(const Xch &x, unsigned tag, int lo, int hi, const Bar &b) {
-  __shared__ int s_ok2;
-  const int t = threadIdx.x, lane = t & 63;
-  if (t < 64) {
-    unsigned spins = 0;
-    int ok = 1;
-    for (;;) {
-      bool ready = true;
-      for (int q = lo + lane; q <= hi; q += 64) ready = ready && get_u32(&x.flag[q * TICKET_PAD]) >= tag;
-      if (__all(ready)) break;
-      ++spins;
-      const int ab = (spins & 255u) == 0u
-                         ? __builtin_amdgcn_readfirstlane(
-                               __hip_atomic_load(b.abort, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT))
-                         : 0;
-      if (spins > b.spin_max || ab) {
-        if (lane == 0)
-          __hip_atomic_store(b.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ok = 0;
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-    if (lane == 0) s_ok2 = ok;
-  }
-  __syncthreads();
-  return s_ok2 != 0;
-}
-
-// The same, then one FP32 word of each outside cell into raw[h].
-__device__ bool halo_wait(const Xch &x, unsigned tag, int lo, int hi, const int *hl, int nhalo,
-                          unsigned *raw, const Bar &b) {
-  if (!halo_poll(x, tag, lo, hi, b)) return false;
-  const int t = threadIdx.x;
-  const unsigned *w32 = x.hx + (size_t)(tag & 1u) * HX_WORDS * (size_t)x.ncell;
-  constexpr int HB = 4;
-  for (int h0 = t; h0 < nhalo; h0 += HB * PB) {
-    unsigned v[HB];
-#pragma unroll
-    for (int u = 0; u < HB; ++u)  // every lane loads
-      v[u] = get_u32(w32 + (size_t)hl[min(h0 + u * PB, nhalo - 1)]);
-#pragma unroll
-    for (int u = 0; u < HB; ++u) {
-      const int h = h0 + u * PB;
-      if (h < nhalo) raw[h] = v[u];
-    }
-  }
-  __syncthreads();
-  return true;
-}
-
-// One FP32 word of each outside cell straight into the window: entry h of the
-// list is the window slot of that cell (b0 - WIN + slot is the cell).  The
-// owners' flags must already be up.
-__device__ void fetch_window32(const Xch &x, unsigned tag, const unsigned short *hs, int nhalo,
-                               int b0, float *win) {
-  const int t = threadIdx.x;
-  const unsigned *w32 = x.hx + (size_t)(tag & 1u) * HX_WORDS * (size_t)x.ncell;
-  constexpr int HB = 4;
-  for (int h0 = t; h0 < nhalo; h0 += HB * PB) {
-    unsigned v[HB];
-    int sl[HB];
-#pragma unroll
-    for (int u = 0; u < HB; ++u) {  // every lane loads
-      sl[u] = hs[min(h0 + u * PB, nhalo - 1)];
-      v[u] = get_u32(w32 + (size_t)(sl[u] + b0 - WIN));
-    }
-#pragma unroll
-    for (int u = 0; u < HB; ++u)
-      if (h0 + u * PB < nhalo) win[sl[u]] = __uint_as_float(v[u]);
-  }
-  __syncthreads();
-}
-
-// FP64 value 0 of each outside cell in the slots of exchange `tag` (posted
-// with put_f64 at word 2*i of that parity's first FP64 plane) into raw[h]
-// (low word) and raw[HMAX + h] (high word); the flags must already be up.
-__device__ void fetch_halo64(const Xch &x, unsigned tag, const int *hl, int nhalo,
-                             unsigned *raw) {
-  const int t = threadIdx.x;
-  const unsigned *w64 = x.hx + (size_t)(tag & 1u) * 2 * 2 * (size_t)x.ncell;
-  constexpr int HB = 4;
-  for (int h0 = t; h0 < nhalo; h0 += HB * PB) {
-    u64 v[HB];
-#pragma unroll
-    for (int u = 0; u < HB; ++u)  // every lane loads
-      v[u] = get_u64(w64 + 2 * (size_t)hl[min(h0 + u * PB, nhalo - 1)]);
-#pragma unroll
-    for (int u = 0; u < HB; ++u) {
-      const int h = h0 + u * PB;
-      if (h < nhalo) {
-        raw[h] = (unsigned)v[u];
-        raw[HMAX + h] = (unsigned)(v[u] >> 32);
-      }
-    }
-  }
-  __syncthreads();
-}
-
 // ---------------------------------------------------------------------
 // Mixed, pipelined: the same FP32 inner solve in the pipelined form of the
 // preconditioned Chronopoulos-Gear CG (Ghysels and Vanroose, 2014): each
@@ -1034,7 +932,6 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
   constexpr bool BIG = CPT > PCGMX_CPT_SMALL;
   static_assert(!BIG || 3 * CPT * PB >= 2 * WIN, "the list of outside cells is formed there");
   __shared__ int hl[BIG ? 1 : 2 * WIN];
-  __shared__ unsigned raw[BIG ? 1 : HMAX];
   __shared__ unsigned short hs[BIG ? 2 * WIN : 1];
   constexpr int ZS = 2 * WIN + CPT * PB;
   // y, q = M^-1 s and z = A' q of the own rows live in LDS
@@ -1058,21 +955,21 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
     if (BIG && k_ % 4 == 3) __builtin_amdgcn_sched_barrier(0);
   };
   auto inside = [&](int j) { return j >= b0 && j < b1; };
-  auto real = [&](int j) { return j > 0 && j != lc0; };
+  auto real = [&](int j) { return j > 0 && j < lc0; };
   auto slot = [&](int j) { return j - b0 + WIN; };
   // the cell of a window slot (ZS: none), and a slot where it is an own cell's
   auto cellof = [&](int sl) { return sl == ZS ? lc0 : sl - WIN + b0; };
   auto ownslot = [&](int sl) { return sl >= WIN && sl < b1 - b0 + WIN ? sl : ZS; };
-  auto hxw = [&](int i, unsigned tag) {
-    return a.xc.hx + (size_t)(tag & 1u) * HX_WORDS * (size_t)a.xc.ncell + (size_t)opaque(i);
+  auto publish_w = [&](int i, unsigned tag, float v) {
+    put_word(hslot32(a.xc, tag) + (size_t)opaque(i), tag, __float_as_uint(v));
   };
   // BIG: the outside-read rows' slots, one base per call and no address kept
   auto post_rows = [&](unsigned tag) {
-    unsigned *h = a.xc.hx + (size_t)(tag & 1u) * HX_WORDS * (size_t)a.xc.ncell +
-                  (size_t)opaque(b0 + (int)threadIdx.x);
+    u64 *h = hslot32(a.xc, tag) + (size_t)opaque(b0 + (int)threadIdx.x);
 #pragma unroll
     for (int k = 0; k < CPT; ++k)
-      if (expo & (1u << k)) put_u32(h + k * PB, __float_as_uint(lds[WIN + k * PB + (int)threadIdx.x]));
+      if (expo & (1u << k))
+        put_word(h + k * PB, tag, __float_as_uint(lds[WIN + k * PB + (int)threadIdx.x]));
   };
   // M^-1 v by the local Neumann polynomial, as in k_pcgmx.  No branch per
   // row: the lanes past b1 (the last workgroup's) hold zero coefficients
@@ -1158,7 +1055,7 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
 
   int *mark = BIG ? (int *)lyqz : hl;  // the list is formed where Y, Q, Z will be
   for (int g = threadIdx.x; g < 2 * WIN; g += PB) mark[g] = 0;
-  if (threadIdx.x == 0) lds[ZS] = 0.0f;
+  if (threadIdx.x == 0) { lds[ZS] = 0.0f; bad() = 0; }
   __syncthreads();
   double fp2 = 0.0;
   // every lane loads (a lane past b1 from the last own cell) and keeps the
@@ -1201,16 +1098,20 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
   }
   __syncthreads();
   const int nhalo = compact_halo(mark, b0, b1);
-  // the workgroups that own the outside cells (hl is sorted)
-  const int span = CPT * PB;
-  const int nlo = nhalo > 0 ? (mark[0] - 1) / span : 1;
-  const int nhi = nhalo > 0 ? (mark[nhalo - 1] - 1) / span : 0;
   if constexpr (BIG) {
     for (int h = threadIdx.x; h < nhalo; h += PB) hs[h] = (unsigned short)slot(mark[h]);
     __syncthreads();  // the list is read before Y takes its place
   }
 
   unsigned tag = a.tag0, gen = 0;
+  // the outside cells' words of exchange `tag` into the window, by every wave
+  // (a wave of the workgroup may still read own slots only)
+  auto halo = [&]() {
+    halo32<4>(a.xc, tag, nhalo, (int)threadIdx.x, PB, a.bar,
+              [&](int h) { return BIG ? (int)hs[h] + b0 - WIN : hl[h]; },
+              [&](int h, float v) { lds[BIG ? (int)hs[h] : slot(hl[h])] = v; });
+    __syncthreads();  // (an abandoned wait: the next exchange leaves)
+  };
   double rsqm = a.rsqm, bnorm2 = 0.0, rsq64 = 0.0, bn_in = 0.0;
   int total = 0, outer = 0, status = 0, inner = 0;
 
@@ -1252,7 +1153,7 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
       v3[1] += own ? (double)rs * (double)rs : 0.0;
       fence(k);
     }
-    post_partials<3>(v3, a.xc, tag);
+    post<3>(v3, a.xc, tag);
     if constexpr (BIG) {
       precond_lds(r);
 #pragma unroll
@@ -1264,14 +1165,14 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
       for (int k = 0; k < CPT; ++k) {
         const int i = b0 + k * PB + (int)threadIdx.x;
         lds[slot(i)] = u[k];
-        if (expo & (1u << k)) put_u32(hxw(i, tag), __float_as_uint(u[k]));
+        if (expo & (1u << k)) publish_w(i, tag, u[k]);
       }
     }
     fp2 = 0.0;
-    post_flag(a.xc, tag);
+    halo();
     {
       double s3[3];
-      if (!exchange<3, BIG ? 0 : 1>(a.xc, tag, hl, nhalo, raw, a.bar, s3)) return;
+      if (!exchange<3, BIG ? 2 : 4>(a.xc, tag, a.bar, s3, NoHalo())) return;
       if (outer == 0) {
         bnorm2 = s3[2];
         rsqm = a.rel_tol > 0.0 ? a.rel_tol * a.rel_tol * bnorm2 : a.rsqm;
@@ -1284,14 +1185,8 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
     const double rt2 = fmax(a.rtol2, INNER_MARGIN2 * rsqm / rsq64);
 
     // ---- w0 = A' u0; s, p, q, z start at 0
-    if constexpr (BIG) {
-      fetch_window32(a.xc, tag, hs, nhalo, b0, lds);
-      spmv_lds(w);
-    } else {
-      for (int h = threadIdx.x; h < nhalo; h += PB) lds[slot(hl[h])] = __uint_as_float(raw[h]);
-      __syncthreads();
-      spmv(u, w);
-    }
+    if constexpr (BIG) spmv_lds(w);
+    else spmv(u, w);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       s[k] = p[k] = 0.0f;
@@ -1311,8 +1206,8 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
         v[2] += (double)r[k] * (double)r[k];
         fence(k);
       }
-      post_partials<3>(v, a.xc, tag);
-      // ... then m = M^-1 w, its outside values, the flag
+      post<3>(v, a.xc, tag);
+      // ... then m = M^-1 w and its outside values
       float m[BIG ? 1 : CPT];
       if constexpr (BIG) {
         precond_lds(w);
@@ -1323,28 +1218,17 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
         for (int k = 0; k < CPT; ++k) {
           const int i = b0 + k * PB + (int)threadIdx.x;
           lds[slot(i)] = m[k];
-          if (expo & (1u << k)) put_u32(hxw(i, tag), __float_as_uint(m[k]));
+          if (expo & (1u << k)) publish_w(i, tag, m[k]);
         }
       }
-      post_flag(a.xc, tag);
       // n = A' m once the neighbouring workgroups' m has arrived
-      if constexpr (BIG) {
-        if (nhalo > 0) {
-          if (!halo_poll(a.xc, tag, nlo, nhi, a.bar)) return;
-          fetch_window32(a.xc, tag, hs, nhalo, b0, lds);
-        }
-        __syncthreads();
-      } else {
-        if (nhalo > 0 && !halo_wait(a.xc, tag, nlo, nhi, hl, nhalo, raw, a.bar)) return;
-        for (int h = threadIdx.x; h < nhalo; h += PB) lds[slot(hl[h])] = __uint_as_float(raw[h]);
-        __syncthreads();
-      }
+      halo();
       float n[CPT];
       if constexpr (BIG) spmv_lds(n);
       else spmv(m, n);
       // the sums of every workgroup
       double s3[3];
-      if (!exchange<3, 0>(a.xc, tag, hl, 0, raw, a.bar, s3)) return;
+      if (!exchange<3, BIG ? 2 : 4>(a.xc, tag, a.bar, s3, NoHalo())) return;
       const double gam = s3[0], del = s3[1];
       if (s3[2] <= rt2 * bn_in || inner >= a.iterm) break;
       double beta, alpha;
@@ -1414,8 +1298,8 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
 // FP64 Jacobi-PCG, pipelined (opt-in: efdc_set_cg64_pipeline).  The
 // reference's PCG (EFDC/congrad.f90:91-169) rewritten in the pipelined order
 // of Ghysels and Vanroose (2014), as k_pcgmx_pl does for the mixed inner
-// solve: an iteration posts its sums (r,u), (w,u), (r,r), the m = CCCI w
-// of its outside-read cells and its flag; it waits only for the workgroups
+// solve: an iteration posts its sums (r,u), (w,u), (r,r) and the m = CCCI w
+// of its outside-read cells; it waits only for the workgroups
 // that own its outside cells, forms n = A m, and only then waits for every
 // workgroup's sums to take alpha and beta.  The Jacobi preconditioner is
 // diagonal, so u = CCCI r, m = CCCI w and q = CCCI s are formed where they
@@ -1433,7 +1317,6 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
   // neighbour that is not a cell, so that every lane loads)
   __shared__ double lds[2 * WIN + CPT * PB + 1];
   __shared__ int hl[2 * WIN];
-  __shared__ unsigned raw[2 * HMAX];
   __shared__ double lzs[CPT * PB];
   constexpr int ZS = 2 * WIN + CPT * PB;
   const int b0 = 1 + (int)blockIdx.x * CPT * PB;
@@ -1448,11 +1331,10 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
   auto Z = [&](int k) -> double & { return lzs[k * PB + threadIdx.x]; };
 
   auto inside = [&](int j) { return j >= b0 && j < b1; };
-  auto real = [&](int j) { return j > 0 && j != lc0; };
+  auto real = [&](int j) { return j > 0 && j < lc0; };
   auto slot = [&](int j) { return j - b0 + WIN; };
-  auto w64 = [&](int i, unsigned tag) {
-    return a.xc.hx + (size_t)(tag & 1u) * 2 * 2 * (size_t)a.xc.ncell +
-           2 * (size_t)opaque(i);
+  auto publish_m = [&](int i, unsigned tag, double v) {
+    put_f64(hslot64(a.xc, tag) + 2 * (size_t)opaque(i), tag, v);
   };
   // y = A v on the own rows from the window (own slots and outside cells);
   // the lanes past b1 have ccc = 1, zero couplings and v = 0
@@ -1472,7 +1354,7 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
   };
 
   for (int g = threadIdx.x; g < 2 * WIN; g += PB) hl[g] = 0;
-  if (threadIdx.x == 0) lds[ZS] = 0.0;
+  if (threadIdx.x == 0) { lds[ZS] = 0.0; bad() = 0; }
   __syncthreads();
   double fp2 = 0.0;
 #pragma unroll
@@ -1522,33 +1404,33 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
   }
   __syncthreads();
   const int nhalo = compact_halo(hl, b0, b1);
-  const int span = CPT * PB;
-  const int nlo = nhalo > 0 ? (hl[0] - 1) / span : 1;
-  const int nhi = nhalo > 0 ? (hl[nhalo - 1] - 1) / span : 0;
 
   // set-up exchange: u = CCCI r of the outside-read cells and |FPTMP|^2;
   // then w = A u (the owners publish u, so no CCCI of an outside cell is
   // loaded)
   unsigned tag = a.tag0;
+  // the outside cells' values of exchange `tag` into the window, by every wave
+  auto halo = [&]() {
+    halo64<2>(a.xc, tag, nhalo, (int)threadIdx.x, PB, a.bar, [&](int h) { return hl[h]; },
+              [&](int h, double v) { lds[slot(hl[h])] = v; });
+    __syncthreads();  // (an abandoned wait: the next exchange leaves)
+  };
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
     const int i = b0 + k * PB + (int)threadIdx.x;
     const double uk = cci[k] * r[k];
     lds[slot(i)] = uk;
-    if (expo & (1u << k)) put_f64(w64(i, tag), uk);
+    if (expo & (1u << k)) publish_m(i, tag, uk);
   }
   {
     double v1[1] = {fp2};
     post<1>(v1, a.xc, tag);
   }
   double s1[1];
-  if (!exchange<1, 0>(a.xc, tag, hl, 0, raw, a.bar, s1)) return;
+  halo();
+  if (!exchange<1, 4>(a.xc, tag, a.bar, s1, NoHalo())) return;
   const double bnorm2 = s1[0];
   const double rsqm = a.rel_tol > 0.0 ? a.rel_tol * a.rel_tol * bnorm2 : a.rsqm;
-  fetch_halo64(a.xc, tag, hl, nhalo, raw);
-  for (int h = threadIdx.x; h < nhalo; h += PB)
-    lds[slot(hl[h])] = __longlong_as_double((long long)(((u64)raw[HMAX + h] << 32) | raw[h]));
-  __syncthreads();
   {
     double u0[CPT];
 #pragma unroll
@@ -1569,34 +1451,25 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
       v[1] += w[k] * uk;
       v[2] += r[k] * r[k];
     }
-    post_partials<3>(v, a.xc, tag);
-    // ... then m = CCCI w on the window (after every read of the last SpMV),
-    // m of the outside-read cells, the flag
-    __syncthreads();
+    post<3>(v, a.xc, tag);
+    // ... then m = CCCI w on the window (every wave is past its reads of the
+    // last SpMV: post's barrier) and m of the outside-read cells
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       const int i = b0 + k * PB + (int)threadIdx.x;
       const double mk = cci[k] * w[k];
       lds[slot(i)] = mk;
-      if (expo & (1u << k)) put_f64(w64(i, tag), mk);
+      if (expo & (1u << k)) publish_m(i, tag, mk);
     }
-    post_flag(a.xc, tag);
     // n = A m once the neighbouring workgroups' m has arrived
-    if (nhalo > 0) {
-      if (!halo_poll(a.xc, tag, nlo, nhi, a.bar)) return;
-      fetch_halo64(a.xc, tag, hl, nhalo, raw);
-      for (int h = threadIdx.x; h < nhalo; h += PB)
-        lds[slot(hl[h])] =
-            __longlong_as_double((long long)(((u64)raw[HMAX + h] << 32) | raw[h]));
-    }
-    __syncthreads();
+    halo();
     double m[CPT], n[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) m[k] = cci[k] * w[k];
     spmv(m, n);
     // the sums of every workgroup
     double s3[3];
-    if (!exchange<3, 0>(a.xc, tag, hl, 0, raw, a.bar, s3)) return;
+    if (!exchange<3, 4>(a.xc, tag, a.bar, s3, NoHalo())) return;
     gam = s3[0];
     const double del = s3[1];
     rsq = s3[2];
@@ -1660,6 +1533,12 @@ __global__ __launch_bounds__(256) void k_mx_coef(const double *ccc, const double
   aw[i] = (float)(ccw[i] * di * dw);
 }
 
+// Slots that carry no exchange's number.
+__global__ __launch_bounds__(256) void k_pcg_clear(u64 *ps, long nps, u64 *hx, long nhx) {
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < nps + nhx; i += gridDim.x * 256L)
+    (i < nps ? ps[i] : hx[i - nps]) = 0;
+}
+
 __global__ void k_pcg_reset(unsigned *ctr, int *abort) {
   const int t = threadIdx.x;
   if (t < PCG_NCTR) ctr[t] = 0u;
@@ -1677,7 +1556,6 @@ int occupancy(K kern) {
 }  // namespace
 
 // Largest cells-per-thread instantiation of each solve.
-constexpr int PCG64_CPT_MAX = 6;
 // Terms of the workgroup-local preconditioner of the mixed persistent solve
 // when the caller leaves the choice to the library.
 constexpr int PCG_PDEG_DEFAULT = 3;
@@ -1715,11 +1593,9 @@ int pcg_prepare(efdc_ctx *c) {
     c->pcg_occmx[k] = k <= PCGMX_CPT_SMALL ? std::min(occmx[k], occpl[k]) : occpl[k];
   c->pcg_ncell = c->n_wet() + 2;
   int s;
-  if ((s = dev_alloc(c, &c->pcg_hx,
-                     sizeof(unsigned) * 2 * (size_t)c->pcg_ncell * HX_WORDS)))
-    return s;
-  if ((s = dev_alloc(c, &c->pcg_ps, sizeof(double) * 2 * NVMAX * PB))) return s;
-  if ((s = dev_alloc(c, (void **)&c->pcg_flag, sizeof(unsigned) * PB * TICKET_PAD))) return s;
+  // two parities of two words a cell, and of NVMAX doubles a workgroup
+  if ((s = dev_alloc(c, &c->pcg_hx, sizeof(u64) * 4 * (size_t)c->pcg_ncell))) return s;
+  if ((s = dev_alloc(c, &c->pcg_ps, sizeof(u64) * 2 * PB * 2 * NVMAX))) return s;
   if ((s = dev_alloc(c, (void **)&c->pcg_ctr, sizeof(unsigned) * PCG_NCTR))) return s;
   c->pcg_abort = &c->st->pabort;
   c->pcg_launch = 0;
@@ -1728,19 +1604,32 @@ int pcg_prepare(efdc_ctx *c) {
 }
 
 // Cells per thread and workgroup count of a persistent solve, or 0 when
-// the problem does not fit in one co-resident grid.
-static int pcg_shape(const efdc_ctx *c, const int *occ, int cpt_max, int &nb) {
+// the problem does not fit in one co-resident grid: the fewest cells per
+// thread that need at most nb_want workgroups, else the most that fit.
+static int pcg_shape(const efdc_ctx *c, const int *occ, int cpt_max, int &nb,
+                     int nb_want = PB) {
   const int n = c->n_wet();
+  int best = 0;
   for (int cpt = 1; cpt <= cpt_max; ++cpt) {
     const int need = (n + cpt * PB - 1) / (cpt * PB);
     const int cap = occ[cpt] * c->pcg_ncu;
     if (occ[cpt] > 0 && need <= cap && need <= PB) {
+      best = cpt;
       nb = need;
-      return cpt;
+      if (need <= nb_want) break;
     }
   }
-  return 0;
+  return best;
 }
+
+// FP64: every workgroup reads the partials of all of them, twice an
+// iteration, which beyond about 64 costs more than a further row per thread
+// (us a solve of 29 iterations, workgroups : cells per thread; 79 k cells 155 :
+// 1 160, 78 : 2 150, 52 : 3 137, 26 : 6 153; 276 k cells 180 : 3 213, 135 : 4
+// 197, 90 : 6 181; 22 k cells 43 : 1 126, 22 : 2 131).  The mixed solve, one
+// exchange per iteration with the preconditioner behind it, gains nothing
+// (169 k cells 166 : 2 109, 111 : 3 114, 83 : 4 117).
+constexpr int PCG64_NB = 64;
 
 // The form of the mixed persistent solve, and its shape: more than 8 cells
 // per thread (1.05 to 2.1 million cells on 256 CUs) in the pipelined form
@@ -1765,7 +1654,7 @@ bool pcg_applicable(efdc_ctx *c, bool mixed) {
   if (pcg_prepare(c) != EFDC_OK || c->pcg_ncu == 0) return false;
   int nb = 0;
   return mixed ? pcg_shape_mx(c, nb) > 0
-               : pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb) > 0;
+               : pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb, PCG64_NB) > 0;
 }
 
 // The persistent grid is sized to be co-resident (the occupancy table times
@@ -1790,14 +1679,16 @@ static int coop_launch(efdc_ctx *c, const void *fn, int nb, Args &args) {
 }
 
 // First exchange number of the next launch.  Launches are numbered
-// 1 .. 4095, so within a cycle exchange numbers only grow and the flags never
-// go backwards; when the numbering starts a new cycle the flags are cleared.
+// 1 .. 4095, so within a cycle a slot never holds a number that is still to
+// come; when the numbering starts a new cycle the slots are cleared.
 static int next_tag0(efdc_ctx *c, unsigned &tag0) {
   const bool wrap = c->pcg_launch == PCG_LAUNCH_CYCLE;
   c->pcg_launch = c->pcg_launch % PCG_LAUNCH_CYCLE + 1u;
-  if (wrap)
-    HIP_TRY(c, hipMemsetAsync(c->pcg_flag, 0, sizeof(unsigned) * PB * TICKET_PAD,
-                              c->stream));
+  if (wrap) {
+    k_pcg_clear<<<512, 256, 0, c->stream>>>((u64 *)c->pcg_ps, 2 * PB * 2 * NVMAX,
+                                            (u64 *)c->pcg_hx, 4 * (long)c->pcg_ncell);
+    HIP_TRY(c, hipGetLastError());
+  }
   tag0 = c->pcg_launch << PCG_TAG_BITS;
   return EFDC_OK;
 }
@@ -1817,7 +1708,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
   Bar bar{c->pcg_ctr, c->pcg_abort,
           plain && c->pcg_spin_test > 0 ? c->pcg_spin_test : SPIN_MAX};
   if (!mixed) {
-    const int cpt = pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb);
+    const int cpt = pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb, PCG64_NB);
     if (!cpt) { c->err = "persistent CG: problem too large"; return EFDC_ERR_ARG; }
     P64Args a;
     a.ccc = c->dH[EFDC_CCC];
@@ -1836,7 +1727,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
     a.lc0 = c->LC - 1;
     a.rowmajor = c->rowmajor ? 1 : 0;
     a.mutual = c->mutual ? 1 : 0;
-    a.xc = Xch{(double *)c->pcg_ps, (unsigned *)c->pcg_hx, c->pcg_flag, c->pcg_ncell};
+    a.xc = Xch{(u64 *)c->pcg_ps, (u64 *)c->pcg_hx, c->pcg_ncell};
     if ((s = next_tag0(c, a.tag0))) return s;
     a.bar = bar;
     a.st = c->st;
@@ -1888,7 +1779,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
     a.ln = c->dLN;
     a.nwet = c->n_wet();
     a.lc0 = c->LC - 1;
-    a.xc = Xch{(double *)c->pcg_ps, (unsigned *)c->pcg_hx, c->pcg_flag, c->pcg_ncell};
+    a.xc = Xch{(u64 *)c->pcg_ps, (u64 *)c->pcg_hx, c->pcg_ncell};
     if ((s = next_tag0(c, a.tag0))) return s;
     a.bar = bar;
     a.st = c->st;

@@ -339,7 +339,7 @@ int efdc_ctx_destroy(efdc_ctx_t *c) {
   dfree(c->part); dfree(c->st); dfree(c->tickets);
   { char *q = (char *)c->pcg_hx; dfree(q); }
   { char *q = (char *)c->pcg_ps; dfree(q); }
-  dfree(c->pcg_ctr); dfree(c->pcg_flag);
+  dfree(c->pcg_ctr);
   seg_free(c);
   adj_free(c);
   uvw_free(c);

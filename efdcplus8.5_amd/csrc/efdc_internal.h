@@ -154,9 +154,8 @@ struct efdc_ctx {
   bool pcg_ready = false;
   int pcg_ncu = 0;             // CUs, 0 when cooperative launch is unsupported
   int pcg_occ64[7] = {}, pcg_occmx[17] = {};  // workgroups per CU by CPT
-  void *pcg_hx = nullptr;      // halo slots [2][ncell][4] words
+  void *pcg_hx = nullptr;      // halo slots [2][ncell][2] tagged words
   void *pcg_ps = nullptr;      // partial slots
-  unsigned *pcg_flag = nullptr;  // exchange flag per workgroup
   int pcg_ncell = 0;
   unsigned pcg_launch = 0;     // launch number, gives the first tag
   unsigned *pcg_ctr = nullptr; // barrier counters

@@ -374,3 +374,26 @@ def test_mixed_persistent_many_cells_per_thread(nx, ny):
     assert eta_err(a.get("P")[i], b.get("P")[i]) <= 1e-7
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_persistent_launch_numbers_start_over(oracle_mod, mixed):
+    """The launches of the persistent solve are numbered 1 to 4095 and then
+    from 1 again: the solves around that give the first one's bits."""
+    from efdc_amd import lib
+    case, system, _ = _lake_system(oracle_mod, 40, 3)
+    kw = dict(cg_kernel=lib.CG_KERNEL_PERSISTENT, ITERM=4000, RSQM=TIGHT)
+    if mixed:
+        kw.update(cg_mode=lib.CG_MIXED, RSQM=1e-20)
+    ctx = lib.Context(case.grid, **kw)
+    for k, v in system.items():
+        ctx.set(k, v)
+    first = ctx.congrad()
+    p = ctx.get("P")
+    for _ in range(4092):  # launches 2 .. 4093, from the solution
+        ctx.congrad()
+    for _ in range(4):     # 4094, 4095, 1, 2
+        ctx.set("P", system["P"])
+        assert ctx.congrad()["iters"] == first["iters"]
+        np.testing.assert_array_equal(ctx.get("P"), p)
+    ctx.close()
