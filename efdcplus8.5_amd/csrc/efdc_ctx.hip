@@ -378,6 +378,7 @@ int efdc_ctx_destroy(efdc_ctx_t *c) {
   }
   { char *t = (char *)c->tran_tmp; dfree(t); }
   for (auto &p : c->adac) { char *q = (char *)p; dfree(q); p = nullptr; }
+  { char *q = (char *)c->adac_more; dfree(q); }
   dfree(c->cdzkk_k); dfree(c->cdzkmk_k); dfree(c->scal); dfree(c->nman);
   dfree(c->bccell);
   for (auto &r : c->trec) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }

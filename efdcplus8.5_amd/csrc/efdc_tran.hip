@@ -896,9 +896,10 @@ __device__ __forceinline__ void tran_lay_layers(const TranArgs<T> &a, double *lc
 
 // EEB, CCLB and VCU of a column (KC > 1), as in tran_col_body; the AB values
 // are loaded eight layers at a time
-template <typename T>
-__device__ __forceinline__ void tran_lay_factors(const TranArgs<T> &a, int i, double *eebs,
+template <typename Args>
+__device__ __forceinline__ void tran_lay_factors(const Args &a, int i, double *eebs,
                                                  double *ccls, double *vcus) {
+  using T = std::remove_const_t<std::remove_pointer_t<decltype(a.ab)>>;
   const int KC = a.KC;
   const size_t pitch = (size_t)a.pitch;
   const double DELTD2 = a.dt, hpi = a.hpi[i];
@@ -1231,7 +1232,7 @@ __global__ void k_closure_post(const double *__restrict__ uhdye, const double *_
 //                 sources (:583-599) and open boundaries (:602-620)
 //   k_fct_beta  : CMAX/CMIN (:627-679), DUU/DVV and the beta limiters
 //                 (:705-734)
-// and k_col_finish applies the (limited) fluxes per column (:737-786),
+// and k_adac_finish applies the (limited) fluxes per column (:737-786),
 // then the vertical diffusion and decay of CALCONC.
 // Ghost cells (L=1, LC) are zero in every field, as the never-written
 // entries of the reference's zero-initialised arrays are.
@@ -1255,13 +1256,49 @@ struct AdacArgs {
   const int *lmask;
 };
 
+// Constituents that go through the passes together, one per blockIdx.z (the
+// finish: blockIdx.y), each with scratch planes of its own: 8 n_scratch planes
+// of `plane` values, constituent 0's in AdacArgs.  n = 0: AdacArgs as it is.
+constexpr int ADAC_GROUP = 8;
+template <typename T>
+struct AdacGroup {
+  int n;
+  T *more;
+  int64_t plane;
+  T *con[ADAC_GROUP];
+  const T *con1[ADAC_GROUP];
+  int isadac[ADAC_GROUP], isfct[ADAC_GROUP], dye_mode[ADAC_GROUP];
+  double dye_f[ADAC_GROUP];
+};
+
+template <typename T>
+__device__ __forceinline__ void adac_take(AdacArgs<T> &a, const AdacGroup<T> &g, int q) {
+  if (g.n == 0) return;
+  a.con = g.con[q];
+  a.con1 = g.con1[q];
+  a.isadac = g.isadac[q];
+  a.isfct = g.isfct[q];
+  if (q == 0) return;
+  T *m = g.more + (int64_t)(q - 1) * 8 * g.plane;
+  a.uuuu = m;
+  a.vvvv = m + g.plane;
+  a.wwww = m + 2 * g.plane;
+  a.fu = m + 3 * g.plane;
+  a.fv = m + 4 * g.plane;
+  a.fw = m + 5 * g.plane;
+  a.duu = m + 6 * g.plane;
+  a.dvv = m + 7 * g.plane;
+}
+
 template <typename T>
 __device__ __forceinline__ double posv(const AdacArgs<T> &a, int j, int64_t o) {
   return (j == 0 || j == a.lc0) ? 0.0 : dmx((double)a.con[j + o], 0.);
 }
 
 template <typename T>
-__global__ __launch_bounds__(EFDC_BLOCK) void k_adac_grad(AdacArgs<T> a) {
+__global__ __launch_bounds__(EFDC_BLOCK) void k_adac_grad(AdacArgs<T> a, AdacGroup<T> g) {
+  adac_take(a, g, blockIdx.z);
+  if (a.isadac <= 0) return;
   const int i = 1 + xcd_tile(blockIdx.x, gridDim.x) * EFDC_BLOCK + threadIdx.x;
   if (i > a.nwet) return;
   const int k = blockIdx.y;
@@ -1291,7 +1328,9 @@ __device__ __forceinline__ bool src_at(const AdacArgs<T> &a, int j, int64_t o) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(EFDC_BLOCK) void k_adac_flux(AdacArgs<T> a) {
+__global__ __launch_bounds__(EFDC_BLOCK) void k_adac_flux(AdacArgs<T> a, AdacGroup<T> g) {
+  adac_take(a, g, blockIdx.z);
+  if (a.isadac <= 0) return;
   const int i = 1 + xcd_tile(blockIdx.x, gridDim.x) * EFDC_BLOCK + threadIdx.x;
   if (i > a.nwet) return;
   const int k = blockIdx.y, K = k + 1;
@@ -1370,7 +1409,9 @@ __device__ __forceinline__ void cont_mx_mn(const AdacArgs<T> &a, int j, int64_t 
 }
 
 template <typename T>
-__global__ __launch_bounds__(EFDC_BLOCK) void k_fct_beta(AdacArgs<T> a) {
+__global__ __launch_bounds__(EFDC_BLOCK) void k_fct_beta(AdacArgs<T> a, AdacGroup<T> g) {
+  adac_take(a, g, blockIdx.z);
+  if (a.isadac <= 0 || a.isfct == 0) return;
   const int i = 1 + xcd_tile(blockIdx.x, gridDim.x) * EFDC_BLOCK + threadIdx.x;
   if (i > a.nwet) return;
   const int k = blockIdx.y, K = k + 1, KC = a.KC;
@@ -1471,86 +1512,87 @@ __device__ __forceinline__ double lim_w(const AdacArgs<T> &a, int i, int K) {
 template <typename T>
 struct FinishArgs {
   AdacArgs<T> ad;
-  T *con;          // in: CON after the open boundaries; out: final CON
   const T *ab, *cdzkk, *cdzkmk;
   const double *cdzkk_k, *cdzkmk_k;
-  int dz_uniform;
+  const double *hpi;
+  int64_t pitch;
+  double dt;
+  int KC, dz_uniform;
   const unsigned char *pbcflag;
-  int adac;        // apply the antidiffusive correction
-  int dye_mode;
-  double dye_f;
 };
 
+// The limited fluxes, the vertical diffusion and the decay of 64 columns of
+// one constituent, laid out as k_tran_lay: the first nlw waves form CON of the
+// layers (wave w the layers w, w + nlw, ..) in LDS, the last wave the factors
+// of the vertical system, then one wave runs the two sweeps from LDS.
+// Bound by the gathered loads of the limiters (22 values a cell), which are
+// unconditional so that a layer's are in flight together; a thread per column
+// made them layer after layer, 38.5 us a
+// constituent of 253x187x9 in FP64, this one 25.2 for three.
 template <typename T>
-__global__ __launch_bounds__(TBLOCK) void k_col_finish(FinishArgs<T> f) {
-  extern __shared__ unsigned char smem[];
-  const AdacArgs<T> &a = f.ad;
-  const int TB = blockDim.x;
-  const int i = 1 + xcd_tile(blockIdx.x, gridDim.x) * TB + (int)threadIdx.x;
-  if (i > a.nwet) return;
-  if (a.lmask && a.lmask[i] == 0) return;  // CON = CON1 from the column kernel
-  const int tid = threadIdx.x, KC = a.KC;
-  const int64_t p = a.pitch;
-  double *vcu = (double *)smem;
-  T *ys = (T *)(vcu + (size_t)KC * TB);
-  const double DDELT = a.dt, DELTD2 = a.dt;
-  const double dxyip = a.dxyip[i], hpi = a.hpi[i];
-  const int LE = a.le[i], LN = a.ln[i], LW = a.lw[i], LS = a.ls[i];
-  const bool eg = (LE == a.lc0), ng = (LN == a.lc0);
-  double vcu_prev = 0.0, yprev = 0.0;
-  for (int k = 0; k < KC; ++k) {
-    const int K = k + 1;
-    const int64_t o = (int64_t)k * p;
-    double con = (double)f.con[i + o];
-    if (f.adac && !(f.pbcflag[i])) {
-      // EFDC/caltran.f90:771-778 (LOBCS cells keep CON, :781-786)
-      const double fui = lim_h(a, a.fu, i, LW, o);
-      const double fue = eg ? 0.0 : lim_h(a, a.fu, LE, a.lw[LE], o);
-      const double fvi = lim_h(a, a.fv, i, LS, o);
-      const double fvn = ng ? 0.0 : lim_h(a, a.fv, LN, a.ls[LN], o);
-      const double cd = con * (double)a.hpk[i + o] +
-                        DDELT * ((fui - fue + fvi - fvn) * dxyip + (lim_w(a, i, K - 1) - lim_w(a, i, K)));
-      con = cd * (double)a.hpki[i + o];
-    }
-    // vertical diffusion, forward sweep (EFDC/calconc.f90:264-422)
-    double y = con;
-    if (KC > 1) {
-      const double ckk = f.dz_uniform ? f.cdzkk_k[k] : (double)f.cdzkk[i + o];
-      const double ckm = f.dz_uniform ? f.cdzkmk_k[k] : (double)f.cdzkmk[i + o];
-      double vcu_k = 0.0;
-      if (K == 1) {
-        const double CCUBTMP = (-DELTD2 * ckk) * hpi * (double)f.ab[i + o];
-        const double eeb = 1.0 / (1.0 - CCUBTMP);
-        vcu_k = CCUBTMP * eeb;
-        y = con * eeb;
-      } else if (K < KC) {
-        const double cclb = (-DELTD2 * ckm) * hpi * (double)f.ab[i + o - p];
-        const double CCUBTMP = (-DELTD2 * ckk) * hpi * (double)f.ab[i + o];
-        const double CCMBTMP = 1.0 - cclb - CCUBTMP;
-        const double eeb = 1.0 / (CCMBTMP - cclb * vcu_prev);
-        vcu_k = CCUBTMP * eeb;
-        y = (con - cclb * yprev) * eeb;
-      } else {
-        const double cclb = (-DELTD2 * ckm) * hpi * (double)f.ab[i + o - p];
-        const double eeb = 1.0 / ((1.0 - cclb) - cclb * vcu_prev);
-        y = (con - cclb * yprev) * eeb;
+__global__ __launch_bounds__(320) void k_adac_finish(FinishArgs<T> f, AdacGroup<T> g, int nlw) {
+  extern __shared__ double lds[];
+  AdacArgs<T> a = f.ad;
+  adac_take(a, g, blockIdx.y);
+  const int lane = threadIdx.x, KC = f.KC;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+  const int i = xcd_tile(blockIdx.x, gridDim.x) * 64 + lane;
+  double *eebs = lds + lane, *ccls = eebs + (size_t)KC * 64, *vcus = ccls + (size_t)KC * 64,
+         *lcs = vcus + (size_t)KC * 64;
+  // a column left out of the transport: CON = CON1 from the column kernel
+  const bool act = i >= 1 && i <= a.nwet && !(a.lmask && a.lmask[i] == 0);
+  if (act && wv < nlw) {
+    const int64_t p = f.pitch;
+    const double DDELT = f.dt, dxyip = a.dxyip[i];
+    const int LE = a.le[i], LN = a.ln[i], LW = a.lw[i], LS = a.ls[i];
+    const bool eg = LE == a.lc0, ng = LN == a.lc0;
+    const bool keep = f.pbcflag[i] != 0, lob = (a.lobflag[i] & 3) != 0;
+    const bool fct = a.isfct != 0;
+    for (int k = wv; k < KC; k += nlw) {
+      const int64_t o = (int64_t)k * p;
+      double con = (double)a.con[i + o];
+      if (a.isadac > 0) {
+        // EFDC/caltran.f90:771-778 (LOBCS cells keep CON, :781-786)
+        double fui = (double)a.fu[i + o], fue = (double)a.fu[LE + o];
+        double fvi = (double)a.fv[i + o], fvn = (double)a.fv[LN + o];
+        double fwb = (double)a.fw[i + o], fwt = (double)a.fw[i + o + p];
+        const double hpk = (double)a.hpk[i + o], hpki = (double)a.hpki[i + o];
+        if (fct) {
+          // :737-766; the W/S neighbour of the cell east/north is the cell
+          // itself (the maps are mutual)
+          const int64_t ob = k > 0 ? o - p : o, ot = k + 1 < KC ? o + p : o;
+          const double uc = (double)a.duu[i + o], vc = (double)a.dvv[i + o];
+          const double uw = (double)a.duu[LW + o], vw = (double)a.dvv[LW + o];
+          const double ue = (double)a.duu[LE + o], ve = (double)a.dvv[LE + o];
+          const double us = (double)a.duu[LS + o], vs = (double)a.dvv[LS + o];
+          const double un = (double)a.duu[LN + o], vn = (double)a.dvv[LN + o];
+          const double ub = (double)a.duu[i + ob], vb = (double)a.dvv[i + ob];
+          const double ut = (double)a.duu[i + ot], vt = (double)a.dvv[i + ot];
+          fui = dmn(vw, uc) * dmx(fui, 0.) + dmn(uw, vc) * dmn(fui, 0.);
+          fue = dmn(vc, ue) * dmx(fue, 0.) + dmn(uc, ve) * dmn(fue, 0.);
+          fvi = dmn(vs, uc) * dmx(fvi, 0.) + dmn(us, vc) * dmn(fvi, 0.);
+          fvn = dmn(vc, un) * dmx(fvn, 0.) + dmn(uc, vn) * dmn(fvn, 0.);
+          fwb = lob ? 0.0 : dmn(vb, uc) * dmx(fwb, 0.) + dmn(ub, vc) * dmn(fwb, 0.);
+          fwt = lob ? 0.0 : dmn(vc, ut) * dmx(fwt, 0.) + dmn(uc, vt) * dmn(fwt, 0.);
+        }
+        fue = eg ? 0.0 : fue;
+        fvn = ng ? 0.0 : fvn;
+        fwb = k > 0 ? fwb : 0.0;
+        fwt = k + 1 < KC ? fwt : 0.0;
+        const double cd = con * hpk +
+                          DDELT * ((fui - fue + fvi - fvn) * dxyip + (fwb - fwt));
+        con = keep ? con : cd * hpki;
       }
-      vcu[(size_t)k * TB + tid] = vcu_k;
-      vcu_prev = vcu_k;
+      lcs[k * 64] = con;
     }
-    ys[(size_t)k * TB + tid] = (T)y;
-    yprev = (double)ys[(size_t)k * TB + tid];
+  } else if (act) {
+    tran_lay_factors(f, i, eebs, ccls, vcus);
   }
-  auto fin = [&](double v) {
-    return f.dye_mode == 1 ? f.dye_f * v : (f.dye_mode == 2 ? v + f.dye_f : v);
-  };
-  double up = (double)ys[(size_t)(KC - 1) * TB + tid];
-  f.con[i + (int64_t)(KC - 1) * p] = (T)fin(up);
-  for (int k = KC - 2; k >= 0; --k) {
-    const double v = (double)ys[(size_t)k * TB + tid] - vcu[(size_t)k * TB + tid] * up;
-    f.con[i + (int64_t)k * p] = (T)fin(v);
-    up = v;
-  }
+  __syncthreads();
+  if (!act || wv != 0) return;
+  const int q = blockIdx.y;
+  tran_lay_solve<T>(KC, (size_t)f.pitch, lcs, eebs, ccls, vcus, nullptr, g.con[q],
+                    (unsigned)i * sizeof(T), g.dye_mode[q], g.dye_f[q], 0.0, 0.0, 0.0, 0.0);
 }
 
 template <typename T>
@@ -1626,41 +1668,69 @@ int adac_pipeline(efdc_ctx *c, TranArgs<T> &ta, const efdc_step_t *step) {
     c->adac_alloc = true;
   }
   AdacArgs<T> a = adac_args<T>(c, ta.uhdy2, ta.vhdx2, ta.w2, ta.hpki, ta.bcrec, step->dt);
-  const dim3 grid((nwet + EFDC_BLOCK - 1) / EFDC_BLOCK, KC);
-  auto lds_for = [&](int tb) { return (sizeof(double) + sizeof(T)) * (size_t)KC * tb; };
-  int tb = TBLOCK;
-  while (tb > 32 && lds_for(tb) > 64 * 1024) tb /= 2;
-  const int nbc = (nwet + tb - 1) / tb;
-  for (int j = 0; j < c->nconst; ++j) {
-    const efdc_constituent_t &d = c->con[j].desc;
-    a.con = ta.nw[j];
-    a.con1 = ta.old[j];
-    a.isadac = d.isadac;
-    a.isfct = d.isfct;
-    if (d.isadac > 0) {
-      if (adj_recording(c)) {
-        const int s = adj_record_adac(c, j, a.con);
+  // As many constituents at a time as keep their scratch within half of the
+  // 256 MB MALL: the passes are short on small grids (253x187x9, 3 constituents, FP64: 8
+  // steps 1217 -> 994 us with the finishing kernel).
+  const int nc = c->nconst;
+  const int fit = (int)((128u << 20) / (8 * plane * sizeof(T)));
+  const int per = std::max(1, std::min({fit, nc, ADAC_GROUP}));
+  if (per > c->adac_sets) {
+    if (c->adac_more) {
+      HIP_TRY(c, hipStreamSynchronize(c->stream));
+      HIP_TRY(c, hipFree(c->adac_more));
+      c->adac_more = nullptr;
+    }
+    c->adac_sets = 1;
+    const int s = dev_alloc(c, &c->adac_more, (size_t)(per - 1) * 8 * plane * sizeof(T));
+    if (s) return s;
+    c->adac_sets = per;
+  }
+  FinishArgs<T> f;
+  f.ad = a;
+  f.ab = ta.ab;
+  f.cdzkk = ta.cdzkk;
+  f.cdzkmk = ta.cdzkmk;
+  f.cdzkk_k = ta.cdzkk_k;
+  f.cdzkmk_k = ta.cdzkmk_k;
+  f.hpi = ta.hpi;
+  f.pitch = c->pitch;
+  f.dt = step->dt;
+  f.KC = KC;
+  f.dz_uniform = ta.dz_uniform;
+  f.pbcflag = c->pbcflag;
+  for (int j0 = 0; j0 < nc; j0 += per) {
+    AdacGroup<T> g;
+    std::memset(&g, 0, sizeof(g));
+    g.n = std::min(per, nc - j0);
+    g.more = (T *)c->adac_more;
+    g.plane = (int64_t)plane;
+    bool adac = false, fct = false;
+    for (int q = 0; q < g.n; ++q) {
+      const int j = j0 + q;
+      const efdc_constituent_t &d = c->con[j].desc;
+      g.con[q] = ta.nw[j];
+      g.con1[q] = ta.old[j];
+      g.isadac[q] = d.isadac;
+      g.isfct[q] = d.isfct;
+      g.dye_mode[q] = ta.dye_mode[j];
+      g.dye_f[q] = ta.dye_f[j];
+      adac = adac || d.isadac > 0;
+      fct = fct || (d.isadac > 0 && d.isfct != 0);
+      if (d.isadac > 0 && adj_recording(c)) {
+        const int s = adj_record_adac(c, j, ta.nw[j]);
         if (s) return s;
       }
-      TIMED(c, TK_ADAC_GRAD, k_adac_grad<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(a));
-      TIMED(c, TK_ADAC_FLUX, k_adac_flux<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(a));
-      if (d.isfct != 0)
-        TIMED(c, TK_FCT, k_fct_beta<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(a));
     }
-    FinishArgs<T> f;
-    f.ad = a;
-    f.con = ta.nw[j];
-    f.ab = ta.ab;
-    f.cdzkk = ta.cdzkk;
-    f.cdzkmk = ta.cdzkmk;
-    f.cdzkk_k = ta.cdzkk_k;
-    f.cdzkmk_k = ta.cdzkmk_k;
-    f.dz_uniform = ta.dz_uniform;
-    f.pbcflag = c->pbcflag;
-    f.adac = d.isadac > 0 ? 1 : 0;
-    f.dye_mode = ta.dye_mode[j];
-    f.dye_f = ta.dye_f[j];
-    TIMED(c, TK_COL_FINISH, k_col_finish<T><<<nbc, tb, lds_for(tb), c->stream>>>(f));
+    const dim3 grid((nwet + EFDC_BLOCK - 1) / EFDC_BLOCK, KC, g.n);
+    if (adac) {
+      TIMED(c, TK_ADAC_GRAD, k_adac_grad<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(a, g));
+      TIMED(c, TK_ADAC_FLUX, k_adac_flux<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(a, g));
+    }
+    if (fct) TIMED(c, TK_FCT, k_fct_beta<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(a, g));
+    const int nlw = std::min(KC, 4);
+    TIMED(c, TK_COL_FINISH,
+          k_adac_finish<T><<<dim3((nwet + 64) / 64, g.n), dim3(64, nlw + (KC > 1 ? 1 : 0)),
+                             sizeof(double) * 4 * 64 * KC, c->stream>>>(f, g, nlw));
   }
   return EFDC_OK;
 }
@@ -2481,9 +2551,9 @@ int adj_adac_impl(efdc_ctx *c, int slot, const AdacAdj &io, const efdc_step_t *s
   const dim3 grid((nwet + EFDC_BLOCK - 1) / EFDC_BLOCK, KC);
   const int nb = (nwet + EFDC_BLOCK - 1) / EFDC_BLOCK;
   // the forward fields from the recorded levels
-  k_adac_grad<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(q.a);
-  k_adac_flux<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(q.a);
-  if (d.isfct != 0) k_fct_beta<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(q.a);
+  k_adac_grad<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(q.a, AdacGroup<T>{});
+  k_adac_flux<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(q.a, AdacGroup<T>{});
+  if (d.isfct != 0) k_fct_beta<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(q.a, AdacGroup<T>{});
   TIMED(c, TK_ADJ_TCOL, k_adj_adac_col<T><<<nb, EFDC_BLOCK, 0, c->stream>>>(q));
   TIMED(c, TK_ADJ_TCOL, k_adj_adac_lim<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(q));
   if (d.isfct != 0) TIMED(c, TK_ADJ_TCOL, k_adj_fct<T><<<grid, EFDC_BLOCK, 0, c->stream>>>(q));
