@@ -48,6 +48,7 @@
 // same partials in the same order, so they take the same branches.
 #include <algorithm>
 #include <cstdio>
+#include <vector>
 
 #include "efdc_internal.h"
 
@@ -140,6 +141,7 @@ struct Xch {
   u64 *ps;             // partials: [parity][workgroup][NVMAX][2 words]
   u64 *hx;             // halo slots: [parity][cell], one word (FP32) or two (FP64) each
   int ncell;
+  int w0, nb;          // the workgroups that take part: w0 .. w0+nb-1
 };
 
 __device__ __forceinline__ u64 *pslot(const Xch &x, unsigned tag, int wg) {
@@ -269,7 +271,7 @@ __device__ __forceinline__ bool exchange(const Xch &x, unsigned tag, const Bar &
                                          double (&sum)[NV], HaloF halo) {
   __shared__ double shs[NV];
   const int t = threadIdx.x, lane = t & 63;
-  const int nb = (int)gridDim.x;
+  const int nb = x.nb;
   if (t < 64) {
     double v[NV];
 #pragma unroll
@@ -285,7 +287,7 @@ __device__ __forceinline__ bool exchange(const Xch &x, unsigned tag, const Bar &
         bool ready = true;
 #pragma unroll
         for (int u = 0; u < UG; ++u) {
-          const u64 *q = pslot(x, tag, min(ln + 64 * (u0 + u), nb - 1));  // every lane loads
+          const u64 *q = pslot(x, tag, x.w0 + min(ln + 64 * (u0 + u), nb - 1));  // every lane loads
 #pragma unroll
           for (int j = 0; j < NV; ++j) {
             lo[u][j] = get_word(q + 2 * j);
@@ -387,9 +389,19 @@ struct P64Args {
   CgState *st;
   double rsqm, rel_tol;
   int iterm;
+  // basins: {first cell, end of the basin, first workgroup, workgroups} and
+  // the basin of every workgroup, the basins' states
+  const int4 *wg;
+  const int *wgseg;
+  CgState *segst;
 };
 
-template <int CPT>
+// SEG: every basin of an ensemble is a solve of its own, by the workgroups of
+// its cells: sums, stop test and iteration count are the basin's, and a basin
+// that has stopped frees its workgroups while the others go on.  Against two
+// launches over all basins per iteration, whose vectors go through memory (40
+// basins of 16000 cells, FP64, 15 iterations): 4 steps 3460 -> 1949 us.
+template <int CPT, bool SEG>
 __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   // the window, then one word that stays zero (read in place of a
   // neighbour that is not a cell, so that every lane loads)
@@ -398,9 +410,21 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   __shared__ double zh[HMAX];  // z of the outside cells
   constexpr int ZS = 2 * WIN + CPT * PB;
   // below the most cells per thread there are at most PCG64_NB workgroups
-  constexpr int UG = CPT < PCG64_CPT_MAX ? 2 : 4;
-  const int b0 = 1 + (int)blockIdx.x * CPT * PB;
-  const int b1 = min(b0 + CPT * PB, a.nwet + 1);
+  constexpr int UG = SEG ? 1 : CPT < PCG64_CPT_MAX ? 2 : 4;
+  int b0 = 1 + (int)blockIdx.x * CPT * PB, b1 = min(b0 + CPT * PB, a.nwet + 1);
+  Xch xc = a.xc;
+  // the cells of this solve: in the row-major form the first cell of a basin
+  // has the last one of the basin before it for i-1, uncoupled
+  int c0 = 1, c1 = a.lc0;
+  if (SEG) {
+    const int4 q = a.wg[blockIdx.x];
+    b0 = q.x;
+    b1 = min(b0 + CPT * PB, q.y);
+    c0 = a.wg[q.z].x;
+    c1 = q.y;
+    xc.w0 = q.z;
+    xc.nb = q.w;
+  }
   const bool fast = a.rowmajor && (a.st->symok == 0);
   const int lc0 = a.lc0;
 
@@ -410,10 +434,10 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   unsigned expo = 0u;        // bit k: another workgroup reads cell k
 
   auto inside = [&](int j) { return j >= b0 && j < b1; };
-  auto real = [&](int j) { return j > 0 && j < lc0; };
+  auto real = [&](int j) { return j >= c0 && j < c1; };
   auto slot = [&](int j) { return j - b0 + WIN; };
   auto publish_z = [&](int i, unsigned tag, double z) {
-    put_f64(hslot64(a.xc, tag) + 2 * (size_t)opaque(i), tag, z);
+    put_f64(hslot64(xc, tag) + 2 * (size_t)opaque(i), tag, z);
   };
 
   for (int g = threadIdx.x; g < 2 * WIN; g += PB) hl[g] = 0;
@@ -476,7 +500,7 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
 
   unsigned tag = a.tag0;
   auto halo = [&](int t, int nt) {
-    halo64<2>(a.xc, tag, nhalo, t, nt, a.bar, [&](int h) { return hl[h]; },
+    halo64<2>(xc, tag, nhalo, t, nt, a.bar, [&](int h) { return hl[h]; },
               [&](int h, double z) { zh[h] = z; });
   };
   // exchange: z of the outside cells (the owner forms it, so they load no
@@ -484,9 +508,9 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
 #pragma unroll
   for (int k = 0; k < CPT; ++k)
     if (expo & (1u << k)) publish_z(b0 + k * PB + (int)threadIdx.x, tag, cci[k] * r[k]);
-  post<2>(v2, a.xc, tag);
+  post<2>(v2, xc, tag);
   double s2[2];
-  if (!exchange<2, UG>(a.xc, tag, a.bar, s2, halo)) return;
+  if (!exchange<2, UG>(xc, tag, a.bar, s2, halo)) return;
   double rpcg = s2[0];
   const double bnorm2 = s2[1];
   const double rsqm = a.rel_tol > 0.0 ? a.rel_tol * a.rel_tol * bnorm2 : a.rsqm;
@@ -525,9 +549,9 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
       v1[0] += ap[k] * p[k];
     }
     ++tag;
-    post<1>(v1, a.xc, tag);
+    post<1>(v1, xc, tag);
     double s1[1];
-    if (!exchange<1, UG>(a.xc, tag, a.bar, s1, NoHalo())) return;
+    if (!exchange<1, UG>(xc, tag, a.bar, s1, NoHalo())) return;
     papcg = s1[0];
     alpha = rpcg / papcg;  // :124
     double v[2] = {0.0, 0.0};
@@ -543,8 +567,8 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
       v[1] += rr * rr;
       if (expo & (1u << k)) publish_z(i, tag, z);
     }
-    post<2>(v, a.xc, tag);
-    if (!exchange<2, UG>(a.xc, tag, a.bar, s2, halo)) return;
+    post<2>(v, xc, tag);
+    if (!exchange<2, UG>(xc, tag, a.bar, s2, halo)) return;
     beta = s2[0] / rpcg;  // :147-148
     rpcg = s2[0];
     rsq = s2[1];
@@ -557,8 +581,8 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
     const int i = b0 + k * PB + (int)threadIdx.x;
     if (i < b1) a.x[opaque(i)] = x[k];
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    CgState *st = a.st;
+  if ((int)blockIdx.x == xc.w0 && threadIdx.x == 0) {
+    CgState *st = SEG ? a.segst + a.wgseg[blockIdx.x] : a.st;
     st->rpcg = rpcg;
     st->papcg = papcg;
     st->alpha = alpha;
@@ -1573,8 +1597,8 @@ int pcg_prepare(efdc_ctx *c) {
   HIP_TRY(c, hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
   c->pcg_ncu = coop ? ncu : 0;
   const int occ64[PCG64_CPT_MAX + 1] = {
-      0, occupancy(k_pcg64<1>), occupancy(k_pcg64<2>), occupancy(k_pcg64<3>),
-      occupancy(k_pcg64<4>), occupancy(k_pcg64<5>), occupancy(k_pcg64<6>)};
+      0, occupancy(k_pcg64<1, false>), occupancy(k_pcg64<2, false>), occupancy(k_pcg64<3, false>),
+      occupancy(k_pcg64<4, false>), occupancy(k_pcg64<5, false>), occupancy(k_pcg64<6, false>)};
   const int occmx[PCGMX_CPT_SMALL + 1] = {
       0, occupancy(k_pcgmx<1>), occupancy(k_pcgmx<2>), occupancy(k_pcgmx<3>),
       occupancy(k_pcgmx<4>), occupancy(k_pcgmx<5>), occupancy(k_pcgmx<6>),
@@ -1588,7 +1612,11 @@ int pcg_prepare(efdc_ctx *c) {
   const int occ64p[PCG64_CPT_MAX + 1] = {
       0, occupancy(k_pcg64_pl<1>), occupancy(k_pcg64_pl<2>), occupancy(k_pcg64_pl<3>),
       occupancy(k_pcg64_pl<4>), occupancy(k_pcg64_pl<5>), occupancy(k_pcg64_pl<6>)};
-  for (int k = 0; k <= PCG64_CPT_MAX; ++k) c->pcg_occ64[k] = std::min(occ64[k], occ64p[k]);
+  const int occ64s[PCG64_CPT_MAX + 1] = {
+      0, occupancy(k_pcg64<1, true>), occupancy(k_pcg64<2, true>), occupancy(k_pcg64<3, true>),
+      occupancy(k_pcg64<4, true>), occupancy(k_pcg64<5, true>), occupancy(k_pcg64<6, true>)};
+  for (int k = 0; k <= PCG64_CPT_MAX; ++k)
+    c->pcg_occ64[k] = std::min({occ64[k], occ64p[k], occ64s[k]});
   for (int k = 0; k <= PCGMX_CPT_MAX; ++k)
     c->pcg_occmx[k] = k <= PCGMX_CPT_SMALL ? std::min(occmx[k], occpl[k]) : occpl[k];
   c->pcg_ncell = c->n_wet() + 2;
@@ -1693,6 +1721,45 @@ static int next_tag0(efdc_ctx *c, unsigned &tag0) {
   return EFDC_OK;
 }
 
+static int p64_args(efdc_ctx *c, int nb, const Bar &bar, P64Args &a) {
+  a.ccc = c->dH[EFDC_CCC];
+  a.ccs = c->dH[EFDC_CCS];
+  a.ccw = c->dH[EFDC_CCW];
+  a.ccn = c->dH[EFDC_CCN];
+  a.cce = c->dH[EFDC_CCE];
+  a.ccci = c->dH[EFDC_CCCI];
+  a.fptmp = c->dH[EFDC_FPTMP];
+  a.x = c->dH[EFDC_P];
+  a.lw = c->dLW;
+  a.le = c->dLE;
+  a.ls = c->dLS;
+  a.ln = c->dLN;
+  a.nwet = c->n_wet();
+  a.lc0 = c->LC - 1;
+  a.rowmajor = c->rowmajor ? 1 : 0;
+  a.mutual = c->mutual ? 1 : 0;
+  a.xc = Xch{(u64 *)c->pcg_ps, (u64 *)c->pcg_hx, c->pcg_ncell, 0, nb};
+  int s;
+  if ((s = next_tag0(c, a.tag0))) return s;
+  a.bar = bar;
+  a.st = c->st;
+  a.rsqm = c->prm.RSQM;
+  a.rel_tol = c->prm.cg_rel_tol;
+  a.iterm = c->prm.ITERM;
+  a.wg = nullptr;
+  a.wgseg = nullptr;
+  a.segst = nullptr;
+  return EFDC_OK;
+}
+
+// Bounded waits: a plain launch may be given a small spin limit (to exercise
+// the retry from the host); the cooperative one always has the full limit.
+static Bar pcg_bar(efdc_ctx *c) {
+  const bool plain = c->pcg_launch_mode == 0 && !c->pcg_force_coop;
+  return Bar{c->pcg_ctr, c->pcg_abort,
+             plain && c->pcg_spin_test > 0 ? c->pcg_spin_test : SPIN_MAX};
+}
+
 int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
   int s;
   if ((s = pcg_prepare(c))) return s;
@@ -1702,38 +1769,12 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
   }
   c->pcg_reset_done = false;  // this launch uses them
   int nb = 0;
-  // a plain launch may be given a small spin limit (to exercise the retry
-  // from the host); the cooperative one always has the full limit
-  const bool plain = c->pcg_launch_mode == 0 && !c->pcg_force_coop;
-  Bar bar{c->pcg_ctr, c->pcg_abort,
-          plain && c->pcg_spin_test > 0 ? c->pcg_spin_test : SPIN_MAX};
+  const Bar bar = pcg_bar(c);
   if (!mixed) {
     const int cpt = pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb, PCG64_NB);
     if (!cpt) { c->err = "persistent CG: problem too large"; return EFDC_ERR_ARG; }
     P64Args a;
-    a.ccc = c->dH[EFDC_CCC];
-    a.ccs = c->dH[EFDC_CCS];
-    a.ccw = c->dH[EFDC_CCW];
-    a.ccn = c->dH[EFDC_CCN];
-    a.cce = c->dH[EFDC_CCE];
-    a.ccci = c->dH[EFDC_CCCI];
-    a.fptmp = c->dH[EFDC_FPTMP];
-    a.x = c->dH[EFDC_P];
-    a.lw = c->dLW;
-    a.le = c->dLE;
-    a.ls = c->dLS;
-    a.ln = c->dLN;
-    a.nwet = c->n_wet();
-    a.lc0 = c->LC - 1;
-    a.rowmajor = c->rowmajor ? 1 : 0;
-    a.mutual = c->mutual ? 1 : 0;
-    a.xc = Xch{(u64 *)c->pcg_ps, (u64 *)c->pcg_hx, c->pcg_ncell};
-    if ((s = next_tag0(c, a.tag0))) return s;
-    a.bar = bar;
-    a.st = c->st;
-    a.rsqm = c->prm.RSQM;
-    a.rel_tol = c->prm.cg_rel_tol;
-    a.iterm = c->prm.ITERM;
+    if ((s = p64_args(c, nb, bar, a))) return s;
     const void *fn = nullptr;
     if (c->pcg64_pipe) {
       switch (cpt) {
@@ -1746,12 +1787,12 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
       }
     } else {
       switch (cpt) {
-        case 1: fn = (const void *)k_pcg64<1>; break;
-        case 2: fn = (const void *)k_pcg64<2>; break;
-        case 3: fn = (const void *)k_pcg64<3>; break;
-        case 4: fn = (const void *)k_pcg64<4>; break;
-        case 5: fn = (const void *)k_pcg64<5>; break;
-        default: fn = (const void *)k_pcg64<6>; break;
+        case 1: fn = (const void *)k_pcg64<1, false>; break;
+        case 2: fn = (const void *)k_pcg64<2, false>; break;
+        case 3: fn = (const void *)k_pcg64<3, false>; break;
+        case 4: fn = (const void *)k_pcg64<4, false>; break;
+        case 5: fn = (const void *)k_pcg64<5, false>; break;
+        default: fn = (const void *)k_pcg64<6, false>; break;
       }
     }
     TIMED(c, TK_PCG64, s = coop_launch(c, fn, nb, a));
@@ -1779,7 +1820,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
     a.ln = c->dLN;
     a.nwet = c->n_wet();
     a.lc0 = c->LC - 1;
-    a.xc = Xch{(u64 *)c->pcg_ps, (u64 *)c->pcg_hx, c->pcg_ncell};
+    a.xc = Xch{(u64 *)c->pcg_ps, (u64 *)c->pcg_hx, c->pcg_ncell, 0, nb};
     if ((s = next_tag0(c, a.tag0))) return s;
     a.bar = bar;
     a.st = c->st;
@@ -1846,6 +1887,88 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
     return EFDC_ERR_HIP;
   }
   return EFDC_OK;
+}
+
+// Cells per thread with which every basin's workgroups fit one co-resident
+// grid together, and their number; 0 if they do not.
+static int pcg_seg_shape(const efdc_ctx *c, int &nb) {
+  for (int cpt = 1; cpt <= PCG64_CPT_MAX; ++cpt) {
+    const int cap = std::min(c->pcg_occ64[cpt] * c->pcg_ncu, PB);
+    long need = 0;
+    for (int q = 0; q < c->nseg; ++q)
+      need += (c->seg_first[q + 1] - c->seg_first[q] + cpt * PB - 1) / (cpt * PB);
+    if (need <= cap) {
+      nb = (int)need;
+      return cpt;
+    }
+  }
+  return 0;
+}
+
+bool pcg_seg_applicable(efdc_ctx *c) {
+  int nb = 0;
+  return c->prm.cg_kernel != EFDC_CG_KERNEL_MULTI && c->band <= WIN &&
+         1L + 2L * c->prm.ITERM < PCG_TAGS_PER_LAUNCH && pcg_prepare(c) == EFDC_OK &&
+         c->pcg_ncu > 0 && pcg_seg_shape(c, nb) > 0;
+}
+
+// The FP64 solve of every basin in one persistent launch; the basins' states
+// are in h_segst afterwards.
+int pcg_seg_solve(efdc_ctx *c) {
+  int s, nb = 0;
+  const int cpt = pcg_seg_shape(c, nb);
+  if (!c->pcg_segwg) {  // (dropped with the basins)
+    std::vector<int4> wg;
+    std::vector<int> seg;
+    for (int q = 0; q < c->nseg; ++q) {
+      const int w0 = (int)wg.size(), end = c->seg_first[q + 1];
+      for (int i = c->seg_first[q]; i < end; i += cpt * PB) {
+        wg.push_back(make_int4(i, end, w0, 0));
+        seg.push_back(q);
+      }
+      for (size_t w = w0; w < wg.size(); ++w) wg[w].w = (int)wg.size() - w0;
+    }
+    if ((s = dev_alloc(c, &c->pcg_segwg, (sizeof(int4) + sizeof(int)) * wg.size()))) return s;
+    HIP_TRY(c, hipMemcpyAsync(c->pcg_segwg, wg.data(), sizeof(int4) * wg.size(),
+                              hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, hipMemcpyAsync((int4 *)c->pcg_segwg + wg.size(), seg.data(),
+                              sizeof(int) * seg.size(), hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+  }
+  k_pcg_reset<<<1, PCG_NCTR, 0, c->stream>>>(c->pcg_ctr, c->pcg_abort);
+  HIP_TRY(c, hipGetLastError());
+  P64Args a;
+  if ((s = p64_args(c, nb, pcg_bar(c), a))) return s;
+  a.wg = (const int4 *)c->pcg_segwg;
+  a.wgseg = (const int *)(a.wg + nb);
+  a.segst = c->d_segst;
+  const void *fn = nullptr;
+  switch (cpt) {
+    case 1: fn = (const void *)k_pcg64<1, true>; break;
+    case 2: fn = (const void *)k_pcg64<2, true>; break;
+    case 3: fn = (const void *)k_pcg64<3, true>; break;
+    case 4: fn = (const void *)k_pcg64<4, true>; break;
+    case 5: fn = (const void *)k_pcg64<5, true>; break;
+    default: fn = (const void *)k_pcg64<6, true>; break;
+  }
+  TIMED(c, TK_PCG64, s = coop_launch(c, fn, nb, a));
+  if (s) return s;
+  HIP_TRY(c, hipMemcpyAsync(c->h_segst, c->d_segst, sizeof(CgState) * c->nseg,
+                            hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(c, hipMemcpyAsync(c->st_host, c->st, sizeof(CgState), hipMemcpyDeviceToHost,
+                            c->stream));
+  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (!c->st_host->pabort) return EFDC_OK;
+  if (!c->pcg_last_plain) {
+    c->err = "persistent CG: an exchange between workgroups timed out";
+    return EFDC_ERR_HIP;
+  }
+  // not co-resident: again, cooperatively, from the P each basin reached
+  ++c->pcg_retries;
+  c->pcg_force_coop = true;
+  s = pcg_seg_solve(c);
+  c->pcg_force_coop = false;
+  return s;
 }
 
 // Autotuner of the mixed persistent solve: the degree of the local

@@ -156,6 +156,7 @@ struct efdc_ctx {
   int pcg_occ64[7] = {}, pcg_occmx[17] = {};  // workgroups per CU by CPT
   void *pcg_hx = nullptr;      // halo slots [2][ncell][2] tagged words
   void *pcg_ps = nullptr;      // partial slots
+  void *pcg_segwg = nullptr;   // workgroup tables of the basins' persistent solve
   int pcg_ncell = 0;
   unsigned pcg_launch = 0;     // launch number, gives the first tag
   unsigned *pcg_ctr = nullptr; // barrier counters
@@ -604,6 +605,8 @@ int efdc_grid_blocks(int n);
 void efdc_thread_error(const char *why);
 // persistent CONGRAD (efdc_cgp.hip)
 bool pcg_applicable(efdc_ctx *c, bool mixed);
+bool pcg_seg_applicable(efdc_ctx *c);
+int pcg_seg_solve(efdc_ctx *c);
 int pcg_solve(efdc_ctx *c, bool mixed, bool defer = false);
 int pcg_tune_degree(efdc_ctx *c);
 // independent basins (efdc_seg.hip)

@@ -2310,10 +2310,14 @@ int seg_cg_run(efdc_ctx *c, efdc_cg_stats_t *stats, bool *ran_mixed) {
   if (c->cg_graph_tune && !c->timing &&
       (s = cg_graph_trial(c, [&](bool g) { return seg_solve_set(c, c->seg_tset, g); })))
     return s;
-  if ((s = seg_solve_set(c, c->seg_tset, c->cg_graph && !c->timing))) return s;
-  HIP_TRY(c, hipMemcpyAsync(c->h_segst, c->d_segst, sizeof(CgState) * c->nseg,
-                            hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (pcg_seg_applicable(c)) {
+    if ((s = pcg_seg_solve(c))) return s;
+  } else {
+    if ((s = seg_solve_set(c, c->seg_tset, c->cg_graph && !c->timing))) return s;
+    HIP_TRY(c, hipMemcpyAsync(c->h_segst, c->d_segst, sizeof(CgState) * c->nseg,
+                              hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+  }
   int imax = 0, bad = 0;
   double rsq = 0.0;
   for (int q = 0; q < c->nseg; ++q) {

@@ -64,7 +64,7 @@ void seg_free(efdc_ctx *c) {
   c->d_segtile0 = nullptr;
   f(c->d_segid); f(c->d_segfirst); f(c->d_segst);
   f(c->d_segtk); f(c->d_segdone); f(c->d_segmin); f(c->d_segpart); f(c->d_segbal);
-  f(c->d_segfin);
+  f(c->d_segfin); f(c->pcg_segwg);
   if (c->h_segst) (void)hipHostFree(c->h_segst);
   c->h_segst = nullptr;
   c->nseg = 1;

@@ -1,0 +1,75 @@
+"""The FP64 solve of an ensemble's basins in one persistent launch (the
+default) against the two-launches-per-iteration solve: the same iterations
+to within one and levels within round-off of the FP64 CG."""
+import numpy as np
+import pytest
+
+from conftest import eta_err
+from test_gpu_ensemble import _ctx, _tidal_ensemble
+
+pytestmark = pytest.mark.gpu
+
+
+def _many(n):
+    from efdc_amd import grids
+    return grids.concat_basins(
+        [grids.tidal_basin(12 + 4 * (i % 4), 10 + 3 * (i % 2), 2, seed=300 + i,
+                           amp=0.05 + 0.003 * (i % 50)) for i in range(n)])
+
+
+def _lakes():
+    from efdc_amd import grids
+    return grids.concat_basins([grids.external_case(grids.lake_mask(n, n, s), seed=s)
+                                for n, s in ((48, 31), (330, 32), (33, 33), (20, 35))])
+
+
+# 5 basins; lakes of 100 to 50000 cells (several workgroups a basin); as many
+# basins as workgroups of the chip; more than that (launch by launch)
+@pytest.mark.parametrize("make,persistent", [
+    (lambda: _tidal_ensemble()[1:], True), (_lakes, True),
+    (lambda: _many(256), True), (lambda: _many(600), False),
+])
+def test_basins_persistent_against_launches(make, persistent):
+    from efdc_amd import lib
+    ens, first = make()
+    a, b = _ctx(ens, cg_kernel=lib.CG_KERNEL_AUTO), _ctx(ens)
+    for x in (a, b):
+        x.set_segments(first)
+    a.timers(True)
+    for n in range(1, 7):
+        a.calpuv2c(ens.dt, n)
+        b.calpuv2c(ens.dt, n)
+        ia, sa = a.segment_stats()
+        ib, sb = b.segment_stats()
+        assert not np.any(sa) and not np.any(sb)
+        assert np.max(np.abs(np.asarray(ia) - np.asarray(ib))) <= 1
+    assert ("cg_persistent64" in a.read_timers()) == persistent
+    L = np.arange(1, ens.grid.LA)
+    assert eta_err(a.get("P")[L], b.get("P")[L]) <= 1e-9
+    a.close()
+    b.close()
+
+
+def test_basins_persistent_cap_and_repeated_launch():
+    from efdc_amd import lib
+    _, ens, first = _tidal_ensemble()
+    c = _ctx(ens, cg_kernel=lib.CG_KERNEL_AUTO, RSQM=1e-30, ITERM=3)
+    c.set_segments(first)
+    with pytest.raises(lib.EfdcError) as e:
+        c.calpuv2c(ens.dt, 1)
+    assert e.value.status == 3
+    it, status = c.segment_stats()
+    assert list(it) == [3] * len(first) and list(status) == [3] * len(first)
+    c.close()
+    # a plain launch whose waits give up is repeated cooperatively
+    a, b = _ctx(ens, cg_kernel=lib.CG_KERNEL_AUTO), _ctx(ens)
+    a.set_segments(first)
+    b.set_segments(first)
+    a.set_cg_launch(0, spin_limit=1)
+    a.calpuv2c(ens.dt, 1)
+    b.calpuv2c(ens.dt, 1)
+    assert a.cg_launch()[1] >= 1
+    L = np.arange(1, ens.grid.LA)
+    assert eta_err(a.get("P")[L], b.get("P")[L]) <= 1e-9
+    a.close()
+    b.close()
