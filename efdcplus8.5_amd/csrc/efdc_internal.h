@@ -605,6 +605,9 @@ int efdc_grid_blocks(int n);
 void efdc_thread_error(const char *why);
 // persistent CONGRAD (efdc_cgp.hip)
 bool pcg_applicable(efdc_ctx *c, bool mixed);
+bool pcg_vec_applicable(efdc_ctx *c, int itmax);
+int pcg_vec_solve(efdc_ctx *c, double *x, const double *rhs, CgState *st, CgState *st_host,
+                  double rel_tol, int itmax);
 bool pcg_seg_applicable(efdc_ctx *c);
 int pcg_seg_solve(efdc_ctx *c);
 int pcg_solve(efdc_ctx *c, bool mixed, bool defer = false);

@@ -1761,6 +1761,19 @@ void cg_graphs_free(efdc_ctx *c) {
 
 int cg_fp64_vec(efdc_ctx *c, double *x, const double *rhs, CgState *st, CgState *st_host,
                 double rel_tol, int itmax, int *iters, double *rsq) {
+  // 40 k cells, 16 iterations: one persistent launch of 60 us against 32 of 7.1
+  // and 6.4 us
+  if (pcg_vec_applicable(c, itmax)) {
+    const int s = pcg_vec_solve(c, x, rhs, st, st_host, rel_tol, itmax);
+    if (s) return s;
+    *iters = st_host->iter;
+    *rsq = st_host->rsq;
+    if (!st_host->done || st_host->status) {
+      c->err = "adjoint CG: no convergence within the iteration cap";
+      return EFDC_ERR_CG_MAXITER;
+    }
+    return EFDC_OK;
+  }
   const int nb = cg_blocks(c->n_wet());
   CgArgs a = cg_args(c);
   a.x = x;
