@@ -218,26 +218,31 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_assemble(
 // one launch over all boundary cells takes the minimum of their CC and
 // zeroes the couplings into the clamped cells.
 // ---------------------------------------------------------------------
+constexpr int TIDE_ARGS = 16;
 struct PbcArgs {
   PbcDev side[4];
-  const double *tide;  // cos(M) at [M], sin(M) at [mtide+M]
+  // cos(M) at [M], sin(M) at [mtide+M]: in the arguments up to TIDE_ARGS
+  // constituents (a copy to the device was 4 us of each step), in memory beyond
+  const double *tide;
+  double tidev[2 * TIDE_ARGS];
   int mtide;
   int *lopenbcdry;
 };
 
-__global__ __launch_bounds__(EFDC_BLOCK) void k_puv_bc_side(
-    HPtr h, PbcArgs b, PbcDev s, int side, const int *__restrict__ lw, const int *__restrict__ le,
-    const int *__restrict__ ls, const int *__restrict__ ln, double dt,
-    double G, double HDRY) {
+// The open-boundary cells LL0, LL0 + stride, .. of one side.
+__device__ __forceinline__ void bc_side_cells(
+    const HPtr &h, const PbcArgs &b, const PbcDev &s, int side, const int *__restrict__ lw,
+    const int *__restrict__ le, const int *__restrict__ ls, const int *__restrict__ ln, double dt,
+    double G, double HDRY, int LL0, int stride) {
   const double D_LTD2 = 0.5 * dt, DELTI = 1. / dt, DE_TI = DELTI;
   const double HDRY2 = 0.2 * HDRY;
+  const bool args = b.mtide <= TIDE_ARGS;
   double *CC = HA(CC), *CS = HA(CS), *CW = HA(CW), *CE = HA(CE), *CN = HA(CN),
          *FP = HA(FP), *DXYP = HA(DXYP), *BELV = HA(BELV), *HRUO = HA(HRUO),
          *HRVO = HA(HRVO), *RCX = HA(RCX), *RCY = HA(RCY), *HUT = HA(H1U),
          *HVT = HA(H1V), *DXIU = HA(DXIU), *DYIU = HA(DYIU), *DXIV = HA(DXIV),
          *DYIV = HA(DYIV), *FUHDYE = HA(FUHDYE), *FVHDXE = HA(FVHDXE);
   {
-    int LL0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
     if (s.serial) {
       if (LL0 != 0) return;
       stride = 1;
@@ -252,8 +257,8 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_bc_side(
       if (b.lopenbcdry[i]) continue;
       double fp = s.pser[LL];
       for (int M = 0; M < b.mtide; ++M)
-        fp = fp + s.pcb[LL * b.mtide + M] * b.tide[M] +
-             s.psb[LL * b.mtide + M] * b.tide[b.mtide + M];
+        fp = fp + s.pcb[LL * b.mtide + M] * (args ? b.tidev[M] : b.tide[M]) +
+             s.psb[LL * b.mtide + M] * (args ? b.tidev[b.mtide + M] : b.tide[b.mtide + M]);
       FP[i] = fp;
       const bool rad = (s.ispb[LL] == 1 || s.ispb[LL] == 2);
       if (side == 0) {
@@ -345,12 +350,22 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_bc_side(
   }
 }
 
-__global__ __launch_bounds__(EFDC_BLOCK) void k_puv_bc_min(
-    HPtr h, PbcArgs b, int ntot, const int *__restrict__ lw, const int *__restrict__ le,
-    const int *__restrict__ ls, const int *__restrict__ ln, double *part, CgState *st,
-    unsigned *st_tk) {
+__global__ __launch_bounds__(EFDC_BLOCK) void k_puv_bc_side(
+    HPtr h, PbcArgs b, PbcDev s, int side, const int *__restrict__ lw, const int *__restrict__ le,
+    const int *__restrict__ ls, const int *__restrict__ ln, double dt,
+    double G, double HDRY) {
+  bc_side_cells(h, b, s, side, lw, le, ls, ln, dt, G, HDRY,
+                (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
+}
+
+// Entry t of the sides' cells one after the other: its CC, and no coupling
+// from the interior into it if it is clamped.
+__device__ __forceinline__ double bc_min_cell(const HPtr &h, const PbcArgs &b, int t, int ntot,
+                                              const int *__restrict__ lw,
+                                              const int *__restrict__ le,
+                                              const int *__restrict__ ls,
+                                              const int *__restrict__ ln) {
   double *CC = HA(CC), *CS = HA(CS), *CW = HA(CW), *CE = HA(CE), *CN = HA(CN);
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
   double m = 1.E+18;
   if (t < ntot) {
     // side of entry t (the sides' cells follow one another)
@@ -377,10 +392,43 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_bc_min(
       else CN[ls[i]] = 0.;
     }
   }
+  return m;
+}
+
+__global__ __launch_bounds__(EFDC_BLOCK) void k_puv_bc_min(
+    HPtr h, PbcArgs b, int ntot, const int *__restrict__ lw, const int *__restrict__ le,
+    const int *__restrict__ ls, const int *__restrict__ ln, double *part, CgState *st,
+    unsigned *st_tk) {
+  const double m =
+      bc_min_cell(h, b, (int)(blockIdx.x * blockDim.x + threadIdx.x), ntot, lw, le, ls, ln);
   double mm;
   if (grid_min(m, part, st_tk + TS_PUV_MIN * TICKET_SITE, gridDim.x, blockIdx.x, mm) &&
       threadIdx.x == 0)
     st->ccmnm = fmin(st->ccmnm, mm);
+}
+
+// All sides one after the other and the minimum in one workgroup, for up to
+// PBC_ONE cells: every launch more costs more than its work (128x64, one side:
+// 4.5 + 4.7 us and the gap between them).
+constexpr int PBC_ONE = 1024;
+__global__ __launch_bounds__(PBC_ONE) void k_puv_bc_all(
+    HPtr h, PbcArgs b, int ntot, const int *__restrict__ lw, const int *__restrict__ le,
+    const int *__restrict__ ls, const int *__restrict__ ln, double dt, double G, double HDRY,
+    CgState *st) {
+  __shared__ double sh[PBC_ONE / 64];
+  for (int q = 0; q < 4; ++q) {
+    if (b.side[q].n == 0) continue;
+    bc_side_cells(h, b, b.side[q], q, lw, le, ls, ln, dt, G, HDRY, (int)threadIdx.x, PBC_ONE);
+    __syncthreads();  // a corner cell may be in two sides
+  }
+  const double m = wave_min(bc_min_cell(h, b, (int)threadIdx.x, ntot, lw, le, ls, ln));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double mm = sh[0];
+    for (int q = 1; q < PBC_ONE / 64; ++q) mm = fmin(mm, sh[q]);
+    st->ccmnm = fmin(st->ccmnm, mm);
+  }
 }
 
 // ---------------------------------------------------------------------
@@ -404,6 +452,7 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_scale(
     for (int q = threadIdx.x; q < nctr; q += blockDim.x) rctr[q] = 0u;
     if (threadIdx.x == 0) *rabort = 0;
   }
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->drychg = 0;
   int tile;
   const int i = cell_index(nwet, tile);
   if (i > nwet) return;
@@ -1127,8 +1176,8 @@ __global__ void k_fill_u32x2(unsigned *a, unsigned *b) {
 // EFDC/negdep.f90:34-45 (negative depth flag).
 // ---------------------------------------------------------------------
 __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_post1(
-    HPtr h, const int *__restrict__ lw, const int *__restrict__ ls, int nwet,
-    double dt) {
+    HPtr h, const int *__restrict__ lw, const int *__restrict__ ls,
+    const unsigned char *__restrict__ pbcflag, int nwet, double dt, double G) {
   int tile;
   const int i = cell_index(nwet, tile);
   if (i > nwet) return;
@@ -1143,6 +1192,27 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_post1(
   HA(VHDXE)[i] = v;
   HA(UHE)[i] = u * HA(DYIU)[i];
   HA(VHE)[i] = v * HA(DXIV)[i];
+  // the depth of an open-boundary cell comes from P: here, so that
+  // k_puv_post23, which changes P, reads no neighbour's P
+  if (pbcflag[i]) {
+    const double GI = 1. / G;
+    HA(HP)[i] = GI * P[i] - HA(BELV)[i];
+  }
+}
+
+// Depth of cell j after the solve (:541-558): k_puv_post1 has formed the
+// open-boundary cells'; a ghost's stays.
+__device__ __forceinline__ double depth_of(const HPtr &h, const int *__restrict__ le,
+                                           const int *__restrict__ ln,
+                                           const unsigned char *__restrict__ pbcflag, int j,
+                                           int nwet, double DELTD2) {
+  const int e = le[j], n = ln[j];
+  const double *U = HA(UHDYE), *U1 = HA(UHDY1E), *V = HA(VHDXE), *V1 = HA(VHDX1E);
+  const double hp = HA(H1P)[j] + DELTD2 * HA(DXYIP)[j] *
+                                     (2. * HA(QSUME)[j] -
+                                      (U[e] + U1[e] - U[j] - U1[j] + V[n] + V1[n] - V[j] - V1[j]));
+  const double old = HA(HP)[j];
+  return (j < 1 || j > nwet || pbcflag[j]) ? old : hp;
 }
 
 __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_post2(
@@ -1151,15 +1221,40 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_post2(
   int tile;
   const int i = cell_index(nwet, tile);
   if (i > nwet) return;
-  const double DELTD2 = 0.5 * dt, GI = 1. / G;
-  const int e = le[i], n = ln[i];
-  const double *U = HA(UHDYE), *U1 = HA(UHDY1E), *V = HA(VHDXE), *V1 = HA(VHDX1E);
-  double hp = HA(H1P)[i] + DELTD2 * HA(DXYIP)[i] *
-                               (2. * HA(QSUME)[i] -
-                                (U[e] + U1[e] - U[i] - U1[i] + V[n] + V1[n] - V[i] - V1[i]));
-  if (pbcflag[i]) hp = GI * HA(P)[i] - HA(BELV)[i];
+  const double hp = depth_of(h, le, ln, pbcflag, i, nwet, 0.5 * dt);
   HA(HP)[i] = hp;
   HA(P)[i] = G * (hp + HA(BELV)[i]);
+}
+
+// k_puv_post2 and k_puv_post3 in one pass, for steps without drying: the west
+// and south cells' depths are formed again from the flows (k_puv_post2's
+// operations, the same bits) instead of read back after a launch.  Three times
+// the loads, from the caches while the arrays fit them: up to POST23_MAX cells
+// (us a step, one pass : two; 6 k cells 117 : 124, 79 k 141 : 145, 255 k 171.5 :
+// 173; 696 k 282 : 279, 2.02 M 908 : 885).
+constexpr int POST23_MAX = 1 << 18;
+__global__ __launch_bounds__(EFDC_BLOCK) void k_puv_post23(
+    HPtr h, const int *__restrict__ lw, const int *__restrict__ le, const int *__restrict__ ls,
+    const int *__restrict__ ln, const unsigned char *__restrict__ pbcflag, int nwet, double dt,
+    double G, CgState *st) {
+  int tile;
+  const int i = cell_index(nwet, tile);
+  if (i > nwet) return;
+  const int w = lw[i], s = ls[i];
+  const double hp = depth_of(h, le, ln, pbcflag, i, nwet, 0.5 * dt);
+  const double hw = depth_of(h, le, ln, pbcflag, w, nwet, 0.5 * dt);
+  const double hs = depth_of(h, le, ln, pbcflag, s, nwet, 0.5 * dt);
+  const double *DXYP = HA(DXYP);
+  const double hu = (DXYP[i] * hp + DXYP[w] * hw) * (0.5 / HA(DXYU)[i]);
+  const double hv = (DXYP[i] * hp + DXYP[s] * hs) * (0.5 / HA(DXYV)[i]);
+  if (!pbcflag[i]) HA(HP)[i] = hp;
+  HA(P)[i] = G * (hp + HA(BELV)[i]);
+  HA(HU)[i] = hu;
+  HA(HV)[i] = hv;
+  HA(HPI)[i] = 1. / hp;
+  HA(HUI)[i] = 1. / hu;
+  HA(HVI)[i] = 1. / hv;
+  if (hp <= 0.) st->negdep = 1;
 }
 
 __global__ __launch_bounds__(EFDC_BLOCK) void k_puv_post3(
@@ -1208,7 +1303,8 @@ __global__ void k_dry_obc_reset(PbcDev s, int *lopenbcdry) {
 // its own cell and zeros faces it shares with its east / north
 // neighbours (the same value from every writer).
 __global__ void k_dry_obc(HPtr h, PbcDev s, const int *le, const int *ln, int *lopenbcdry,
-                          int *iscdry, double dt, double G, double HDRY) {
+                          int *iscdry, double dt, double G, double HDRY, const CgState *st) {
+  if (st->pabort) return;  // an abandoned solve is repeated first
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= s.n) return;
   const int i = s.L[t];
@@ -1260,6 +1356,7 @@ __device__ __forceinline__ void raise_flag_once(bool mine, CgState *st) {
 __global__ __launch_bounds__(EFDC_BLOCK) void k_dry_cells(HPtr h, const int *le, const int *ln,
                                                           int *iscdry, int nwet, double HDRY,
                                                           CgState *st) {
+  if (st->pabort) return;
   int tile;
   const int i = cell_index(nwet, tile);
   bool newly = false;
@@ -1278,7 +1375,6 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_dry_cells(HPtr h, const int *le,
   raise_flag_once(newly, st);
 }
 
-__global__ void k_dry_flag_reset(CgState *st) { st->drychg = 0; }
 
 // Draining of isolated wet cells, NDRYSTP < 0 (:838-893, 1010-1018): a wet
 // cell (HP >= HDRY) whose four faces are closed counts its isolated steps
@@ -1362,6 +1458,7 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_dry99(HPtr h, const int *lw, con
                                                       int *iscdry, double *sub_n,
                                                       double *svb_n, int nwet, double HDRY,
                                                       CgState *st) {
+  if (st->pabort) return;
   int tile;
   const int i = cell_index(nwet, tile);
   bool chg = false;
@@ -1414,7 +1511,9 @@ __global__ __launch_bounds__(EFDC_BLOCK) void k_dry99(HPtr h, const int *lw, con
 }
 
 __global__ __launch_bounds__(EFDC_BLOCK) void k_dry99_commit(HPtr h, const double *sub_n,
-                                                             const double *svb_n, int nwet) {
+                                                             const double *svb_n, int nwet,
+                                                             const CgState *st) {
+  if (st->pabort) return;
   int tile;
   const int i = cell_index(nwet, tile);
   if (i > nwet) return;
@@ -1887,10 +1986,36 @@ int puv_run(efdc_ctx *c, const efdc_step_t *step, efdc_cg_stats_t *stats) {
         c->prm.RITB1, c->prm.SNLT, dry ? 1 : 0, c->prm.implicit_drag ? 1 : 0, rot, fold,
         c->st));
   c->ncordry = 0;
-  // a step that may solve more than once (drying) or records the solution
-  // (adjoint) launches the persistent solve cooperatively, so that it never
-  // has to be solved again after the passes that follow it
-  c->pcg_force_coop = dry || adj_recording(c);
+  const bool post23 = !dry && nwet <= POST23_MAX;
+  const bool cells = c->prm.ISDRY < 98 || c->prm.ISDRY == 99;
+  // the passes between a solve and the drying test
+  auto after_solve = [&]() -> int {
+    int q;
+    if (adj_recording(c) && (q = adj_record_ps(c))) return q;
+    TIMED(c, TK_PUV_POST1, k_puv_post1<<<nb, EFDC_BLOCK, 0, c->stream>>>(
+        h, c->dLW, c->dLS, c->pbcflag, nwet, dt, G));
+    if (post23) return EFDC_OK;
+    TIMED(c, TK_PUV_POST2, k_puv_post2<<<nb, EFDC_BLOCK, 0, c->stream>>>(
+        h, c->dLE, c->dLN, c->pbcflag, nwet, dt, G));
+    if (!dry) return EFDC_OK;
+    // open-boundary drying (:497-530), then the cell drying and its flag
+    // (:574-602); P already is G (HP + BELV) (:559-569, k_puv_post2)
+    for (int q = 0; q < 4; ++q)
+      if (c->pbc[q].n > 0)
+        k_dry_obc<<<(c->pbc[q].n + 255) / 256, 256, 0, c->stream>>>(
+            h, c->pbc[q], c->dLE, c->dLN, c->lopenbcdry, c->iscdry, dt, G, c->prm.HDRY, c->st);
+    if (cells && c->prm.ISDRY < 98) {
+      k_dry_cells<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLE, c->dLN, c->iscdry, nwet,
+                                                    c->prm.HDRY, c->st);
+    } else if (cells) {
+      k_dry99<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLW, c->dLE, c->dLS, c->dLN,
+                                                c->iscdry, c->sub_n, c->svb_n, nwet,
+                                                c->prm.HDRY, c->st);
+      k_dry99_commit<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->sub_n, c->svb_n, nwet, c->st);
+    }
+    HIP_TRY(c, hipGetLastError());
+    return EFDC_OK;
+  };
   bool ran_mixed = false;
   int cgs = EFDC_OK;
   for (;;) {
@@ -1910,7 +2035,7 @@ int puv_run(efdc_ctx *c, const efdc_step_t *step, efdc_cg_stats_t *stats) {
         c->tide_host[M] = std::cos(TM);
         c->tide_host[c->mtide + M] = std::sin(TM);
       }
-      if (c->mtide > 0)
+      if (c->mtide > TIDE_ARGS && c->ncordry == 0)
         HIP_TRY(c, hipMemcpyAsync(c->tide_dev, c->tide_host,
                                   sizeof(double) * 2 * c->mtide,
                                   hipMemcpyHostToDevice, c->stream));
@@ -1918,18 +2043,25 @@ int puv_run(efdc_ctx *c, const efdc_step_t *step, efdc_cg_stats_t *stats) {
       for (int s = 0; s < 4; ++s) b.side[s] = c->pbc[s];
       b.tide = c->tide_dev;
       b.mtide = c->mtide;
+      if (c->mtide <= TIDE_ARGS)
+        for (int M = 0; M < 2 * c->mtide; ++M) b.tidev[M] = c->tide_host[M];
       b.lopenbcdry = c->lopenbcdry;
       int ntot = 0;
-      for (int q = 0; q < 4; ++q) {
-        if (c->pbc[q].n == 0) continue;
-        ntot += c->pbc[q].n;
-        const int nbs = c->pbc[q].serial ? 1 : (c->pbc[q].n + EFDC_BLOCK - 1) / EFDC_BLOCK;
-        TIMED(c, TK_PUV_BC, k_puv_bc_side<<<nbs, EFDC_BLOCK, 0, c->stream>>>(
-            h, b, c->pbc[q], q, c->dLW, c->dLE, c->dLS, c->dLN, dt, G, c->prm.HDRY));
+      for (int q = 0; q < 4; ++q) ntot += c->pbc[q].n;
+      if (ntot <= PBC_ONE) {
+        TIMED(c, TK_PUV_BC, k_puv_bc_all<<<1, PBC_ONE, 0, c->stream>>>(
+            h, b, ntot, c->dLW, c->dLE, c->dLS, c->dLN, dt, G, c->prm.HDRY, c->st));
+      } else {
+        for (int q = 0; q < 4; ++q) {
+          if (c->pbc[q].n == 0) continue;
+          const int nbs = c->pbc[q].serial ? 1 : (c->pbc[q].n + EFDC_BLOCK - 1) / EFDC_BLOCK;
+          TIMED(c, TK_PUV_BC, k_puv_bc_side<<<nbs, EFDC_BLOCK, 0, c->stream>>>(
+              h, b, c->pbc[q], q, c->dLW, c->dLE, c->dLS, c->dLN, dt, G, c->prm.HDRY));
+        }
+        TIMED(c, TK_PUV_BC, k_puv_bc_min<<<(ntot + EFDC_BLOCK - 1) / EFDC_BLOCK, EFDC_BLOCK, 0,
+                                           c->stream>>>(h, b, ntot, c->dLW, c->dLE, c->dLS,
+                                                        c->dLN, c->part, c->st, c->tickets));
       }
-      TIMED(c, TK_PUV_BC, k_puv_bc_min<<<(ntot + EFDC_BLOCK - 1) / EFDC_BLOCK, EFDC_BLOCK, 0,
-                                         c->stream>>>(h, b, ntot, c->dLW, c->dLE, c->dLS,
-                                                      c->dLN, c->part, c->st, c->tickets));
     }
     const bool segs = c->nseg > 1;
     if (segs) {
@@ -1949,39 +2081,28 @@ int puv_run(efdc_ctx *c, const efdc_step_t *step, efdc_cg_stats_t *stats) {
     c->mx_coef_ok = false;
     if (s != EFDC_OK && s != EFDC_ERR_CG_MAXITER) return s;
     cgs = s;
-    if (adj_recording(c) && (s = adj_record_ps(c))) return s;
-    TIMED(c, TK_PUV_POST1, k_puv_post1<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLW, c->dLS, nwet, dt));
-    TIMED(c, TK_PUV_POST2, k_puv_post2<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLE, c->dLN, c->pbcflag,
-                                                  nwet, dt, G));
+    if ((s = after_solve())) return s;
     if (!dry) break;
-    // open-boundary drying (:497-530), then the cell drying and its flag
-    // (:574-602); P already is G (HP + BELV) (:559-569, k_puv_post2)
-    for (int q = 0; q < 4; ++q)
-      if (c->pbc[q].n > 0)
-        k_dry_obc<<<(c->pbc[q].n + 255) / 256, 256, 0, c->stream>>>(
-            h, c->pbc[q], c->dLE, c->dLN, c->lopenbcdry, c->iscdry, dt, G, c->prm.HDRY);
-    const bool cells = c->prm.ISDRY < 98 || c->prm.ISDRY == 99;
-    if (cells) {
-      k_dry_flag_reset<<<1, 1, 0, c->stream>>>(c->st);
-      if (c->prm.ISDRY < 98) {
-        k_dry_cells<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLE, c->dLN, c->iscdry, nwet,
-                                                      c->prm.HDRY, c->st);
-      } else {
-        k_dry99<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLW, c->dLE, c->dLS, c->dLN,
-                                                  c->iscdry, c->sub_n, c->svb_n, nwet,
-                                                  c->prm.HDRY, c->st);
-        k_dry99_commit<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->sub_n, c->svb_n, nwet);
-      }
-    }
-    HIP_TRY(c, hipGetLastError());
     if ((s = read_state(c))) return s;
     if (c->pcg_deferred) {
       c->pcg_deferred = false;
-      if (c->st_host->pabort) {
+      if (c->st_host->pabort && c->pcg_last_plain) {
+        // the plain launch was not co-resident (the drying passes saw its
+        // abort and changed nothing): solve again, cooperatively, from the P
+        // reached, then the passes again
+        ++c->pcg_retries;
+        c->pcg_force_coop = true;
+        s = cg_dispatch(c, stats, /*defer=*/false, &ran_mixed);
+        c->pcg_force_coop = false;
+        if (s != EFDC_OK && s != EFDC_ERR_CG_MAXITER) return s;
+        cgs = s;
+        if ((s = after_solve()) || (s = read_state(c))) return s;
+      } else if (c->st_host->pabort) {
         c->err = "persistent CG: an exchange between workgroups timed out";
         return EFDC_ERR_HIP;
+      } else {
+        cgs = cg_finish(c, ran_mixed, stats);
       }
-      cgs = cg_finish(c, ran_mixed, stats);
     }
     if (!cells || !c->st_host->drychg || cgs != EFDC_OK) break;
     if (++c->ncordry >= 500) {
@@ -2003,15 +2124,24 @@ int puv_run(efdc_ctx *c, const efdc_step_t *step, efdc_cg_stats_t *stats) {
           (float *)c->dK[EFDC_H1PK - EFDC_HPK], (const float *)c->dK[EFDC_DZC - EFDC_HPK],
           c->pitch, c->KC, nwet, c->prm.HDRY, -c->prm.NDRYSTP, dt);
   }
-  TIMED(c, TK_PUV_POST3, k_puv_post3<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLW, c->dLS, nwet, c->st));
+  auto last_pass = [&]() -> int {
+    if (post23)
+      TIMED(c, TK_PUV_POST2, k_puv_post23<<<nb, EFDC_BLOCK, 0, c->stream>>>(
+          h, c->dLW, c->dLE, c->dLS, c->dLN, c->pbcflag, nwet, dt, G, c->st));
+    else
+      TIMED(c, TK_PUV_POST3, k_puv_post3<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLW, c->dLS,
+                                                                           nwet, c->st));
+    return EFDC_OK;
+  };
+  int s;
+  if ((s = last_pass())) return s;
   if (dry)
     k_dry_mask<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLE, c->dLN, c->sub1, c->svb1,
                                                  c->lmaskdry, nwet, c->prm.HDRY);
-  int s;
   if ((s = read_state(c))) return s;
   if (c->pcg_deferred) {
     c->pcg_deferred = false;
-    if (c->st_host->pabort && c->pcg_last_plain && !c->pcg_force_coop) {
+    if (c->st_host->pabort && c->pcg_last_plain) {
       // the plain launch was not co-resident: solve again, cooperatively,
       // from the P the step reached (any P is a starting iterate of the same
       // system), then redo the passes that followed the solve
@@ -2022,10 +2152,7 @@ int puv_run(efdc_ctx *c, const efdc_step_t *step, efdc_cg_stats_t *stats) {
       if (s != EFDC_OK && s != EFDC_ERR_CG_MAXITER) return s;
       cgs = s;
       k_clear_negdep<<<1, 1, 0, c->stream>>>(c->st);
-      TIMED(c, TK_PUV_POST1, k_puv_post1<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLW, c->dLS, nwet, dt));
-      TIMED(c, TK_PUV_POST2, k_puv_post2<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLE, c->dLN, c->pbcflag,
-                                                    nwet, dt, G));
-      TIMED(c, TK_PUV_POST3, k_puv_post3<<<nb, EFDC_BLOCK, 0, c->stream>>>(h, c->dLW, c->dLS, nwet, c->st));
+      if ((s = after_solve()) || (s = last_pass())) return s;
       HIP_TRY(c, hipGetLastError());
       if ((s = read_state(c))) return s;
     } else if (c->st_host->pabort) {
