@@ -607,9 +607,9 @@ int efdc_get_cg_pipeline(efdc_ctx_t *ctx, int32_t *mode);
    launch, which is co-resident whenever no other work holds the CUs; if it
    was not, its bounded waits give up and the solve is repeated with a
    cooperative launch from the P the first one reached (in a CALPUV2C step,
-   together with the passes after the solve), so the result is a converged
-   solve either way; steps with drying or adjoint recording launch
-   cooperatively.  mode 1: always the cooperative launch (guaranteed
+   together with the passes after the solve; drying passes do nothing after
+   an abandoned solve), so the result is a converged solve either way.
+   mode 1: always the cooperative launch (guaranteed
    co-residency, about 15 us more per solve).  spin_limit > 0 gives the
    plain launches' waits that many polling rounds instead of the full limit,
    which makes them give up whenever a wait is not met at once (to exercise
