@@ -22,7 +22,6 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -705,7 +704,7 @@ static void copy_out(char *dst, const char *src, size_t n) {
     const size_t m = n / parts;
     try {
       th[t] = std::thread([=] { std::memcpy(dst + at, src + at, m); });
-    } catch (const std::system_error &) {
+    } catch (...) {
       break;  // no thread to be had: the rest is copied here
     }
     at += m;
