@@ -328,6 +328,63 @@ struct NoHalo {
   __device__ void operator()(int, int) const {}
 };
 
+// The same sums with nothing to fetch beside them and a large state in
+// registers: wave g < 4 polls the partials of workgroups 64 g .. 64 g + 63
+// (and 256 further on), one group of words in its registers.  Four in wave 0,
+// as exchange holds them, are registers that every wave is allotted (FP64
+// pipelined solve, 6 cells per thread: 106 spilled).
+template <int NV>
+__device__ __forceinline__ bool exchange_waves(const Xch &x, unsigned tag, const Bar &b,
+                                               double (&sum)[NV]) {
+  constexpr int G = 4;
+  __shared__ double shw[G][NV];
+  const int lane = threadIdx.x & 63;
+  const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (g < G) {
+    double v[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = 0.0;
+    bool ok = true;
+    for (int q0 = 64 * g; q0 < x.nb && ok; q0 += 64 * G) {
+      u64 lo[NV], hi[NV];
+      unsigned spins = 0;
+      for (;;) {
+        const int ln = opaque(lane);  // as in exchange
+        const u64 *q = pslot(x, tag, x.w0 + min(q0 + ln, x.nb - 1));  // every lane loads
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          lo[j] = get_word(q + 2 * j);
+          hi[j] = get_word(q + 2 * j + 1);
+        }
+        bool ready = true;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) ready = ready && has_tag(lo[j], tag) && has_tag(hi[j], tag);
+        if (__all(ready)) break;
+        if (give_up(b, spins)) { ok = false; break; }
+      }
+#pragma unroll
+      for (int j = 0; j < NV; ++j) v[j] += q0 + lane < x.nb ? f64_of(lo[j], hi[j]) : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = wave_sum_dpp(v[j]);
+    if (lane == 0) {
+#pragma unroll
+      for (int j = 0; j < NV; ++j) shw[g][j] = v[j];
+    }
+  }
+  // shw is written again only after every wave has passed the next post()
+  __syncthreads();
+  if (bad()) return false;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < G; ++q) s += shw[q][j];
+    sum[j] = s;
+  }
+  return true;
+}
+
 // neighbour slots of a row
 enum { NS = 0, NN = 1, NW = 2, NE = 3 };
 
@@ -1334,6 +1391,10 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
 // exchange per iteration instead of two.  The stop test is the
 // reference's, (r,r) <= RSQM (:165), made on the sums of the iteration
 // that would update from r.
+// Bound by the exchange, and at 6 cells per thread by 256 registers: x in LDS
+// and the neighbours' window slots in 16 bits each leave 12 spilled (us a
+// solve of 18 to 19 iterations, this form : the default one; 79 k cells 74 : 85,
+// 276 k 105 : 118, 483 k 133 : 153, 696 k 174 : 190).
 // ---------------------------------------------------------------------
 template <int CPT>
 __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
@@ -1341,7 +1402,7 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
   // neighbour that is not a cell, so that every lane loads)
   __shared__ double lds[2 * WIN + CPT * PB + 1];
   __shared__ int hl[2 * WIN];
-  __shared__ double lzs[CPT * PB];
+  __shared__ double lzs[CPT * PB], lxs[CPT * PB];
   constexpr int ZS = 2 * WIN + CPT * PB;
   const int b0 = 1 + (int)blockIdx.x * CPT * PB;
   const int b1 = min(b0 + CPT * PB, a.nwet + 1);
@@ -1349,11 +1410,12 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
   const int lc0 = a.lc0;
 
   double ccc[CPT], cs[CPT], cn[CPT], cw[CPT], ce[CPT], cci[CPT];
-  double x[CPT], r[CPT], w[CPT], s[CPT], p[CPT];
-  int nb[CPT][4];
+  double r[CPT], w[CPT], s[CPT], p[CPT];
+  unsigned nj[CPT][2];       // window slots of S | N << 16 and W | E << 16
   unsigned expo = 0u;        // bit k: another workgroup reads cell k
   auto Z = [&](int k) -> double & { return lzs[k * PB + threadIdx.x]; };
 
+  auto X = [&](int k) -> double & { return lxs[k * PB + threadIdx.x]; };
   auto inside = [&](int j) { return j >= b0 && j < b1; };
   auto real = [&](int j) { return j > 0 && j < lc0; };
   auto slot = [&](int j) { return j - b0 + WIN; };
@@ -1368,8 +1430,8 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
       double pq[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int j = nb[k][q];
-        pq[q] = lds[real(j) ? slot(j) : ZS];
+        const unsigned u = (unsigned)opaque((int)nj[k][q >> 1]);
+        pq[q] = lds[q & 1 ? u >> 16 : u & 0xffffu];
       }
       // APCG = CCC*PCG + CCS*PS + CCN*PN + CCW*PW + CCE*PE (:113)
       y[k] = ccc[k] * v[k] + cs[k] * pq[NS] + cn[k] * pq[NN] + cw[k] * pq[NW] +
@@ -1384,10 +1446,10 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
     const int i = b0 + k * PB + (int)threadIdx.x;
-    x[k] = r[k] = w[k] = s[k] = p[k] = 0.0;
+    X(k) = r[k] = w[k] = s[k] = p[k] = 0.0;
     Z(k) = 0.0;
     ccc[k] = 1.0; cs[k] = cn[k] = cw[k] = ce[k] = cci[k] = 0.0;
-    nb[k][NS] = nb[k][NN] = nb[k][NW] = nb[k][NE] = lc0;
+    nj[k][0] = nj[k][1] = ZS | (unsigned)ZS << 16;
     if (i < b1) {
       // the row as in the multi-kernel solve (row_of)
       const int js = a.ls[i], jn = a.ln[i];
@@ -1406,23 +1468,27 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
         if (jw == lc0) w_ = 0.0;
       }
       if (js == lc0) s_ = 0.0;
-      nb[k][NS] = js; nb[k][NN] = jn; nb[k][NW] = jw; nb[k][NE] = je;
+      const int nb[4] = {js, jn, jw, je};
       ccc[k] = a.ccc[i]; cs[k] = s_; cn[k] = n_; cw[k] = w_; ce[k] = e_;
       cci[k] = a.ccci[i];
       bool out = false;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int j = nb[k][q];
+        const int j = nb[q];
         if (real(j) && !inside(j)) {
           out = true;
           hl[ghost_of(j, b0, b1)] = 1;
         }
       }
+      auto ws = [&](int j) { return real(j) ? (unsigned)slot(j) : (unsigned)ZS; };
+      nj[k][0] = ws(js) | ws(jn) << 16;
+      nj[k][1] = ws(jw) | ws(je) << 16;
       if (out || !a.mutual) expo |= 1u << k;
       const double *P = a.x;
-      x[k] = P[i];
+      const double x0 = P[i];
+      X(k) = x0;
       // RCG = FPTMP - CCC*P - CCN*PN - CCS*PS - CCW*PW - CCE*PE (:73)
-      r[k] = a.fptmp[i] - ccc[k] * x[k] - n_ * P[jn] - s_ * P[js] - w_ * P[jw] - e_ * P[je];
+      r[k] = a.fptmp[i] - ccc[k] * x0 - n_ * P[jn] - s_ * P[js] - w_ * P[jw] - e_ * P[je];
       fp2 += a.fptmp[i] * a.fptmp[i];
     }
   }
@@ -1452,7 +1518,7 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
   }
   double s1[1];
   halo();
-  if (!exchange<1, 4>(a.xc, tag, a.bar, s1, NoHalo())) return;
+  if (!exchange_waves<1>(a.xc, tag, a.bar, s1)) return;
   const double bnorm2 = s1[0];
   const double rsqm = a.rel_tol > 0.0 ? a.rel_tol * a.rel_tol * bnorm2 : a.rsqm;
   {
@@ -1493,7 +1559,7 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
     spmv(m, n);
     // the sums of every workgroup
     double s3[3];
-    if (!exchange<3, 4>(a.xc, tag, a.bar, s3, NoHalo())) return;
+    if (!exchange_waves<3>(a.xc, tag, a.bar, s3)) return;
     gam = s3[0];
     const double del = s3[1];
     rsq = s3[2];
@@ -1511,7 +1577,7 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
       const double zk = n[k] + beta * Z(k);
       s[k] = w[k] + beta * s[k];
       p[k] = cci[k] * r[k] + beta * p[k];
-      x[k] = x[k] + alpha * p[k];
+      X(k) = X(k) + alpha * p[k];
       r[k] = r[k] - alpha * s[k];
       w[k] = w[k] - alpha * zk;
       Z(k) = zk;
@@ -1523,7 +1589,7 @@ __global__ __launch_bounds__(PB) void k_pcg64_pl(P64Args a) {
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
     const int i = b0 + k * PB + (int)threadIdx.x;
-    if (i < b1) a.x[opaque(i)] = x[k];
+    if (i < b1) a.x[opaque(i)] = X(k);
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     CgState *st = a.st;
@@ -1658,6 +1724,14 @@ static int pcg_shape(const efdc_ctx *c, const int *occ, int cpt_max, int &nb,
 // exchange per iteration with the preconditioner behind it, gains nothing
 // (169 k cells 166 : 2 109, 111 : 3 114, 83 : 4 117).
 constexpr int PCG64_NB = 64;
+// The pipelined form reads them once, behind the SpMV, so it takes more
+// workgroups before a row more (us a solve of 18 iterations, workgroups : cells
+// per thread; 156 k cells 153 : 2 85, 102 : 3 82, 61 : 5 86; 276 k 180 : 3 105,
+// 108 : 5 104, 90 : 6 114; 483 k 236 : 4 139, 189 : 5 133, 158 : 6 141).
+constexpr int PCG64_PIPE_NB = 192;
+static int pcg_shape64(const efdc_ctx *c, int &nb) {
+  return pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb, c->pcg64_pipe ? PCG64_PIPE_NB : PCG64_NB);
+}
 
 // The form of the mixed persistent solve, and its shape: more than 8 cells
 // per thread (1.05 to 2.1 million cells on 256 CUs) in the pipelined form
@@ -1682,7 +1756,7 @@ bool pcg_applicable(efdc_ctx *c, bool mixed) {
   if (pcg_prepare(c) != EFDC_OK || c->pcg_ncu == 0) return false;
   int nb = 0;
   return mixed ? pcg_shape_mx(c, nb) > 0
-               : pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb, PCG64_NB) > 0;
+               : pcg_shape64(c, nb) > 0;
 }
 
 // The persistent grid is sized to be co-resident (the occupancy table times
@@ -1783,7 +1857,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
   int nb = 0;
   const Bar bar = pcg_bar(c);
   if (!mixed) {
-    const int cpt = pcg_shape(c, c->pcg_occ64, PCG64_CPT_MAX, nb, PCG64_NB);
+    const int cpt = pcg_shape64(c, nb);
     if (!cpt) { c->err = "persistent CG: problem too large"; return EFDC_ERR_ARG; }
     P64Args a;
     if ((s = p64_args(c, nb, bar, a))) return s;

@@ -351,6 +351,35 @@ def test_fp64_pipelined_form_in_steps(oracle_mod):
     ctx.close()
 
 
+@pytest.mark.parametrize("nx,ny", [(400, 390), (526, 524), (610, 600), (700, 690), (835, 833)])
+def test_fp64_pipelined_form_shapes_and_time(nx, ny):
+    """The pipelined FP64 solve with 2 to 6 cells per thread against the
+    reference's recurrences: one step's P within 1e-9 m, the same iterations
+    to within one, and no longer (the fastest of 20 solves each; measured
+    ratios 0.82 to 0.92, so 1.05 holds unless a form has lost its speed)."""
+    from efdc_amd import grids, lib
+    case = grids.external_case(np.pad(np.ones((ny, nx), bool), 1), seed=nx, dt=10.0)
+    i = wet_index(case)
+    p, its, us = {}, {}, {}
+    for form in (False, True):
+        ctx = lib.Context(case.grid, RSQM=1e-20, ITERM=400,
+                          cg_kernel=lib.CG_KERNEL_PERSISTENT).upload_case(case)
+        ctx.set_cg64_pipeline(form)
+        its[form] = ctx.calpuv2c(case.dt, 1)["iters"]
+        p[form] = ctx.get("P")[i]
+        ctx.timers(True)
+        us[form] = 1e30
+        for n in range(2, 22):
+            it = ctx.calpuv2c(case.dt, n)["iters"]
+            t = ctx.read_timers()["cg_persistent64"]
+            us[form] = min(us[form], t[1] / t[0] * 1e3 / it)
+        ctx.close()
+    print(f"{nx * ny} cells: {us[False]:.2f} us an iteration, pipelined {us[True]:.2f}")
+    assert eta_err(p[True], p[False]) <= 1e-9
+    assert abs(its[True] - its[False]) <= 1
+    assert us[True] <= 1.05 * us[False]
+
+
 @pytest.mark.parametrize("nx,ny", [(1100, 960), (1500, 1000), (1700, 1050), (2048, 1020)])
 def test_mixed_persistent_many_cells_per_thread(nx, ny):
     """The pipelined mixed solve with 10, 12, 14 and 16 cells per thread (the
