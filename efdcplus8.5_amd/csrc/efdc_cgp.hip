@@ -67,6 +67,7 @@ constexpr int WIN = 2048;         // LDS window reach beyond the own range
 constexpr int HMAX = 2 * WIN;     // outside cells of one workgroup, at most
 constexpr int NVMAX = 3;          // partials per exchange, at most
 constexpr int PCG64_CPT_MAX = 6;     // cells per thread, FP64
+constexpr int PSLOTS = PB * PCG64_CPT_MAX;  // slots of partials: a workgroup's or a basin tile's
 constexpr int PCGMX_CPT_SMALL = 8;  // cells per thread of every mixed form
 constexpr int PCGMX_CPT_MAX = 16;   // of the pipelined form alone
 
@@ -138,14 +139,14 @@ __device__ bool grid_barrier(const Bar &b, unsigned gen) {
 }
 
 struct Xch {
-  u64 *ps;             // partials: [parity][workgroup][NVMAX][2 words]
+  u64 *ps;             // partials: [parity][slot][NVMAX][2 words]
   u64 *hx;             // halo slots: [parity][cell], one word (FP32) or two (FP64) each
   int ncell;
-  int w0, nb;          // the workgroups that take part: w0 .. w0+nb-1
+  int w0, nb;          // the slots that take part: w0 .. w0+nb-1
 };
 
-__device__ __forceinline__ u64 *pslot(const Xch &x, unsigned tag, int wg) {
-  return x.ps + ((size_t)(tag & 1u) * PB + wg) * (2 * NVMAX);
+__device__ __forceinline__ u64 *pslot(const Xch &x, unsigned tag, int slot) {
+  return x.ps + ((size_t)(tag & 1u) * PSLOTS + slot) * (2 * NVMAX);
 }
 __device__ __forceinline__ u64 *hslot32(const Xch &x, unsigned tag) {
   return x.hx + (size_t)(tag & 1u) * x.ncell;
@@ -385,6 +386,131 @@ __device__ __forceinline__ bool exchange_waves(const Xch &x, unsigned tag, const
   return true;
 }
 
+// ---- sums of a basin, in the order of the per-basin launches (k_scg_*):
+// 512-cell tiles from the basin's first cell, 256 threads of two cells each;
+// waves, then the four waves of a tile, then the tiles as sum_parts adds them.
+
+// wave_sum's tree for M values of each lane together, without LDS: the lanes
+// 32 apart by exchanging register halves, where a pair of values shares the
+// halves from then on, those 16 apart by exchanging rows, where two pairs share
+// the rows; after that a row's values repeat every 8 lanes, then every 4, so a
+// rotation within the row brings the partner's.  r[i] holds value 4 i + (0, 2,
+// 1, 3) in the rows 0 to 3 (M <= 2: value 0 in rows 0 and 1, value 1 in 2 and 3).
+__device__ __forceinline__ double fold32(double x, double y) {
+  const u64 a = (u64)__double_as_longlong(x), b = (u64)__double_as_longlong(y);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
+  const auto hi =
+      __builtin_amdgcn_permlane32_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+  return f64_of(lo[0], hi[0]) + f64_of(lo[1], hi[1]);
+}
+__device__ __forceinline__ double fold16(double x, double y) {
+  const u64 a = (u64)__double_as_longlong(x), b = (u64)__double_as_longlong(y);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+  const auto hi =
+      __builtin_amdgcn_permlane16_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+  return f64_of(lo[0], hi[0]) + f64_of(lo[1], hi[1]);
+}
+template <int M>
+__device__ __forceinline__ void wave_sums_tree(const double (&v)[M], double (&r)[(M + 3) / 4]) {
+  constexpr int P = (M + 1) / 2;
+  double w[P];
+#pragma unroll
+  for (int i = 0; i < P; ++i) w[i] = fold32(v[2 * i], v[2 * i + 1 < M ? 2 * i + 1 : 2 * i]);
+#pragma unroll
+  for (int i = 0; i < (M + 3) / 4; ++i) {
+    double s = fold16(w[2 * i], w[2 * i + 1 < P ? 2 * i + 1 : 2 * i]);
+    s += dpp_move<0x128, 0xf>(s);  // row_ror:8
+    s += dpp_move<0x124, 0xf>(s);  // row_ror:4
+    s += dpp_move<0x4e, 0xf>(s);   // quad_perm [2,3,0,1]
+    s += dpp_move<0xb1, 0xf>(s);   // quad_perm [1,0,3,2]
+    r[i] = s;
+  }
+}
+
+// The partials of this workgroup's tiles (v[m]: tile 2 m + half, half 1 the
+// upper four waves) into their slots; ntile of them exist.
+template <int NV, int NT>
+__device__ __forceinline__ void post_tiles(double (&v)[NT][NV], const Xch &x, unsigned tag,
+                                           int ntile) {
+  constexpr int M = NT * NV, R = (M + 3) / 4;
+  __shared__ double sh[4 * R][PW];  // value m NV + j of every wave
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double u[M], r[R];
+#pragma unroll
+  for (int q = 0; q < M; ++q) u[q] = v[q / NV][q % NV];
+  wave_sums_tree<M>(u, r);
+  if ((lane & 15) == 0) {
+    const int row = lane >> 4, q = M <= 2 ? row >> 1 : (row & 1) * 2 + (row >> 1);
+#pragma unroll
+    for (int i = 0; i < R; ++i) sh[4 * i + q][w] = r[i];
+  }
+  __syncthreads();
+  if (threadIdx.x < 2 * NT * NV) {
+    const int tile = (int)threadIdx.x / NV, j = (int)threadIdx.x % NV;
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < PW / 2; ++q) s += sh[(tile >> 1) * NV + j][(tile & 1) * (PW / 2) + q];
+    if (tile < ntile)
+      put_f64(pslot(x, tag, (int)blockIdx.x * 2 * NT + tile) + 2 * j, tag, s);
+  }
+}
+
+// exchange over the tiles of a basin in sum_parts' order: thread t of 256
+// adds tiles t, t + 256, .., then its tree.  As many of the first four waves as the
+// tiles need poll (wave 0 alone up to 64 tiles); the others run halo(t, nt).
+template <int NV, typename HaloF>
+__device__ __forceinline__ bool exchange_tiles(const Xch &x, unsigned tag, const Bar &b,
+                                               double (&sum)[NV], HaloF halo) {
+  constexpr int W = EFDC_BLOCK / 64;  // sum_parts' waves
+  static_assert(NV <= 2, "value j of the sums lies in the rows 2 j and 2 j + 1");
+  __shared__ double shs[W][2];
+  const int lane = threadIdx.x & 63;
+  const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int nw = min(W, (x.nb + 63) >> 6);
+  if (g < nw) {
+    double v[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = 0.0;
+    bool ok = true;
+    for (int h0 = 64 * g; h0 < x.nb && ok; h0 += 64 * W) {
+      u64 lo[NV], hi[NV];
+      unsigned spins = 0;
+      for (;;) {
+        const int ln = opaque(lane);  // as in exchange
+        const u64 *p = pslot(x, tag, x.w0 + min(h0 + ln, x.nb - 1));  // every lane loads
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          lo[j] = get_word(p + 2 * j);
+          hi[j] = get_word(p + 2 * j + 1);
+        }
+        bool ready = true;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+          ready = ready && has_tag(lo[j], tag) && has_tag(hi[j], tag);
+        if (__all(ready)) break;
+        if (give_up(b, spins)) { ok = false; break; }
+      }
+#pragma unroll
+      for (int j = 0; j < NV; ++j) v[j] += h0 + lane < x.nb ? f64_of(lo[j], hi[j]) : 0.0;
+    }
+    double r[1];
+    wave_sums_tree<NV>(v, r);
+    if ((lane & 31) == 0) shs[g][lane >> 5] = r[0];
+  } else {
+    halo((int)threadIdx.x - 64 * nw, PB - 64 * nw);
+  }
+  // shs is written again only after every wave has passed the next post_tiles()
+  __syncthreads();
+  if (bad()) return false;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    double s = 0.0;
+    for (int q = 0; q < nw; ++q) s += shs[q][j];
+    sum[j] = s;
+  }
+  return true;
+}
+
 // neighbour slots of a row
 enum { NS = 0, NN = 1, NW = 2, NE = 3 };
 
@@ -446,18 +572,23 @@ struct P64Args {
   CgState *st;
   double rsqm, rel_tol;
   int iterm;
-  // basins: {first cell, end of the basin, first workgroup, workgroups} and
-  // the basin of every workgroup, the basins' states
+  // basins: {first cell, end of the basin, first workgroup, tiles} and the
+  // basin of every workgroup, the basins' states, a copy of x
   const int4 *wg;
   const int *wgseg;
   CgState *segst;
+  double *xsave;
 };
 
 // SEG: every basin of an ensemble is a solve of its own, by the workgroups of
 // its cells: sums, stop test and iteration count are the basin's, and a basin
-// that has stopped frees its workgroups while the others go on.  Against two
-// launches over all basins per iteration, whose vectors go through memory (40
-// basins of 16000 cells, FP64, 15 iterations): 4 steps 3460 -> 1949 us.
+// that has stopped frees its workgroups while the others go on.  Its sums are
+// taken over the tiles and in the order of the per-basin launches, so a
+// basin's bits are those of the basin alone with those launches, whatever
+// basins share the context and however many cells a thread has: a half of
+// the workgroup owns a tile, a thread two cells of it 256 apart (CPT is even).
+// Against two launches over all basins per iteration, whose vectors go through
+// memory (40 basins of 16000 cells, FP64, 15 iterations): 4 steps 3460 -> 1960 us.
 template <int CPT, bool SEG>
 __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   // the window, then one word that stays zero (read in place of a
@@ -467,7 +598,9 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   __shared__ double zh[HMAX];  // z of the outside cells
   constexpr int ZS = 2 * WIN + CPT * PB;
   // below the most cells per thread there are at most PCG64_NB workgroups
-  constexpr int UG = SEG ? 1 : CPT < PCG64_CPT_MAX ? 2 : 4;
+  constexpr int UG = CPT < PCG64_CPT_MAX ? 2 : 4;
+  static_assert(!SEG || CPT % 2 == 0, "a tile is two cells a thread of half a workgroup");
+  constexpr int NT = SEG ? CPT / 2 : 1;
   int b0 = 1 + (int)blockIdx.x * CPT * PB, b1 = min(b0 + CPT * PB, a.nwet + 1);
   Xch xc = a.xc;
   // the cells of this solve: in the row-major form the first cell of a basin
@@ -479,9 +612,16 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
     b1 = min(b0 + CPT * PB, q.y);
     c0 = a.wg[q.z].x;
     c1 = q.y;
-    xc.w0 = q.z;
+    xc.w0 = q.z * CPT;
     xc.nb = q.w;
   }
+  const int ntile = (b1 - b0 + PB - 1) / PB;
+  // the cell of row k
+  auto cell = [&](int k) {
+    const int t = (int)threadIdx.x;
+    return SEG ? b0 + ((k & ~1) + (t >> 8)) * PB + (k & 1) * (PB / 2) + (t & (PB / 2 - 1))
+               : b0 + k * PB + t;
+  };
   const bool fast = a.rowmajor && (a.st->symok == 0);
   const int lc0 = a.lc0;
 
@@ -500,10 +640,11 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   for (int g = threadIdx.x; g < 2 * WIN; g += PB) hl[g] = 0;
   if (threadIdx.x == 0) { lds[ZS] = 0.0; bad() = 0; }
   __syncthreads();
-  double v2[2] = {0.0, 0.0};
+  // partials: the thread's, or (SEG) those of its cells in each of its tiles
+  double v2[NT][2] = {};
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int i = b0 + k * PB + (int)threadIdx.x;
+    const int i = cell(k);
     x[k] = r[k] = p[k] = ap[k] = 0.0;
     ccc[k] = 1.0; cs[k] = cn[k] = cw[k] = ce[k] = cci[k] = 0.0;
     nb[k][NS] = nb[k][NN] = nb[k][NW] = nb[k][NE] = lc0;
@@ -540,12 +681,13 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
       if (out || !a.mutual) expo |= 1u << k;
       const double *P = a.x;
       x[k] = P[i];
+      if (SEG) a.xsave[i] = x[k];
       // RCG = FPTMP - CCC*P - CCN*PN - CCS*PS - CCW*PW - CCE*PE (:73)
       const double rr = a.fptmp[i] - ccc[k] * x[k] - n_ * P[jn] - s_ * P[js] -
                         w_ * P[jw] - e_ * P[je];
       r[k] = rr;
-      v2[0] += rr * (rr * cci[k]);   // RPCG = sum RCG*PCG (:80-85)
-      v2[1] += a.fptmp[i] * a.fptmp[i];
+      v2[SEG ? k >> 1 : 0][0] += rr * (rr * cci[k]);   // RPCG = sum RCG*PCG (:80-85)
+      v2[SEG ? k >> 1 : 0][1] += a.fptmp[i] * a.fptmp[i];
     }
   }
   __syncthreads();
@@ -564,10 +706,15 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   // CCCI of an outside cell), RPCG and |FPTMP|^2
 #pragma unroll
   for (int k = 0; k < CPT; ++k)
-    if (expo & (1u << k)) publish_z(b0 + k * PB + (int)threadIdx.x, tag, cci[k] * r[k]);
-  post<2>(v2, xc, tag);
+    if (expo & (1u << k)) publish_z(cell(k), tag, cci[k] * r[k]);
   double s2[2];
-  if (!exchange<2, UG>(xc, tag, a.bar, s2, halo)) return;
+  if constexpr (SEG) {
+    post_tiles<2, NT>(v2, xc, tag, ntile);
+    if (!exchange_tiles<2>(xc, tag, a.bar, s2, halo)) return;
+  } else {
+    post<2>(v2[0], xc, tag);
+    if (!exchange<2, UG>(xc, tag, a.bar, s2, halo)) return;
+  }
   double rpcg = s2[0];
   const double bnorm2 = s2[1];
   const double rsqm = a.rel_tol > 0.0 ? a.rel_tol * a.rel_tol * bnorm2 : a.rsqm;
@@ -583,7 +730,7 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       p[k] = cci[k] * r[k] + beta * p[k];
-      lds[slot(b0 + k * PB + (int)threadIdx.x)] = p[k];
+      lds[slot(cell(k))] = p[k];
     }
     // ... and on the outside cells
     for (int h = threadIdx.x; h < nhalo; h += PB) {
@@ -591,7 +738,7 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
       pj = zh[h] + beta * pj;
     }
     __syncthreads();
-    double v1[1] = {0.0};
+    double v1[NT][1] = {};
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       double pq[4];
@@ -603,29 +750,39 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
       // APCG = CCC*PCG + CCS*PS + CCN*PN + CCW*PW + CCE*PE (:113)
       ap[k] = ccc[k] * p[k] + cs[k] * pq[NS] + cn[k] * pq[NN] + cw[k] * pq[NW] +
               ce[k] * pq[NE];
-      v1[0] += ap[k] * p[k];
+      v1[SEG ? k >> 1 : 0][0] += ap[k] * p[k];
     }
     ++tag;
-    post<1>(v1, xc, tag);
     double s1[1];
-    if (!exchange<1, UG>(xc, tag, a.bar, s1, NoHalo())) return;
+    if constexpr (SEG) {
+      post_tiles<1, NT>(v1, xc, tag, ntile);
+      if (!exchange_tiles<1>(xc, tag, a.bar, s1, NoHalo())) return;
+    } else {
+      post<1>(v1[0], xc, tag);
+      if (!exchange<1, UG>(xc, tag, a.bar, s1, NoHalo())) return;
+    }
     papcg = s1[0];
     alpha = rpcg / papcg;  // :124
-    double v[2] = {0.0, 0.0};
+    double v[NT][2] = {};
     ++tag;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int i = b0 + k * PB + (int)threadIdx.x;
+      const int i = cell(k);
       x[k] = x[k] + alpha * p[k];        // :132
       const double rr = r[k] - alpha * ap[k];  // :133
       r[k] = rr;
       const double z = cci[k] * rr;      // :134
-      v[0] += rr * z;
-      v[1] += rr * rr;
+      v[SEG ? k >> 1 : 0][0] += rr * z;
+      v[SEG ? k >> 1 : 0][1] += rr * rr;
       if (expo & (1u << k)) publish_z(i, tag, z);
     }
-    post<2>(v, xc, tag);
-    if (!exchange<2, UG>(xc, tag, a.bar, s2, halo)) return;
+    if constexpr (SEG) {
+      post_tiles<2, NT>(v, xc, tag, ntile);
+      if (!exchange_tiles<2>(xc, tag, a.bar, s2, halo)) return;
+    } else {
+      post<2>(v[0], xc, tag);
+      if (!exchange<2, UG>(xc, tag, a.bar, s2, halo)) return;
+    }
     beta = s2[0] / rpcg;  // :147-148
     rpcg = s2[0];
     rsq = s2[1];
@@ -635,10 +792,10 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   }
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int i = b0 + k * PB + (int)threadIdx.x;
+    const int i = cell(k);
     if (i < b1) a.x[opaque(i)] = x[k];
   }
-  if ((int)blockIdx.x == xc.w0 && threadIdx.x == 0) {
+  if ((SEG ? (int)blockIdx.x * CPT == xc.w0 : blockIdx.x == 0) && threadIdx.x == 0) {
     CgState *st = SEG ? a.segst + a.wgseg[blockIdx.x] : a.st;
     st->rpcg = rpcg;
     st->papcg = papcg;
@@ -1678,18 +1835,21 @@ int pcg_prepare(efdc_ctx *c) {
   const int occ64p[PCG64_CPT_MAX + 1] = {
       0, occupancy(k_pcg64_pl<1>), occupancy(k_pcg64_pl<2>), occupancy(k_pcg64_pl<3>),
       occupancy(k_pcg64_pl<4>), occupancy(k_pcg64_pl<5>), occupancy(k_pcg64_pl<6>)};
+  // 2, 4 and 6 cells per thread for basins
   const int occ64s[PCG64_CPT_MAX + 1] = {
-      0, occupancy(k_pcg64<1, true>), occupancy(k_pcg64<2, true>), occupancy(k_pcg64<3, true>),
-      occupancy(k_pcg64<4, true>), occupancy(k_pcg64<5, true>), occupancy(k_pcg64<6, true>)};
-  for (int k = 0; k <= PCG64_CPT_MAX; ++k)
-    c->pcg_occ64[k] = std::min({occ64[k], occ64p[k], occ64s[k]});
+      0, 0, occupancy(k_pcg64<2, true>), 0, occupancy(k_pcg64<4, true>), 0,
+      occupancy(k_pcg64<6, true>)};
+  for (int k = 0; k <= PCG64_CPT_MAX; ++k) {
+    c->pcg_occ64[k] = std::min(occ64[k], occ64p[k]);
+    c->pcg_occseg[k] = occ64s[k];
+  }
   for (int k = 0; k <= PCGMX_CPT_MAX; ++k)
     c->pcg_occmx[k] = k <= PCGMX_CPT_SMALL ? std::min(occmx[k], occpl[k]) : occpl[k];
   c->pcg_ncell = c->n_wet() + 2;
   int s;
   // two parities of two words a cell, and of NVMAX doubles a workgroup
   if ((s = dev_alloc(c, &c->pcg_hx, sizeof(u64) * 4 * (size_t)c->pcg_ncell))) return s;
-  if ((s = dev_alloc(c, &c->pcg_ps, sizeof(u64) * 2 * PB * 2 * NVMAX))) return s;
+  if ((s = dev_alloc(c, &c->pcg_ps, sizeof(u64) * 2 * PSLOTS * 2 * NVMAX))) return s;
   if ((s = dev_alloc(c, (void **)&c->pcg_ctr, sizeof(unsigned) * PCG_NCTR))) return s;
   c->pcg_abort = &c->st->pabort;
   c->pcg_launch = 0;
@@ -1787,7 +1947,7 @@ static int next_tag0(efdc_ctx *c, unsigned &tag0) {
   const bool wrap = c->pcg_launch == PCG_LAUNCH_CYCLE;
   c->pcg_launch = c->pcg_launch % PCG_LAUNCH_CYCLE + 1u;
   if (wrap) {
-    k_pcg_clear<<<512, 256, 0, c->stream>>>((u64 *)c->pcg_ps, 2 * PB * 2 * NVMAX,
+    k_pcg_clear<<<512, 256, 0, c->stream>>>((u64 *)c->pcg_ps, 2 * PSLOTS * 2 * NVMAX,
                                             (u64 *)c->pcg_hx, 4 * (long)c->pcg_ncell);
     HIP_TRY(c, hipGetLastError());
   }
@@ -1795,15 +1955,21 @@ static int next_tag0(efdc_ctx *c, unsigned &tag0) {
   return EFDC_OK;
 }
 
-template <bool SEG>
 static const void *p64_kernel(int cpt) {
   switch (cpt) {
-    case 1: return (const void *)k_pcg64<1, SEG>;
-    case 2: return (const void *)k_pcg64<2, SEG>;
-    case 3: return (const void *)k_pcg64<3, SEG>;
-    case 4: return (const void *)k_pcg64<4, SEG>;
-    case 5: return (const void *)k_pcg64<5, SEG>;
-    default: return (const void *)k_pcg64<6, SEG>;
+    case 1: return (const void *)k_pcg64<1, false>;
+    case 2: return (const void *)k_pcg64<2, false>;
+    case 3: return (const void *)k_pcg64<3, false>;
+    case 4: return (const void *)k_pcg64<4, false>;
+    case 5: return (const void *)k_pcg64<5, false>;
+    default: return (const void *)k_pcg64<6, false>;
+  }
+}
+static const void *pseg_kernel(int cpt) {
+  switch (cpt) {
+    case 2: return (const void *)k_pcg64<2, true>;
+    case 4: return (const void *)k_pcg64<4, true>;
+    default: return (const void *)k_pcg64<6, true>;
   }
 }
 
@@ -1835,6 +2001,7 @@ static int p64_args(efdc_ctx *c, int nb, const Bar &bar, P64Args &a) {
   a.wg = nullptr;
   a.wgseg = nullptr;
   a.segst = nullptr;
+  a.xsave = nullptr;
   return EFDC_OK;
 }
 
@@ -1872,7 +2039,7 @@ int pcg_solve(efdc_ctx *c, bool mixed, bool defer) {
         default: fn = (const void *)k_pcg64_pl<6>; break;
       }
     } else {
-      fn = p64_kernel<false>(cpt);
+      fn = p64_kernel(cpt);
     }
     TIMED(c, TK_PCG64, s = coop_launch(c, fn, nb, a));
     if (s) return s;
@@ -1994,7 +2161,7 @@ int pcg_vec_solve(efdc_ctx *c, double *x, const double *rhs, CgState *st, CgStat
   a.rsqm = 0.0;
   a.rel_tol = rel_tol;
   a.iterm = itmax;
-  TIMED(c, TK_ADJ_CG, s = coop_launch(c, p64_kernel<false>(cpt), nb, a));
+  TIMED(c, TK_ADJ_CG, s = coop_launch(c, p64_kernel(cpt), nb, a));
   if (s) return s;
   HIP_TRY(c, hipMemcpyAsync(st_host, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -2014,8 +2181,8 @@ int pcg_vec_solve(efdc_ctx *c, double *x, const double *rhs, CgState *st, CgStat
 // Cells per thread with which every basin's workgroups fit one co-resident
 // grid together, and their number; 0 if they do not.
 static int pcg_seg_shape(const efdc_ctx *c, int &nb) {
-  for (int cpt = 1; cpt <= PCG64_CPT_MAX; ++cpt) {
-    const int cap = std::min(c->pcg_occ64[cpt] * c->pcg_ncu, PB);
+  for (int cpt = 2; cpt <= PCG64_CPT_MAX; cpt += 2) {
+    const int cap = std::min(c->pcg_occseg[cpt] * c->pcg_ncu, PB);
     long need = 0;
     for (int q = 0; q < c->nseg; ++q)
       need += (c->seg_first[q + 1] - c->seg_first[q] + cpt * PB - 1) / (cpt * PB);
@@ -2043,12 +2210,11 @@ int pcg_seg_solve(efdc_ctx *c) {
     std::vector<int4> wg;
     std::vector<int> seg;
     for (int q = 0; q < c->nseg; ++q) {
-      const int w0 = (int)wg.size(), end = c->seg_first[q + 1];
-      for (int i = c->seg_first[q]; i < end; i += cpt * PB) {
-        wg.push_back(make_int4(i, end, w0, 0));
+      const int w0 = (int)wg.size(), first = c->seg_first[q], end = c->seg_first[q + 1];
+      for (int i = first; i < end; i += cpt * PB) {
+        wg.push_back(make_int4(i, end, w0, (end - first + PB - 1) / PB));
         seg.push_back(q);
       }
-      for (size_t w = w0; w < wg.size(); ++w) wg[w].w = (int)wg.size() - w0;
     }
     if ((s = dev_alloc(c, &c->pcg_segwg, (sizeof(int4) + sizeof(int)) * wg.size()))) return s;
     HIP_TRY(c, hipMemcpyAsync(c->pcg_segwg, wg.data(), sizeof(int4) * wg.size(),
@@ -2064,7 +2230,8 @@ int pcg_seg_solve(efdc_ctx *c) {
   a.wg = (const int4 *)c->pcg_segwg;
   a.wgseg = (const int *)(a.wg + nb);
   a.segst = c->d_segst;
-  TIMED(c, TK_PCG64, s = coop_launch(c, p64_kernel<true>(cpt), nb, a));
+  a.xsave = c->r;  // (the launches' residual, which every solve of theirs writes first)
+  TIMED(c, TK_PCG64, s = coop_launch(c, pseg_kernel(cpt), nb, a));
   if (s) return s;
   HIP_TRY(c, hipMemcpyAsync(c->h_segst, c->d_segst, sizeof(CgState) * c->nseg,
                             hipMemcpyDeviceToHost, c->stream));
@@ -2076,7 +2243,10 @@ int pcg_seg_solve(efdc_ctx *c) {
     c->err = "persistent CG: an exchange between workgroups timed out";
     return EFDC_ERR_HIP;
   }
-  // not co-resident: again, cooperatively, from the P each basin reached
+  // not co-resident: again, cooperatively, from the P of the first launch
+  // (some basins may have finished), so that every basin's bits stay its own
+  HIP_TRY(c, hipMemcpyAsync(c->dH[EFDC_P] + 1, c->r + 1, sizeof(double) * c->n_wet(),
+                            hipMemcpyDeviceToDevice, c->stream));
   ++c->pcg_retries;
   c->pcg_force_coop = true;
   s = pcg_seg_solve(c);

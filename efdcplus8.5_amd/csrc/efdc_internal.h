@@ -153,7 +153,7 @@ struct efdc_ctx {
   // persistent solve (efdc_cgp.hip), allocated on first use
   bool pcg_ready = false;
   int pcg_ncu = 0;             // CUs, 0 when cooperative launch is unsupported
-  int pcg_occ64[7] = {}, pcg_occmx[17] = {};  // workgroups per CU by CPT
+  int pcg_occ64[7] = {}, pcg_occseg[7] = {}, pcg_occmx[17] = {};  // workgroups per CU by CPT
   void *pcg_hx = nullptr;      // halo slots [2][ncell][2] tagged words
   void *pcg_ps = nullptr;      // partial slots
   void *pcg_segwg = nullptr;   // workgroup tables of the basins' persistent solve

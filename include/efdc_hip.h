@@ -608,7 +608,9 @@ int efdc_get_cg_pipeline(efdc_ctx_t *ctx, int32_t *mode);
    was not, its bounded waits give up and the solve is repeated with a
    cooperative launch from the P the first one reached (in a CALPUV2C step,
    together with the passes after the solve; drying passes do nothing after
-   an abandoned solve), so the result is a converged solve either way.
+   an abandoned solve; basins start again from the P they started from, so
+   that each one's bits stay its own), so the result is a converged solve
+   either way.
    mode 1: always the cooperative launch (guaranteed
    co-residency, about 15 us more per solve).  spin_limit > 0 gives the
    plain launches' waits that many polling rounds instead of the full limit,

@@ -73,3 +73,58 @@ def test_basins_persistent_cap_and_repeated_launch():
     assert eta_err(a.get("P")[L], b.get("P")[L]) <= 1e-9
     a.close()
     b.close()
+
+
+def _rect(nx, ny, seed):
+    from efdc_amd import grids
+    return grids.external_case(np.pad(np.ones((ny, nx), bool), 1), seed=seed, depth_sigma=2.0)
+
+
+def _companies():
+    """The same three basins (one tile, 11 tiles with a ragged end, 70 tiles) first,
+    in the middle and last, beside small ones, beside one of 300 tiles and
+    beside as many as leave two, four and six cells a thread."""
+    from efdc_amd import grids
+    three = [_rect(20, 17, 41),
+             grids.external_case(grids.lake_mask(96, 88, 42), seed=42, depth_sigma=2.0),
+             _rect(211, 169, 43)]
+    small = [_rect(16 + i, 9 + i % 3, 50 + i) for i in range(4)]
+    wide = [_rect(401, 383, 60)]
+    many = [_rect(250, 201, 70 + i) for i in range(9)]
+    return three, [(0, three + small), (4, small + three + wide), (9, many + three),
+                   (1, wide + three + many)]
+
+
+def test_basin_bits_do_not_depend_on_its_company():
+    """With the kernel left to the library, which takes the persistent solve, a
+    basin's fields are bit for bit those of the basin alone with
+    CG_KERNEL_MULTI, whichever basins share its context; also where the launch
+    was abandoned and repeated."""
+    from efdc_amd import grids, lib
+    fields = ["P", "P1", "HP", "H1P", "HU", "UHDYE", "VHDXE", "CCC", "CCS", "FPTMP"]
+    three, companies = _companies()
+    alone = []
+    for b in three:
+        c = _ctx(b)
+        its = [c.calpuv2c(b.dt, n)["iters"] for n in (1, 2, 3)]
+        alone.append((its, {f: c.get(f)[1:1 + b.grid.nwet] for f in fields}))
+        c.close()
+    for at, basins in companies:
+        ens, first = grids.concat_basins(basins)
+        for spin in (0, 1):
+            c = _ctx(ens, cg_kernel=lib.CG_KERNEL_AUTO)
+            c.set_segments(first)
+            c.set_cg_launch(0, spin_limit=spin)
+            c.timers(True)
+            its = []
+            for n in (1, 2, 3):
+                c.calpuv2c(ens.dt, n)
+                its.append(list(c.segment_stats()[0][at:at + 3]))
+            assert "cg_persistent64" in c.read_timers()
+            assert (c.cg_launch()[1] >= 1) == (spin == 1)
+            for q in range(3):
+                sl = grids.basin_slice(ens, first, at + q)
+                assert [i[q] for i in its] == alone[q][0], (at, spin, q)
+                for f in fields:
+                    assert np.array_equal(c.get(f)[sl], alone[q][1][f]), (at, spin, q, f)
+            c.close()
