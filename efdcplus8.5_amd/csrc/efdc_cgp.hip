@@ -2216,12 +2216,20 @@ int pcg_seg_solve(efdc_ctx *c) {
         seg.push_back(q);
       }
     }
-    if ((s = dev_alloc(c, &c->pcg_segwg, (sizeof(int4) + sizeof(int)) * wg.size()))) return s;
-    HIP_TRY(c, hipMemcpyAsync(c->pcg_segwg, wg.data(), sizeof(int4) * wg.size(),
-                              hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, hipMemcpyAsync((int4 *)c->pcg_segwg + wg.size(), seg.data(),
-                              sizeof(int) * seg.size(), hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    void *tab = nullptr;  // the context's only once it is whole
+    if ((s = dev_alloc(c, &tab, (sizeof(int4) + sizeof(int)) * wg.size()))) return s;
+    hipError_t e = hipMemcpyAsync(tab, wg.data(), sizeof(int4) * wg.size(),
+                                  hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync((int4 *)tab + wg.size(), seg.data(), sizeof(int) * seg.size(),
+                         hipMemcpyHostToDevice, c->stream);
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess || es != hipSuccess) {
+      (void)hipFree(tab);
+      HIP_TRY(c, e);
+      HIP_TRY(c, es);
+    }
+    c->pcg_segwg = tab;
   }
   k_pcg_reset<<<1, PCG_NCTR, 0, c->stream>>>(c->pcg_ctr, c->pcg_abort);
   HIP_TRY(c, hipGetLastError());
