@@ -935,6 +935,7 @@ int efdc_set_cg_replay(efdc_ctx_t *c, int32_t mode) {
   if (!c || mode < 0 || mode > 2) return EFDC_ERR_ARG;
   c->cg_graph = mode == 1;
   c->cg_graph_tune = mode == 2;
+  if (mode == 0) c->seg_launches = false;
   return EFDC_OK;
 }
 
@@ -987,7 +988,7 @@ int efdc_autotune(efdc_ctx_t *c, int32_t on) {
   c->tune_pending = on != 0;
   c->tune_cg_pending = on != 0;
   c->cg_graph_tune = on != 0;
-  if (!on) c->cg_graph = false;
+  if (!on) c->cg_graph = c->seg_launches = false;
   if (on) {
     c->tune_n = 0;
     c->tune_best = -1;

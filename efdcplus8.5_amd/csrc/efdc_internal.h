@@ -128,6 +128,7 @@ struct efdc_ctx {
   int4 *d_tiles_s[4] = {};
   int *d_segtile0_s[4] = {};
   int ntiles_s[4] = {};
+  bool seg_launches = false;   // a trial found the launches faster than the persistent solve
   int seg_tset = 1;
   bool seg_tune_pending = false;
   double *tune_psave = nullptr;  // P saved for the CG trials (LCM)

@@ -1638,11 +1638,12 @@ void key_of(std::vector<unsigned char> &k, const A &...a) {
   (k.insert(k.end(), (const unsigned char *)&a, (const unsigned char *)&a + sizeof(a)), ...);
 }
 
-// A timed trial of the two replay modes of a solve (`solve(graph)` runs
-// it whole), each from the P the solve starts from; the faster becomes
-// the context's mode and P is restored.
+// A timed trial of the two replay modes of a solve and, for basins, of the
+// persistent solve (`solve(m)`, m < nmode, runs it whole: launch by launch,
+// replayed, persistent), each from the P the solve starts from; the fastest
+// becomes the context's mode and P is restored.
 template <typename F>
-int cg_graph_trial(efdc_ctx *c, F solve) {
+int cg_graph_trial(efdc_ctx *c, int nmode, F solve) {
   int s;
   const size_t bytes = sizeof(double) * c->LCM;
   if (!c->tune_psave && (s = dev_alloc(c, (void **)&c->tune_psave, bytes))) return s;
@@ -1651,9 +1652,9 @@ int cg_graph_trial(efdc_ctx *c, F solve) {
   hipEvent_t e0, e1;
   HIP_TRY(c, hipEventCreate(&e0));
   HIP_TRY(c, hipEventCreate(&e1));
-  float ms[2] = {0.f, 0.f};
+  float ms[3] = {0.f, 0.f, 0.f};
   s = EFDC_OK;
-  for (int g = 0; g < 2 && !s; ++g) {
+  for (int g = 0; g < nmode && !s; ++g) {
     hipError_t e = hipMemcpyAsync(c->dH[EFDC_P], c->tune_psave, bytes, hipMemcpyDeviceToDevice,
                                   c->stream);
     if (e == hipSuccess) e = hipEventRecord(e0, c->stream);
@@ -1662,7 +1663,7 @@ int cg_graph_trial(efdc_ctx *c, F solve) {
       s = EFDC_ERR_HIP;
       break;
     }
-    if ((s = solve(g == 1))) break;
+    if ((s = solve(g))) break;
     e = hipEventRecord(e1, c->stream);
     if (e == hipSuccess) e = hipEventSynchronize(e1);
     if (e == hipSuccess) e = hipEventElapsedTime(&ms[g], e0, e1);
@@ -1674,14 +1675,16 @@ int cg_graph_trial(efdc_ctx *c, F solve) {
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (s) return s;
-  c->cg_graph = ms[1] < ms[0];
+  const int best = (int)(std::min_element(ms, ms + nmode) - ms);
+  c->cg_graph = best == 1;
+  if (nmode > 2) c->seg_launches = best != 2;
   c->cg_graph_tune = false;
-  const char *names[2] = {"cg_fp64 launches", "cg_fp64 graphs"};
-  for (int g = 0; g < 2; ++g)
+  const char *names[3] = {"cg_fp64 launches", "cg_fp64 graphs", "cg_fp64 persistent"};
+  for (int g = 0; g < nmode; ++g)
     if (c->tune_n < 8) {
       std::snprintf(c->tune_name[c->tune_n], 32, "%s", names[g]);
       c->tune_ms[c->tune_n] = ms[g];
-      c->tune_chosen[c->tune_n] = (g == 1) == c->cg_graph ? 1 : 0;
+      c->tune_chosen[c->tune_n] = g == best ? 1 : 0;
       ++c->tune_n;
     }
   HIP_TRY(c, hipMemcpyAsync(c->dH[EFDC_P], c->tune_psave, bytes, hipMemcpyDeviceToDevice,
@@ -1741,7 +1744,7 @@ int cg_fp64_solve(efdc_ctx *c, bool graph) {
 int cg_fp64(efdc_ctx *c) {
   int s;
   if (c->cg_graph_tune && !c->timing &&
-      (s = cg_graph_trial(c, [&](bool g) { return cg_fp64_solve(c, g); })))
+      (s = cg_graph_trial(c, 2, [&](int g) { return cg_fp64_solve(c, g == 1); })))
     return s;
   return cg_fp64_solve(c, c->cg_graph && !c->timing);
 }
@@ -2292,8 +2295,10 @@ int seg_solve_set(efdc_ctx *c, int q, bool graph) {
   }
 }
 
-// The tile trials: each set solves the same system from the same P, timed
-// with events on the context stream; the fastest becomes the current set.
+// The tile trials: each set, and the persistent solve where it applies, solves
+// the same system from the same P, timed with events on the context stream;
+// the fastest becomes the current one (the persistent solve with set 1, whose
+// tiles it sums).
 int seg_tune_tiles(efdc_ctx *c) {
   int s;
   if (!c->tune_psave && (s = dev_alloc(c, (void **)&c->tune_psave, sizeof(double) * c->LCM)))
@@ -2308,18 +2313,20 @@ int seg_tune_tiles(efdc_ctx *c) {
   int bq = c->seg_tset;
   const bool timing = c->timing;
   c->timing = false;
-  for (int q = 0; q < 4; ++q) {
+  const bool pers = pcg_seg_applicable(c);
+  for (int q = 0; q < (pers ? 5 : 4); ++q) {
     HIP_TRY(c, hipMemcpyAsync(c->dH[EFDC_P], c->tune_psave, bytes, hipMemcpyDeviceToDevice,
                               c->stream));
-    seg_select_tiles(c, q);
+    if (q < 4) seg_select_tiles(c, q);
     HIP_TRY(c, hipEventRecord(e0, c->stream));
-    if ((s = seg_solve_set(c, q, false))) break;
+    if ((s = q < 4 ? seg_solve_set(c, q, false) : pcg_seg_solve(c))) break;
     HIP_TRY(c, hipEventRecord(e1, c->stream));
     HIP_TRY(c, hipEventSynchronize(e1));
     float ms = 0.f;
     HIP_TRY(c, hipEventElapsedTime(&ms, e0, e1));
     if (c->tune_n < 8) {
-      std::snprintf(c->tune_name[c->tune_n], 32, "seg_cg_tile_%d", EFDC_BLOCK << q);
+      if (q < 4) std::snprintf(c->tune_name[c->tune_n], 32, "seg_cg_tile_%d", EFDC_BLOCK << q);
+      else std::snprintf(c->tune_name[c->tune_n], 32, "seg_cg_persistent");
       c->tune_ms[c->tune_n] = ms;
       c->tune_chosen[c->tune_n] = 0;
       ++c->tune_n;
@@ -2333,10 +2340,14 @@ int seg_tune_tiles(efdc_ctx *c) {
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (s) return s;
-  for (int j = 0; j < c->tune_n; ++j)
+  for (int j = 0; j < c->tune_n; ++j) {
     if (std::strncmp(c->tune_name[j], "seg_cg_tile_", 12) == 0)
-      c->tune_chosen[j] = std::atoi(c->tune_name[j] + 12) == (EFDC_BLOCK << bq) ? 1 : 0;
-  seg_select_tiles(c, bq);
+      c->tune_chosen[j] = bq < 4 && std::atoi(c->tune_name[j] + 12) == (EFDC_BLOCK << bq) ? 1 : 0;
+    else if (std::strcmp(c->tune_name[j], "seg_cg_persistent") == 0)
+      c->tune_chosen[j] = bq == 4 ? 1 : 0;
+  }
+  seg_select_tiles(c, bq < 4 ? bq : 1);
+  c->seg_launches = bq < 4;
   HIP_TRY(c, hipMemcpyAsync(c->dH[EFDC_P], c->tune_psave, bytes, hipMemcpyDeviceToDevice,
                             c->stream));
   c->seg_tune_pending = false;
@@ -2447,10 +2458,16 @@ int seg_cg_run(efdc_ctx *c, efdc_cg_stats_t *stats, bool *ran_mixed) {
     }
   }
   if (c->seg_tune_pending && (s = seg_tune_tiles(c))) return s;
+  // The persistent solve takes the place of the launches with the default
+  // tile, whose bits it gives, unless replays were asked for or a trial found
+  // them or the launches faster
+  const bool pers = c->seg_tset == 1 && pcg_seg_applicable(c);
   if (c->cg_graph_tune && !c->timing &&
-      (s = cg_graph_trial(c, [&](bool g) { return seg_solve_set(c, c->seg_tset, g); })))
+      (s = cg_graph_trial(c, pers ? 3 : 2, [&](int m) {
+         return m == 2 ? pcg_seg_solve(c) : seg_solve_set(c, c->seg_tset, m == 1);
+       })))
     return s;
-  if (pcg_seg_applicable(c)) {
+  if (pers && !c->cg_graph && !c->seg_launches) {
     if ((s = pcg_seg_solve(c))) return s;
   } else {
     if ((s = seg_solve_set(c, c->seg_tset, c->cg_graph && !c->timing))) return s;

@@ -68,6 +68,7 @@ void seg_free(efdc_ctx *c) {
   if (c->h_segst) (void)hipHostFree(c->h_segst);
   c->h_segst = nullptr;
   c->nseg = 1;
+  c->seg_launches = false;
   c->seg_first.clear();
   c->ntiles = 0;
 }
@@ -172,6 +173,7 @@ int efdc_set_segment_tile(efdc_ctx_t *c, int32_t cells) {
   for (int q = 0; q < 4; ++q)
     if (cells == (EFDC_BLOCK << q)) {
       c->seg_tune_pending = false;
+      c->seg_launches = false;
       if (c->nseg > 1) seg_select_tiles(c, q);
       else c->seg_tset = q;
       return EFDC_OK;

@@ -624,13 +624,15 @@ class Context:
         self.nseg = len(a)
 
     def set_segment_tile(self, cells: int):
-        """CG tile of the basins: 256, 512 (bitwise, the default), 1024,
-        2048, or 0 to time the four on the next solve."""
+        """CG tile of the basins: 256, 512 (bitwise, the default; solved by
+        the persistent launch where it applies), 1024, 2048, or 0 to time
+        the four and that launch on the next solve."""
         self._check(self.lib.efdc_set_segment_tile(self.h, cells))
 
     def set_cg_replay(self, mode: int):
         """0 launch by launch, 1 captured graphs, 2 time both on the next
-        solve (FP64 multi-kernel CG)."""
+        solve (FP64 multi-kernel CG; for basins 0 takes the persistent
+        launch where it applies and 2 times it too)."""
         self._check(self.lib.efdc_set_cg_replay(self.h, mode))
 
     def cg_replay(self) -> int:

@@ -576,10 +576,14 @@ int efdc_set_segments(efdc_ctx_t *ctx, int32_t nseg, const int32_t *first_L);
    (256, 512, 1024 or 2048) whose partial sums the basin's reduction adds in
    order.  512, the default, is the tile of the single-model solve, so each
    basin's results are bit for bit those of the basin alone; other sizes
-   sum in another order (results within round-off).  cells = 0 times the
-   four sizes on the next solve (each from the same P) and keeps the
-   fastest; efdc_get_segment_tile gives the size in use and
-   efdc_tune_report lists the trial times. */
+   sum in another order (results within round-off).  With 512 and the kernel
+   left to the library (or EFDC_CG_KERNEL_PERSISTENT) the basins are solved
+   by one persistent launch, with the same bits, while their rows fit one
+   co-resident grid; other sizes are solved by two launches per iteration.
+   cells = 0 times the four sizes and, where it applies, the persistent
+   solve on the next solve (each from the same P) and keeps the fastest;
+   efdc_get_segment_tile gives the size in use (512 for the persistent
+   solve) and efdc_tune_report lists the trial times. */
 int efdc_set_segment_tile(efdc_ctx_t *ctx, int32_t cells);
 int efdc_get_segment_tile(efdc_ctx_t *ctx, int32_t *cells);
 
@@ -588,7 +592,10 @@ int efdc_get_segment_tile(efdc_ctx_t *ctx, int32_t *cells);
    hipGraphs of 8 and 1 iterations, 2 time both on the next solve from the
    same P and keep the faster (efdc_autotune(ctx, 1) does the same).  The
    two give the same bits; with the library's timers on the solves launch
-   kernel by kernel. */
+   kernel by kernel.  Basins are solved by replays with mode 1, by the
+   persistent launch where it applies with mode 0, and mode 2 times all
+   three.  One model replays only where its FP64 solve is the multi-kernel
+   one. */
 int efdc_set_cg_replay(efdc_ctx_t *ctx, int32_t mode);
 int efdc_get_cg_replay(efdc_ctx_t *ctx, int32_t *mode);
 /* Form of the mixed persistent inner solve (EFDC_CG_MIXED on one

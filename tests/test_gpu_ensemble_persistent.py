@@ -128,3 +128,52 @@ def test_basin_bits_do_not_depend_on_its_company():
                 for f in fields:
                     assert np.array_equal(c.get(f)[sl], alone[q][1][f]), (at, spin, q, f)
             c.close()
+
+
+def test_settings_of_the_basins_solve_act():
+    """The tile and the replay of the per-basin launches select them; the
+    trials time the persistent solve beside them and what they choose is what
+    the next solve runs.  Every choice but another tile gives the same bits."""
+    from efdc_amd import grids, lib
+    ens, first = grids.concat_basins([_rect(120, 101, 5), _rect(64, 33, 6), _rect(90, 90, 7)])
+
+    def run(setup, auto=True):
+        kern = lib.CG_KERNEL_AUTO if auto else lib.CG_KERNEL_MULTI
+        c = _ctx(ens, cg_kernel=kern)
+        c.set_segments(first)
+        setup(c)
+        c.calpuv2c(ens.dt, 1)  # trials, if any
+        c.timers(True)
+        c.calpuv2c(ens.dt, 2)
+        t = c.read_timers()
+        p, rep, tile, rp = c.get("P"), c.tune_report(), c.segment_tile(), c.cg_replay()
+        c.close()
+        assert ("cg_persistent64" in t) != ("cg_spmv_pupdate" in t)
+        return p, "cg_persistent64" in t, rep, tile, rp
+
+    want = run(lambda c: None, auto=False)[0]
+    for setup, persistent in ((lambda c: None, True), (lambda c: c.set_segment_tile(512), True),
+                              (lambda c: c.set_cg_replay(1), False),
+                              (lambda c: (c.set_cg_replay(1), c.set_cg_replay(0)), True)):
+        p, pers, _, tile, _ = run(setup)
+        assert pers == persistent and tile == 512
+        assert np.array_equal(p, want)
+    p, pers, _, tile, _ = run(lambda c: c.set_segment_tile(1024))
+    assert not pers and tile == 1024
+    assert eta_err(p, want) <= 1e-9
+    for setup, names in (
+            (lambda c: c.set_segment_tile(0), ["seg_cg_tile_256", "seg_cg_tile_512",
+                                               "seg_cg_tile_1024", "seg_cg_tile_2048",
+                                               "seg_cg_persistent"]),
+            (lambda c: c.set_cg_replay(2), ["cg_fp64 launches", "cg_fp64 graphs",
+                                            "cg_fp64 persistent"])):
+        p, pers, rep, tile, rp = run(setup)
+        assert list(rep["shapes"]) == names
+        chosen = rep["chosen"]
+        assert chosen == [min(names, key=rep["shapes"].get)]
+        assert pers == chosen[0].endswith("persistent")
+        assert rp == (1 if chosen[0].endswith("graphs") else 0)
+        if chosen[0].startswith("seg_cg_tile_"):
+            assert tile == int(chosen[0][12:])
+        if tile == 512:
+            assert np.array_equal(p, want)
