@@ -1176,15 +1176,29 @@ __global__ __launch_bounds__(256) void k_copy_pieces(PieceTab t, char *buf, int 
   if (o < bytes && o >= base && whole - base < (size_t)U * 4096) dst[o] = src[o];
 }
 
+// Whether p .. p + bytes lies in one allocation (`unknown`: p is in none).
+bool holds(const void *p, size_t bytes, bool unknown) {
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+    (void)hipGetLastError();  // no allocation of this runtime's
+    return unknown;
+  }
+  return (size_t)((const char *)p - (const char *)base) + bytes <= size;
+}
+
 // Copy the pieces to (save) or from (load) consecutive 256-byte aligned
 // slots of buf on the context's stream.  The kernel takes a 16-byte aligned
-// buffer in this device's memory; any other buffer goes piece by piece
-// through the runtime's copies.
+// buffer in one allocation of this device's memory that holds every slot; any
+// other buffer goes piece by piece through the runtime's copies, and one whose
+// allocation is known to end within or before a slot is refused before anything
+// is copied, as the runtime refuses a copy past an allocation's end.
 int copy_pieces(efdc_ctx *c, const std::vector<Piece> &pcs, char *buf, bool save) {
   bool direct = ((uintptr_t)buf & 15) == 0;
-  size_t total = 0;
+  size_t total = 0, need = 0;  // need: to the end of the last piece
   for (const Piece &p : pcs) {
     total += p.bytes;
+    if (p.bytes) need = ((need + 255) & ~(size_t)255) + p.bytes;
     if (p.bytes && (!p.p || ((uintptr_t)p.p & 15))) direct = false;
   }
   if (direct) {
@@ -1192,11 +1206,22 @@ int copy_pieces(efdc_ctx *c, const std::vector<Piece> &pcs, char *buf, bool save
     if (hipPointerGetAttributes(&at, buf) != hipSuccess) {
       (void)hipGetLastError();  // an unregistered host pointer
       direct = false;
-    } else if (at.type != hipMemoryTypeDevice || at.device != c->device) {
+    } else if (at.type != hipMemoryTypeDevice || at.device != c->device ||
+               !holds(buf, need, false)) {
       direct = false;
     }
   }
   if (!direct) {
+    const char *slot = buf;
+    const bool unknown = holds(buf, 0, true) && !holds(buf, 0, false);
+    for (const Piece &p : pcs) {
+      if (p.bytes && !holds(slot, p.bytes, unknown)) {
+        c->err = "the buffer is smaller than its contents (efdc_state_bytes, "
+                 "efdc_adj_record_bytes)";
+        return EFDC_ERR_ARG;
+      }
+      slot += (p.bytes + 255) & ~(size_t)255;
+    }
     for (const Piece &p : pcs) {
       if (save)
         HIP_TRY(c, hipMemcpyAsync(buf, p.p, p.bytes, hipMemcpyDeviceToDevice, c->stream));

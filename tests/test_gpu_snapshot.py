@@ -77,3 +77,31 @@ def test_snapshot_copies(nx, ny, kc, internal, store):
     other.close()
     a.free()
     b.free()
+
+
+@pytest.mark.parametrize("align", [0, 8])
+def test_short_buffer_is_refused(align):
+    """A device buffer that ends within the snapshot is refused on the host
+    before anything is copied, in both directions, also where the one-launch
+    copy would take it (16-byte aligned)."""
+    from efdc_amd import grids, lib
+    case = grids.tidal_basin(100, 80, 2, seed=9)
+    ctx = lib.Context(case.grid, RSQM=1e-20, ITERM=500)
+    ctx.upload_case(case)
+    ctx.step(case.dt, 1)
+    nb = ctx.state_bytes()
+    p = ctx.get("P")
+    whole, short = _DeviceBytes(nb + 8), _DeviceBytes(nb // 2)
+    for call in (ctx.state_save, ctx.state_load):
+        with pytest.raises(lib.EfdcError) as e:
+            call(short.p.value + align)
+        assert e.value.status == 1
+    assert np.all(short.get() == 0xAB)
+    assert np.array_equal(ctx.get("P"), p)
+    ctx.state_save(whole.p.value + align)
+    ctx.step(case.dt, 2)
+    ctx.state_load(whole.p.value + align)
+    assert np.array_equal(ctx.get("P"), p)
+    ctx.close()
+    whole.free()
+    short.free()
