@@ -675,6 +675,10 @@ int efdc_add_constituent(efdc_ctx_t *c, const efdc_constituent_t *d,
     k.buf[j] = p;
   }
   *slot = c->nconst++;
+  // the tuned transport kernel was timed without it
+  c->tran_ncg = 0;
+  c->tran_w3 = 0;
+  c->tran_tuned = false;
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   return EFDC_OK;
 }

@@ -1969,12 +1969,15 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
       c->ev_pool.push_back(e0);
       c->ev_pool.push_back(e1);
     }
-    // untuned default: k_tran_lay where it fits, else 2 constituents per
-    // wave (column kernel with mutual maps), else as many lanes as fit
+    // untuned default (and where the tuned shape does not fit): k_tran_lay
+    // where it fits, else 2 constituents per wave (column kernel with mutual
+    // maps), else as many lanes as fit (nq > 0: k_tran_lay or a column shape fits)
     int q = req != 0 ? (req < 0 ? -req : req) : c->tran_tuned ? c->tran_ncg : 0;
     int var = req != 0 ? req_var : c->tran_tuned ? c->tran_w3 : 0;
-    if (q == 0 && !lay.ncg) var = 0;
-    if (q == 0 ? !lay.ncg : !shape_ok(q)) q = (colm && shape_ok(2)) ? 2 : qs[0];
+    if (q == 0 ? !lay.ncg : !shape_ok(q)) {
+      q = lay.ncg ? 0 : (colm && shape_ok(2)) ? 2 : qs[0];
+      var = 0;
+    }
     TIMED(c, TK_TRAN, launch(q, var));
     const bool settled = q == 0 && settles;
     if (any_adac) {

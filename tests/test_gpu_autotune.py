@@ -56,3 +56,36 @@ def test_autotuned_mixed_solve_degree():
     assert eta_err(m.get("P")[i], d.get("P")[i]) <= 1e-6
     m.close()
     d.close()
+
+
+@pytest.mark.parametrize("kc", [5, 64])
+def test_constituent_added_after_tuning(kc):
+    """A constituent that is added after the tuner has chosen a column kernel
+    may leave no column shape that fits (64 layers in FP64: one fills the
+    64 KiB, two take 96): the next step runs a kernel that fits, with the bits
+    of a context that was never tuned."""
+    from efdc_amd import grids, lib
+    case = grids.tidal_basin(130, 120, kc, seed=8)
+    case.sources = case.conc_bc = case.open_bc = None
+    both = case.consts
+    one, two = case.copy(), case.copy()
+    one.consts = [both[0]]
+    a = lib.Context(one.grid).upload_case(one)
+    a.autotune(True)
+    for n in (1, 2):
+        a.calconc(case.dt, n)
+    assert len(a.tune_report()["chosen"]) == 1
+    con, con1 = a.get_constituent(0)
+    c = both[1]
+    slot = a.add_constituent(c["mo"], c["isadac"], c["isfct"], c["rkdye"], c["is_dye"])
+    a.set_constituent(slot, c["con"], c["con1"])
+    two.consts = [dict(both[0], con=con, con1=con1), dict(c, wset=0.0)]
+    b = lib.Context(two.grid).upload_case(two)
+    for n in (3, 4):
+        a.calconc(case.dt, n)
+        b.calconc(case.dt, n)
+    for j in range(2):
+        assert all(np.array_equal(x, y) for x, y in zip(a.get_constituent(j),
+                                                        b.get_constituent(j))), j
+    a.close()
+    b.close()
