@@ -1735,6 +1735,15 @@ int adac_pipeline(efdc_ctx *c, TranArgs<T> &ta, const efdc_step_t *step) {
   return EFDC_OK;
 }
 
+// The settling sweep of constituent j's new concentrations.
+template <typename T>
+void settle_con(efdc_ctx *c, const TranArgs<T> &a, const efdc_step_t *step, int j) {
+  const efdc_constituent_t &d = c->con[j].desc;
+  TIMED(c, TK_SETTLE, k_settle<T><<<(a.nwet + 256) / 256, 256, 0, c->stream>>>(
+      a.nw[j], a.hpki, a.pitch, a.KC, a.nwet, step->dt, d.wset, d.probdep * d.wset,
+      d.wese, a.lmask));
+}
+
 // CON1 of the open-boundary columns, then the CON/CON1 buffer swap.
 template <typename T>
 int finish_tran(efdc_ctx *c, TranArgs<T> &a, const efdc_step_t *step, bool settled = false) {
@@ -1745,9 +1754,7 @@ int finish_tran(efdc_ctx *c, TranArgs<T> &a, const efdc_step_t *step, bool settl
       const int s = adj_record_settle(c, j, a.nw[j]);
       if (s) return s;
     }
-    TIMED(c, TK_SETTLE, k_settle<T><<<(a.nwet + 256) / 256, 256, 0, c->stream>>>(
-        a.nw[j], a.hpki, a.pitch, a.KC, a.nwet, step->dt, d.wset, d.probdep * d.wset,
-        d.wese, a.lmask));
+    settle_con(c, a, step, j);
   }
   if (c->nbcrec > 0) {
     const int tot = c->nbcrec * c->KC;
@@ -1919,7 +1926,8 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
       // every shape computes the same bits, and a repeated launch
       // rewrites the same outputs (CON from CON1, the recovery memory of
       // outflow boundary layers), so the shapes are timed on the step
-      // itself; the chosen one runs last
+      // itself; the chosen one runs last.  A column kernel is timed with the
+      // settling launches that it needs and k_tran_lay does not
       c->tune_pending = false;
       int best = -1;
       float best_ms = 1e30f;
@@ -1938,6 +1946,9 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
           for (int r = 0; r < 4; ++r) {
             HIP_TRY(c, hipEventRecord(e0, c->stream));
             launch(cand[qi], w3);
+            if (cand[qi] != 0 && settles)
+              for (int j = 0; j < nc; ++j)
+                if (c->con[j].desc.wset > 0.0) settle_con(c, a, step, j);
             HIP_TRY(c, hipEventRecord(e1, c->stream));
             HIP_TRY(c, hipEventSynchronize(e1));
             float ms = 0.f;

@@ -89,3 +89,30 @@ def test_constituent_added_after_tuning(kc):
                                                         b.get_constituent(j))), j
     a.close()
     b.close()
+
+
+def test_column_kernels_are_timed_with_their_settling():
+    """The layer kernel settles in its own pass, the column kernels need a
+    launch for it: the tuner times both with the settling, and the step it
+    tunes on gives the bits of an untuned one."""
+    from efdc_amd import grids, lib
+    case = grids.tidal_basin(64, 48, 6, seed=8)
+    case.consts[1].update(wset=3e-4, probdep=0.6, wese=1e-6)
+    a = lib.Context(case.grid).upload_case(case)
+    b = lib.Context(case.grid).upload_case(case)
+    a.timers(True)
+    a.autotune(True)
+    a.calconc(case.dt, 1)
+    b.calconc(case.dt, 1)
+    rep = a.tune_report()
+    columns = [n for n in rep["shapes"] if n.startswith("tran_colm")]
+    assert "tran_layers" in rep["shapes"] and columns
+    n = a.read_timers()["settle"][0]
+    assert n == 4 * len(columns) + (rep["chosen"][0] != "tran_layers")
+    a.calconc(case.dt, 2)
+    b.calconc(case.dt, 2)
+    for j in range(len(case.consts)):
+        assert all(np.array_equal(x, y) for x, y in zip(a.get_constituent(j),
+                                                        b.get_constituent(j))), j
+    a.close()
+    b.close()
