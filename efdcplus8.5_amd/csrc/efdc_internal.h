@@ -220,6 +220,7 @@ struct efdc_ctx {
   bool adac_alloc = false;
   void *adac_more = nullptr;   // scratch of further constituents, 8 (adac_sets - 1) planes
   int adac_sets = 0;
+  int adac_most = EFDC_MAXC;   // constituents at a time that the memory was there for
   // uniform layer constants (sigma grid): CDZKK/CDZKMK per K
   bool dz_uni_kk = true, dz_uni_kmk = true;
   bool dz_uniform() const { return dz_uni_kk && dz_uni_kmk; }

@@ -1673,7 +1673,7 @@ int adac_pipeline(efdc_ctx *c, TranArgs<T> &ta, const efdc_step_t *step) {
   // steps 1217 -> 994 us with the finishing kernel).
   const int nc = c->nconst;
   const int fit = (int)((128u << 20) / (8 * plane * sizeof(T)));
-  const int per = std::max(1, std::min({fit, nc, ADAC_GROUP}));
+  int per = std::max(1, std::min({fit, nc, ADAC_GROUP, c->adac_most}));
   if (per > c->adac_sets) {
     if (c->adac_more) {
       HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -1681,8 +1681,15 @@ int adac_pipeline(efdc_ctx *c, TranArgs<T> &ta, const efdc_step_t *step) {
       c->adac_more = nullptr;
     }
     c->adac_sets = 1;
-    const int s = dev_alloc(c, &c->adac_more, (size_t)(per - 1) * 8 * plane * sizeof(T));
-    if (s) return s;
+    // without the memory for all of them, fewer at a time: one needs no more
+    while (per > 1) {
+      const int s = dev_alloc(c, &c->adac_more, (size_t)(per - 1) * 8 * plane * sizeof(T));
+      if (s == EFDC_OK) break;
+      if (s != EFDC_ERR_NOMEM) return s;
+      (void)hipGetLastError();
+      per /= 2;
+      c->adac_most = per;  // not tried again on every step
+    }
     c->adac_sets = per;
   }
   FinishArgs<T> f;
