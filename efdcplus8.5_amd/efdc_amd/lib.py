@@ -31,7 +31,9 @@ CG_KERNEL_AUTO, CG_KERNEL_MULTI, CG_KERNEL_PERSISTENT = 0, 1, 2
 STORE_FP64, STORE_FP32 = 0, 1
 
 
-_PY_BYTES = C.pythonapi.PyBytes_FromStringAndSize
+# a handle of its own: restype and argtypes of C.pythonapi's functions belong to
+# whichever module sets them last
+_PY_BYTES = C.PyDLL(None).PyBytes_FromStringAndSize
 _PY_BYTES.restype, _PY_BYTES.argtypes = C.py_object, [C.c_char_p, C.c_ssize_t]
 
 

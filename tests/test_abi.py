@@ -104,3 +104,21 @@ def test_noalloc_congrad_refuses_sizes_beyond_its_scratch():
         rc = L.efdc_congrad_noalloc(la, *dummy, 1e-9, 100, None, C.byref(st))
         assert rc == STATUS["EFDC_ERR_ARG"]
         assert b"LA+1" in L.efdc_last_error(None)
+
+
+def test_bytes_constructor_is_the_modules_own():
+    """The constructor of the restart text's bytes object does not change with
+    what another module sets on the process-wide ctypes.pythonapi function, and
+    sets nothing there itself."""
+    import ctypes as C
+    from efdc_amd import lib
+    f = C.pythonapi.PyBytes_FromStringAndSize
+    saved = f.restype, f.argtypes
+    try:
+        f.restype, f.argtypes = C.c_int, [C.c_int]
+        b = lib._PY_BYTES(None, 5)
+        assert type(b) is bytes and len(b) == 5
+        assert lib._PY_BYTES is not f
+    finally:
+        f.restype = saved[0]
+        f.argtypes = saved[1]
