@@ -1903,8 +1903,10 @@ int tran_impl(efdc_ctx *c, const efdc_step_t *step) {
         const dim3 grid(nbc, lay.ngrp), lblk(64, lay.nlw + (a.vd && KC > 1 ? 1 : 0));
         if (lay.ncg == 1) k_tran_lay<T, 1><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
         else if (lay.ncg == 2) k_tran_lay<T, 2><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
-        else if (lay.ncg == 3) k_tran_lay<T, 3><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
-        else k_tran_lay<T, 4><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
+        else if constexpr (sizeof(T) == 4) {  // (lay_shape: at most 2 in FP64)
+          if (lay.ncg == 3) k_tran_lay<T, 3><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
+          else k_tran_lay<T, 4><<<grid, lblk, lay.lds, c->stream>>>(a, sa, lay.nlw);
+        }
         return;
       }
       const dim3 blk(64, waves_of(q));

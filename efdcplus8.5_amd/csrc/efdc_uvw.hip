@@ -1239,12 +1239,17 @@ int uvw_launch(efdc_ctx *c, const efdc_step_t *st, const efdc_uvw_opts_t *o) {
     UVW_EXACT(10) UVW_EXACT(12) UVW_EXACT(16) UVW_EXACT(20)
 #undef UVW_EXACT
     default:
-      if (KC <= 8)
+      // (9 to 31 layers, in FP32 up to 35, take k_uvw_lay)
+      if (KC <= 8) {
         TIMED(c, TK_UVW_COL, k_uvw_col<T, 8, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
-      else if (KC <= 32)  // (9 to 31 take k_uvw_lay)
-        TIMED(c, TK_UVW_COL, k_uvw_col<T, 32, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
-      else
-        TIMED(c, TK_UVW_COL, k_uvw_col<T, 64, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
+        break;
+      }
+      if constexpr (sizeof(T) == 8)
+        if (KC <= 32) {
+          TIMED(c, TK_UVW_COL, k_uvw_col<T, 32, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
+          break;
+        }
+      TIMED(c, TK_UVW_COL, k_uvw_col<T, 64, false><<<nb, EFDC_BLOCK, 0, c->stream>>>(a));
   }
   if (KC > 1)
     TIMED(c, TK_UVW_W, (k_uvw_w<T, true><<<nb, EFDC_BLOCK, 0, c->stream>>>(a)));
