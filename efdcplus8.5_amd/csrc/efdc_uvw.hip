@@ -380,20 +380,26 @@ constexpr bool uvw_exact(int KC) {
   return (KC >= 2 && KC <= 6) || KC == 8 || KC == 10 || KC == 12 || KC == 16 || KC == 20;
 }
 
-// Whether the columns take k_uvw_lay.  Up to 560 tiles of 64 cells k_uvw_col
-// has a wave for half of the 1024 SIMDs and every wave waits for its own loads
-// (us a call, layers : columns, FP32 storage; 544 tiles 5 layers 16.2 : 17.8,
-// 10 22.1 : 26.5, 20 44.7 : 50.7, 24 67.6 : 95.5; 128 tiles 20 layers 24.8 :
-// 47.2; but 2 layers 13.9 : 11.3).  From there to one wave a SIMD the columns
-// are faster where they have straight-line code (938 tiles, 10 layers 34.5 :
-// 30.0, 20 72.1 : 64.4), beyond it only below 12 layers (4000 tiles, 10 layers
-// 112 : 105, 12 136 : 177, 16 185 : 215, 20 269 : 277).  Other counts above 8
-// predicate each layer of a larger instance, which is slower at any size (4000
-// tiles, 9 layers 100 : 182; 938 tiles, 13 38 : 66) as long as two workgroups
-// fit a CU's LDS (FP64, 1875 tiles, 32 layers 436 : 306).
+// Whether the columns take k_uvw_lay (us a call, layers : columns, at tiles of
+// 64 cells).  k_uvw_col has one wave a tile and face, which waits for its own
+// loads: up to 512 tiles there is none for half of the 1024 SIMDs.  From 4
+// layers on the layers are faster there (FP32 storage, 127 tiles 4 layers 11.4 :
+// 14.2, 8 13.2 : 19.5, 20 24.8 : 47.2; 479 tiles 5 layers 15.8 : 19.0, 8 19.1 : 22.4;
+// 3 layers equal, 2 slower), from 6 on up to 768 tiles, where six workgroups a
+// CU are full and a second round begins (562 tiles 4 layers 20.6 : 16.3, 5 21.1 :
+// 17.6, 6 18.5 : 19.5, 10 22.0 : 27.9, 20 45.7 : 50.0; 719 tiles 8 layers 21.4 :
+// 25.1, 12 25.9 : 32.1, 16 40.5 : 39.9, 20 52.1 : 52.5; 806 tiles 8 layers 28.0 :
+// 23.8, 12 35.8 : 32.0, 20 66.3 : 52.5; FP64 alike).  Beyond, the columns are the faster
+// where they have straight-line code, up to one wave a SIMD at any count
+// (1021 tiles 12 layers 37.0 : 33.7, 20 76.4 : 65.0; 1148 tiles 12 layers 42.9 : 59.1, 20
+// 79.6 : 117.1), then below 12 layers (4000 tiles, 10 layers 112 : 105, 12 136 :
+// 177, 16 185 : 215, 20 269 : 277).  Other counts above 8 predicate each layer of a
+// larger instance, which is slower at any size (4000 tiles, 9 layers 100 : 182;
+// 938 tiles, 13 38 : 66) as long as two workgroups fit a CU's LDS (FP64, 1875
+// tiles, 32 layers 436 : 306).
 template <typename T>
 bool uvw_lay(int KC, int tiles) {
-  if (tiles <= 560) return KC >= 4 && uvw_lay_lds<T>(KC) <= 160 * 1024;
+  if (KC >= 4 && tiles <= (KC < 6 ? 512 : 768)) return uvw_lay_lds<T>(KC) <= 160 * 1024;
   if (uvw_exact(KC)) return KC >= 12 && tiles > 1024;
   return KC > 8 && uvw_lay_lds<T>(KC) <= 80 * 1024;
 }
