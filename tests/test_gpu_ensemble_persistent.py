@@ -1,6 +1,7 @@
 """The FP64 solve of an ensemble's basins in one persistent launch (the
-default) against the two-launches-per-iteration solve: the same iterations
-to within one and levels within round-off of the FP64 CG."""
+default) against the two-launches-per-iteration solve: a basin's bits are its
+own with either, whatever basins share the context, and the settings and
+trials of the solve choose between them."""
 import numpy as np
 import pytest
 
