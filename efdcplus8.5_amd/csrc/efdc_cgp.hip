@@ -1,4 +1,4 @@
-// efdc_cgp.hip -- CONGRAD as one persistent cooperative launch per solve.
+// efdc_cgp.hip -- CONGRAD as one persistent launch per solve.
 //
 // The multi-kernel solve (efdc_puv.hip) pays two launches and two grid
 // reductions per iteration; at the sizes of a real lake (10^4 .. 10^6 wet
@@ -597,7 +597,10 @@ __global__ __launch_bounds__(PB) void k_pcg64(P64Args a) {
   __shared__ int hl[2 * WIN];
   __shared__ double zh[HMAX];  // z of the outside cells
   constexpr int ZS = 2 * WIN + CPT * PB;
-  // below the most cells per thread there are at most PCG64_NB workgroups
+  // Groups of 64 slots in flight.  Below the most cells per thread there are at
+  // most PCG64_NB workgroups, one group: the second one's loads repeat its last
+  // slot, and without them a solve is no faster (us, 2 : 1; 21 k cells 73.8 :
+  // 75.0, 79 k 86.7 : 87.9, 276 k 117.7 : 118.5).
   constexpr int UG = CPT < PCG64_CPT_MAX ? 2 : 4;
   static_assert(!SEG || CPT % 2 == 0, "a tile is two cells a thread of half a workgroup");
   constexpr int NT = SEG ? CPT / 2 : 1;
@@ -1162,11 +1165,12 @@ __global__ __launch_bounds__(PB) void k_pcgmx_pl(PMxArgs a) {
   // straight to the window; towards 256 VGPRs, a row keeps the window slots
   // of its south and north neighbours in one word, M^-1 v stays in the window,
   // and the rows' addresses are formed where they are used.  Bound by the
-  // exchanges and, at 16 cells per thread, by about 100 spilled registers.
-  // Against two launches per iteration of the multi-kernel solve (31 inner
-  // iterations, this one 17): 1.10 M cells 988 -> 237 us, 1.37 M 1101 -> 283,
-  // 2.02 M 1335 -> 546.  Up to 8 the plain form is the faster one (6 cells:
-  // 163 against 180 us).
+  // exchanges and, at 12, 14 and 16 cells per thread, by 30, 91 and 157 spilled
+  // registers.  Against two launches per iteration of the multi-kernel solve
+  // (31 inner iterations, this one 17; lakes, event-timed): 1.10 M cells 1024 -> 233
+  // us, 1.37 M 1108 -> 269, 2.02 M 1320 -> 525.  Up to 8 the plain form is the
+  // faster one for all its spills (30 at 7, 69 at 8; us a solve of 13
+  // iterations, plain : BIG; 6 cells 134 : 155, 7 156 : 168, 8 172 : 178).
   constexpr bool BIG = CPT > PCGMX_CPT_SMALL;
   static_assert(!BIG || 3 * CPT * PB >= 2 * WIN, "the list of outside cells is formed there");
   __shared__ int hl[BIG ? 1 : 2 * WIN];
@@ -1802,7 +1806,6 @@ int occupancy(K kern) {
 
 }  // namespace
 
-// Largest cells-per-thread instantiation of each solve.
 // Terms of the workgroup-local preconditioner of the mixed persistent solve
 // when the caller leaves the choice to the library.
 constexpr int PCG_PDEG_DEFAULT = 3;

@@ -1,7 +1,7 @@
 """The two launch strategies of CONGRAD against the oracle.
 
 * multi-kernel: two launches per iteration (EFDC_CG_KERNEL_MULTI);
-* persistent: one cooperative launch per solve with the rows held in
+* persistent: one launch per solve with the rows held in
   registers (EFDC_CG_KERNEL_PERSISTENT).
 
 Both run the FP64 Jacobi-PCG of the reference (|d eta| <= 1e-9 m against
