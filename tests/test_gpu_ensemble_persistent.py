@@ -43,10 +43,10 @@ def test_basins_persistent_against_launches(make, persistent):
         ia, sa = a.segment_stats()
         ib, sb = b.segment_stats()
         assert not np.any(sa) and not np.any(sb)
-        assert np.max(np.abs(np.asarray(ia) - np.asarray(ib))) <= 1
+        assert list(ia) == list(ib)
     assert ("cg_persistent64" in a.read_timers()) == persistent
     L = np.arange(1, ens.grid.LA)
-    assert eta_err(a.get("P")[L], b.get("P")[L]) <= 1e-9
+    assert np.array_equal(a.get("P")[L], b.get("P")[L])
     a.close()
     b.close()
 
@@ -71,7 +71,7 @@ def test_basins_persistent_cap_and_repeated_launch():
     b.calpuv2c(ens.dt, 1)
     assert a.cg_launch()[1] >= 1
     L = np.arange(1, ens.grid.LA)
-    assert eta_err(a.get("P")[L], b.get("P")[L]) <= 1e-9
+    assert np.array_equal(a.get("P")[L], b.get("P")[L])
     a.close()
     b.close()
 
@@ -100,7 +100,8 @@ def test_basin_bits_do_not_depend_on_its_company():
     """With the kernel left to the library, which takes the persistent solve, a
     basin's fields are bit for bit those of the basin alone with
     CG_KERNEL_MULTI, whichever basins share its context; also where the launch
-    was abandoned and repeated."""
+    was abandoned and repeated.  All basins of a context (up to 300 tiles, more
+    than a reduction's 256 threads) against its solve by launches."""
     from efdc_amd import grids, lib
     fields = ["P", "P1", "HP", "H1P", "HU", "UHDYE", "VHDXE", "CCC", "CCS", "FPTMP"]
     three, companies = _companies()
@@ -112,6 +113,10 @@ def test_basin_bits_do_not_depend_on_its_company():
         c.close()
     for at, basins in companies:
         ens, first = grids.concat_basins(basins)
+        m = _ctx(ens)
+        m.set_segments(first)
+        for n in (1, 2, 3):
+            m.calpuv2c(ens.dt, n)
         for spin in (0, 1):
             c = _ctx(ens, cg_kernel=lib.CG_KERNEL_AUTO)
             c.set_segments(first)
@@ -128,7 +133,10 @@ def test_basin_bits_do_not_depend_on_its_company():
                 assert [i[q] for i in its] == alone[q][0], (at, spin, q)
                 for f in fields:
                     assert np.array_equal(c.get(f)[sl], alone[q][1][f]), (at, spin, q, f)
+            for f in fields:
+                assert np.array_equal(c.get(f)[1:ens.grid.LA], m.get(f)[1:ens.grid.LA]), (at, f)
             c.close()
+        m.close()
 
 
 def test_settings_of_the_basins_solve_act():
